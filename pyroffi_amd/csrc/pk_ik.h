@@ -89,6 +89,7 @@ struct IkArgs {
   float* state;                   // (total_seeds, 2 * n_act + 3) or null
   int iter_begin, iter_end;
   GridArgs grid;
+  int seeds_per_wave;  // ls_ik_kernel with a shared penalty: seeds of one wave, at most 8
   // When non-null, the batched kernel adds the number of sphere-pair tests
   // its collision penalty executed (per seed, summed over its iterations).
   unsigned long long* work;
@@ -97,7 +98,7 @@ struct IkArgs {
 // Shared-memory image of one problem, built by the prologue.
 template <int MAXA, int NEE>
 struct IkShared {
-  NodeRec nodes[MAXA + kMaxJoints];   // worst case: every joint moves
+  NodeRec nodes[MAXA];                // a robot with more moving joints is reported, not solved
   int n_nodes;
   int ee_node[NEE];
   float ee_rel[NEE][7];               // node frame -> EE frame
@@ -119,8 +120,7 @@ __device__ __forceinline__ void pose_to(float* p, const Pose& v) {
 // Single-lane tree folding (J <= 64 joints, runs once per workgroup).
 template <int MAXA, int NEE>
 __device__ void build_problem(const IkArgs& a, const JointRec* recs, const int* slot_of,
-                              IkShared<MAXA, NEE>& sh, int* anchor, float* rel,
-                              float4* sph, int* sph_node_tmp) {
+                              IkShared<MAXA, NEE>& sh, int* anchor, float* rel) {
   const int J = a.tables.n_joints;
   int nn = 0;
   for (int i = 0; i < J; ++i) {
@@ -134,6 +134,9 @@ __device__ void build_problem(const IkArgs& a, const JointRec* recs, const int* 
     if (r.kind == 0) {
       anchor[i] = base;
       pose_to(rel + 7 * i, compose(bt, load_pose(r.ptf)));
+    } else if (nn >= MAXA) {
+      anchor[i] = nn++;  // counted only
+      pose_to(rel + 7 * i, pose_identity());
     } else {
       NodeRec& n = sh.nodes[nn];
       pose_to(n.ptf, compose(bt, load_pose(r.ptf)));
@@ -183,31 +186,69 @@ __device__ void build_problem(const IkArgs& a, const JointRec* recs, const int* 
       }
     }
   }
-  // Robot spheres, regrouped by node (group g = node + 1; group 0 = world-fixed).
-  const int K = a.enable_collision ? a.n_robot_spheres : 0;
-  int* count = sh.cnt;
-  for (int g = 0; g <= nn; ++g) count[g] = 0;
-  for (int k = 0; k < K; ++k) {
-    const int jidx = a.robot_sphere_joint[k];
+}
+
+// Robot spheres regrouped by node (group g = node + 1; group 0 = world-fixed),
+// in table order within a group, by the whole wave: every lane looks one
+// sphere's group up, and a ballot per group gives the spheres their places.
+// (On one lane the dependent table loads of K spheres took longer than an LM
+// iteration of every seed: 111 spheres, about 0.1 ms.)
+template <int MAXA, int NEE>
+__device__ void group_spheres(const IkArgs& a, const int* slot_of, IkShared<MAXA, NEE>& sh, const int* anchor,
+                              const float* rel, float4* sph, int* sph_group) {
+  const int J = a.tables.n_joints;
+  const int K = (a.enable_collision && !sh.too_many_nodes) ? a.n_robot_spheres : 0;
+  const int nn = sh.too_many_nodes ? 0 : sh.n_nodes;
+  const int lane = threadIdx.x;
+  for (int g = lane; g <= nn; g += kWave) sh.cnt[g] = 0;
+  __syncthreads();
+  for (int k0 = 0; k0 < K; k0 += kWave) {
+    const int k = k0 + lane;
     int g = -1;
-    if (jidx >= 0 && jidx < J && slot_of[jidx] >= 0) g = anchor[slot_of[jidx]] + 1;
-    sph_node_tmp[k] = g;
-    if (g >= 0) ++count[g];
+    if (k < K) {
+      const int j = a.robot_sphere_joint[k];
+      const int s = (j >= 0 && j < J) ? slot_of[j] : -1;
+      if (s >= 0) g = anchor[s] + 1;
+      sph_group[k] = g;
+    }
+    for (int c = 0; c <= nn; ++c) {
+      const int n = __popcll(__ballot(g == c));
+      if (lane == 0) sh.cnt[c] += n;
+    }
   }
-  int acc = 0;
-  for (int g = 0; g <= nn; ++g) { sh.sph_start[g] = acc; acc += count[g]; count[g] = sh.sph_start[g]; }
-  sh.sph_start[nn + 1] = acc;
-  sh.n_sph = acc;
-  for (int k = 0; k < K; ++k) {
-    const int g = sph_node_tmp[k];
-    if (g < 0) continue;
-    const int jidx = a.robot_sphere_joint[k];
-    const int s = slot_of[jidx];
-    const Pose rp = pose_from(rel + 7 * s);
-    const float* sp = a.robot_spheres + 4 * k;
-    float cx, cy, cz;
-    quat_rotate(rp.w, rp.x, rp.y, rp.z, sp[0], sp[1], sp[2], cx, cy, cz);
-    sph[count[g]++] = make_float4(cx + rp.tx, cy + rp.ty, cz + rp.tz, sp[3]);
+  __syncthreads();
+  if (lane == 0) {
+    int acc = 0;
+    for (int g = 0; g <= nn; ++g) {
+      sh.sph_start[g] = acc;
+      acc += sh.cnt[g];
+      sh.cnt[g] = sh.sph_start[g];
+    }
+    sh.sph_start[nn + 1] = acc;
+    sh.n_sph = acc;
+  }
+  __syncthreads();
+  for (int k0 = 0; k0 < K; k0 += kWave) {
+    const int k = k0 + lane;
+    const int g = (k < K) ? sph_group[k] : -1;
+    int at = -1;
+    for (int c = 0; c <= nn; ++c) {
+      const unsigned long long mask = __ballot(g == c);
+      if (g == c)
+        at = sh.cnt[c] + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                             static_cast<unsigned>(mask >> 32),
+                             __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u)));
+      __syncthreads();
+      if (lane == 0) sh.cnt[c] += __popcll(mask);
+    }
+    __syncthreads();
+    if (at >= 0) {
+      const Pose rp = pose_from(rel + 7 * slot_of[a.robot_sphere_joint[k]]);
+      const float* sp = a.robot_spheres + 4 * k;
+      float cx, cy, cz;
+      quat_rotate(rp.w, rp.x, rp.y, rp.z, sp[0], sp[1], sp[2], cx, cy, cz);
+      sph[at] = make_float4(cx + rp.tx, cy + rp.ty, cz + rp.tz, sp[3]);
+    }
   }
 }
 
@@ -423,16 +464,29 @@ __device__ __forceinline__ void group_penalty(float& pen, const Pose& T, int k0,
 
 // Penalty of the world-fixed spheres (group 0, placed by the identity): the
 // same for every seed and iteration of a problem, so the prologue evaluates
-// it once per workgroup.  It is the running sum sphere_penalty used to reach
-// after group 0, term for term, so starting from it changes no result.
+// it once per workgroup: one sphere a lane, then the spheres' terms (world
+// spheres, other shapes) added up in order, the same sum as one lane's.
+// (On one lane, 20 spheres against 256 obstacles took about 0.15 ms.)
 template <int MAXA, int NEE>
 __device__ __forceinline__ float static_sphere_penalty(const IkShared<MAXA, NEE>& sh, const float4* sph,
                                                        const float4* ws, int M, const GridArgs& grid,
                                                        const OtherWorld& ow) {
+  const int n_other = ow.nc + ow.nb + ow.nh;
   float pen = 0.f;
-  unsigned work = 0;
-  group_penalty<MAXA>(pen, pose_identity(), sh.sph_start[0], sh.sph_start[1], sph, ws, M, grid, ow,
-                      ow.nc + ow.nb + ow.nh, work);
+  for (int k0 = sh.sph_start[0]; k0 < sh.sph_start[1]; k0 += kWave) {
+    const int n = min(kWave, sh.sph_start[1] - k0);
+    float t = 0.f, u = 0.f;
+    unsigned work = 0;
+    if (static_cast<int>(threadIdx.x) < n) {
+      const float4 s = sph[k0 + threadIdx.x];
+      group_penalty<MAXA>(t, pose_identity(), k0 + threadIdx.x, k0 + threadIdx.x + 1, sph, ws, M, grid, ow, 0, work);
+      if (n_other > 0) u = other_penalty(s.x, s.y, s.z, s.w, ow);
+    }
+    for (int i = 0; i < n; ++i) {
+      pen += __shfl(t, i, kWave);
+      if (n_other > 0) pen += __shfl(u, i, kWave);
+    }
+  }
   return pen;
 }
 
@@ -533,15 +587,24 @@ struct IkView {
   OtherWorld ow;
 };
 
+// |W r|^2 at q, without the collision penalty; the node poses, residuals and
+// EE poses are left in P, r and Tee.
 template <int MAXA, int NEE>
-__device__ __forceinline__ float weighted_error(const IkView<MAXA, NEE>& v, const float (&tg)[NEE][7],
-                                                const float* W, const float* q, Pose* P, float* r,
-                                                Pose* Tee, const GridArgs& grid, unsigned& work) {
+__device__ __forceinline__ float pose_error(const IkView<MAXA, NEE>& v, const float (&tg)[NEE][7], const float* W,
+                                            const float* q, Pose* P, float* r, Pose* Tee) {
   node_fk(*v.sh, q, P);
   residuals(*v.sh, P, tg, r, Tee);
   float e = 0.f;
 #pragma unroll
   for (int i = 0; i < 6 * NEE; ++i) { const float x = r[i] * W[i % 6]; e += x * x; }
+  return e;
+}
+
+template <int MAXA, int NEE>
+__device__ __forceinline__ float weighted_error(const IkView<MAXA, NEE>& v, const float (&tg)[NEE][7],
+                                                const float* W, const float* q, Pose* P, float* r,
+                                                Pose* Tee, const GridArgs& grid, unsigned& work) {
+  float e = pose_error(v, tg, W, q, P, r, Tee);
   if (v.coll) e += v.wc * sphere_penalty(*v.sh, P, v.sph, v.ws, v.M, grid, v.ow, work);
   return e;
 }
@@ -569,14 +632,227 @@ __device__ __forceinline__ void jac_column(const Pose& Pn, const float* ax, int 
   for (int k = 0; k < 6; ++k) out6[k] = (mul * g[k]) * W[k];
 }
 
+// Collision penalty of the NP line-search points of one seed, by the whole
+// wave, to the bit the sum one lane gets by testing every robot sphere against
+// every obstacle.  That costs K x M pair tests a point (24,832 for 97 spheres
+// and 256 obstacles), nearly all of them out of reach, where the term is zero
+// and adding it changes nothing.  Here every 12 consecutive spheres of a node
+// (60 lanes at five points) carry a bounding sphere, and per such cluster:
+//   1. a ball around its bounding spheres at all the points is tested against
+//      64 obstacles at a time, one a lane;
+//   2. lanes over (sphere, point) take the obstacles in reach, read from the
+//      lane that holds them, in index order (even and odd ones summed apart,
+//      as world_penalty_all does);
+//   3. lane i adds point i's terms in sphere order.
+// 61 problems x 32 seeds of Fetch, 40 iterations, 256 obstacles: 41.6 -> 2.55
+// ms a call (2.78 with one bounding sphere per node).
+// The bounds carry slack for rounding, so a dropped pair's term is zero; the
+// tests are phrased so that a NaN keeps its pair.
+constexpr int kLineSteps = 5;
+constexpr float kNoBound = -1e30f;  // radius no obstacle reaches
+
+constexpr int kCluster = 12;
+static_assert(kCluster * kLineSteps <= kWave, "one lane per sphere and point");
+
+// Clusters of K spheres on at most n_nodes nodes.
+__host__ __device__ constexpr int max_clusters(int K, int n_nodes) { return K / kCluster + n_nodes; }
+
+template <int MAXA>
+struct PenLds {
+  float pose[kLineSteps][MAXA][7];   // node poses of the points
+  float term[kWave], other[kWave];   // per (sphere, point) of a cluster
+  int n_clusters, pad[3];
+};
+
+// The tables behind it, one entry per cluster (at: one per point and cluster).
+struct PenClusters {
+  float4* bound;  // bounding sphere, node frame
+  float4* hull;   // ball around `at` of all the points
+  float4* at;     // the bounding sphere in the world at each point
+  int* node;
+  int* first;     // first sphere; the cluster ends at the next one's or its node's
+  int max;
+};
+
+template <int MAXA>
+__host__ __device__ inline size_t pen_lds_bytes(int K) {
+  return sizeof(PenLds<MAXA>) + (sizeof(float4) * (2 + kLineSteps) + 2 * sizeof(int)) * max_clusters(K, MAXA);
+}
+
+template <int MAXA>
+__device__ __forceinline__ PenClusters pen_clusters(PenLds<MAXA>* pl, int K) {
+  PenClusters o;
+  o.max = max_clusters(K, MAXA);
+  o.bound = reinterpret_cast<float4*>(pl + 1);
+  o.hull = o.bound + o.max;
+  o.at = o.hull + o.max;
+  o.node = reinterpret_cast<int*>(o.at + kLineSteps * o.max);
+  o.first = o.node + o.max;
+  return o;
+}
+
+// Whether balls of radii b.w (a bound) and o.w can touch; the slack covers the
+// rounding of centres up to the size of the coordinates.
+__device__ __forceinline__ bool in_reach(const float4& b, const float4& o) {
+  const float dx = b.x - o.x, dy = b.y - o.y, dz = b.z - o.z;
+  float reach = b.w + o.w;
+  reach += 1e-5f + 4e-6f * (fabsf(b.x) + fabsf(b.y) + fabsf(b.z) + fabsf(reach));
+  return !(reach < 0.f) && !(dx * dx + dy * dy + dz * dz > reach * reach);
+}
+
+// The clusters and their bounding spheres (once per workgroup).
+template <int MAXA, int NEE>
+__device__ __forceinline__ void stage_clusters(const IkView<MAXA, NEE>& v, PenLds<MAXA>& pl, const PenClusters& pc) {
+  const IkShared<MAXA, NEE>& sh = *v.sh;
+  const int lane = threadIdx.x;
+  int base = 0;
+  for (int n = 0; n < sh.n_nodes; ++n) {
+    const int k0 = sh.sph_start[n + 1], ns = sh.sph_start[n + 2] - k0;
+    const int nc = (ns + kCluster - 1) / kCluster;
+    for (int c = lane; c < nc; c += kWave) {
+      const int f = k0 + c * kCluster, e = min(f + kCluster, k0 + ns);
+      float lx = INFINITY, ly = INFINITY, lz = INFINITY, hx = -INFINITY, hy = -INFINITY, hz = -INFINITY;
+      for (int k = f; k < e; ++k) {
+        const float4 s = v.sph[k];
+        lx = fminf(lx, s.x); ly = fminf(ly, s.y); lz = fminf(lz, s.z);
+        hx = fmaxf(hx, s.x); hy = fmaxf(hy, s.y); hz = fmaxf(hz, s.z);
+      }
+      float4 b = make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), kNoBound);
+      for (int k = f; k < e; ++k) {
+        const float4 s = v.sph[k];
+        const float dx = s.x - b.x, dy = s.y - b.y, dz = s.z - b.z;
+        b.w = fmaxf(b.w, sqrtf(dx * dx + dy * dy + dz * dz) + s.w);
+      }
+      pc.bound[base + c] = b;
+      pc.node[base + c] = n;
+      pc.first[base + c] = f;
+    }
+    base += nc;
+  }
+  if (lane == 0) pl.n_clusters = base;
+  wave_sync();
+}
+
+// quat_to_rot with its products' roundings spelled out, as the compiler
+// contracts it in group_penalty: in another loop it fuses other ones, and a
+// last-bit change of a penalty can send a seed another way.
+__device__ __forceinline__ Rot3 quat_to_rot_fixed(const Pose& p) {
+  const float xx = p.x * p.x, yy = p.y * p.y;
+  const float wx = p.w * p.x, wy = p.w * p.y, wz = p.w * p.z;
+  Rot3 r;
+  r.m00 = fmaf(fmaf(p.z, p.z, yy), -2.f, 1.f);
+  r.m11 = fmaf(fmaf(p.z, p.z, xx), -2.f, 1.f);
+  r.m22 = fmaf(fmaf(p.y, p.y, xx), -2.f, 1.f);
+  r.m01 = 2.f * fmaf(p.x, p.y, -wz);
+  r.m10 = 2.f * fmaf(p.x, p.y, wz);
+  r.m02 = 2.f * fmaf(p.z, p.x, wy);
+  r.m20 = 2.f * fmaf(p.z, p.x, -wy);
+  r.m12 = 2.f * fmaf(p.z, p.y, -wx);
+  r.m21 = 2.f * fmaf(p.z, p.y, wx);
+  return r;
+}
+
+// Penalties (unweighted) of the points whose node poses are in pl.pose[0 ..
+// NP); lane i < NP returns point i's, the world-fixed spheres' included.
+// Every lane of the wave takes part.
+template <int NP, int MAXA, int NEE>
+__device__ __forceinline__ float wave_penalty(const IkView<MAXA, NEE>& v, PenLds<MAXA>& pl, const PenClusters& pc) {
+  const IkShared<MAXA, NEE>& sh = *v.sh;
+  const int lane = threadIdx.x;
+  const int n_other = v.ow.nc + v.ow.nb + v.ow.nh;
+  wave_sync();
+  const int n_cl = pl.n_clusters;
+  for (int c = lane; c < n_cl; c += kWave) {
+    const int n = pc.node[c];
+    const float4 b = pc.bound[c];
+    float4 at[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const Pose T = load_pose(pl.pose[i][n]);
+      float x, y, z;
+      quat_rotate(T.w, T.x, T.y, T.z, b.x, b.y, b.z, x, y, z);
+      at[i] = make_float4(x + T.tx, y + T.ty, z + T.tz, b.w);
+    }
+    // The points lie on a segment in joint space: the middle of the first
+    // (longest step) and the last is a fair centre.
+    const float4 p = at[0], q = at[NP - 1];
+    float4 h = make_float4(0.5f * (p.x + q.x), 0.5f * (p.y + q.y), 0.5f * (p.z + q.z), 0.f);
+    float d2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const float dx = at[i].x - h.x, dy = at[i].y - h.y, dz = at[i].z - h.z;
+      const float e2 = dx * dx + dy * dy + dz * dz;
+      d2 = (e2 > d2 || e2 != e2) ? e2 : d2;
+    }
+    h.w = b.w + sqrtf(d2);
+    pc.hull[c] = h;
+  }
+  wave_sync();
+  float total = sh.static_pen;
+  for (int c = 0; c < n_cl; ++c) {
+    const int n = __builtin_amdgcn_readfirstlane(pc.node[c]);
+    const int k0 = __builtin_amdgcn_readfirstlane(pc.first[c]);
+    const int cnt = min(kCluster, sh.sph_start[n + 2] - k0) * NP;  // tasks: sphere k0 + t / NP at point t % NP
+    const float4 hull = pc.hull[c];
+    bool placed = false;
+    float cx = 0.f, cy = 0.f, cz = 0.f, r = 0.f, p0 = 0.f, p1 = 0.f;
+    auto place = [&]() {
+      const int t = min(lane, cnt - 1);
+      const Pose T = load_pose(pl.pose[t % NP][n]);
+      const Rot3 R = quat_to_rot_fixed(T);
+      const float4 s = v.sph[k0 + t / NP];
+      cx = fmaf(R.m02, s.z, fmaf(R.m00, s.x, R.m01 * s.y)) + T.tx;
+      cy = fmaf(R.m12, s.z, fmaf(R.m10, s.x, R.m11 * s.y)) + T.ty;
+      cz = fmaf(R.m22, s.z, fmaf(R.m20, s.x, R.m21 * s.y)) + T.tz;
+      r = s.w;
+      placed = true;
+    };
+    if (n_other > 0) place();
+    for (int m0 = 0; m0 < v.M; m0 += kWave) {
+      const float4 o = v.ws[min(m0 + lane, v.M - 1)];
+      const unsigned long long mask = __ballot(m0 + lane < v.M && in_reach(hull, o));
+      if (mask == 0) continue;
+      if (!placed) place();
+      auto one = [&](int j, float& p) {
+        const float ax = cx - __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o.x), j));
+        const float ay = cy - __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o.y), j));
+        const float az = cz - __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o.z), j));
+        const float e0 = fminf(__builtin_amdgcn_sqrtf(fmaf(az, az, fmaf(ax, ax, ay * ay))) -
+                                   __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o.w), j)) - r, 0.f);
+        p = fmaf(e0, e0, p);
+      };
+      for (unsigned long long m = mask & 0x5555555555555555ull; m != 0; m &= m - 1) one(__builtin_ctzll(m), p0);
+      for (unsigned long long m = mask & 0xaaaaaaaaaaaaaaaaull; m != 0; m &= m - 1) one(__builtin_ctzll(m), p1);
+    }
+    if (!placed) continue;  // every term is zero
+    pl.term[lane] = p0 + p1;
+    if (n_other > 0) pl.other[lane] = other_penalty(cx, cy, cz, r, v.ow);
+    wave_sync();
+    if (lane < NP) {
+      for (int i = lane; i < cnt; i += NP) {
+        total += pl.term[i];
+        if (n_other > 0) total += pl.other[i];
+      }
+    }
+    wave_sync();
+  }
+  return total;
+}
+
 // LM iterations [it0, it1) of one seed (the algorithm in the file header).
 // G = 1: one lane per seed.  G = 8: the 8 lanes of an aligned group hold the
 // same seed, compute the same step, and lane k evaluates line-search step k
 // (k < 5); an argmin over the group gives every lane the sequential pick.
-template <int MAXA, int NEE, int G = 1>
+// COOP (G = 8): the wave's n_groups seeds share the collision penalty seed by
+// seed (wave_penalty), so a lane whose seed is done stays for the others' and
+// st.best_err holds the first iterate's error on entry.
+template <int MAXA, int NEE, int G = 1, bool COOP = false>
 __device__ __forceinline__ void lm_iterate(const IkView<MAXA, NEE>& v, const float (&tg)[NEE][7],
                                            const float* W, const IkArgs& a, LmState<MAXA>& st,
-                                           int it0, int it1, const GridArgs& grid) {
+                                           int it0, int it1, const GridArgs& grid,
+                                           PenLds<MAXA>* pl = nullptr, const PenClusters* pc = nullptr,
+                                           int n_groups = 0) {
+  static_assert(!COOP || G == 8, "the penalty is shared among groups of 8 lanes");
   const IkShared<MAXA, NEE>& sh = *v.sh;
   Pose P[MAXA];
   Pose Tee[NEE];
@@ -590,8 +866,16 @@ __device__ __forceinline__ void lm_iterate(const IkView<MAXA, NEE>& v, const flo
   // the accepted point as well, instead of being recomputed.
   constexpr bool kReuse = (G == 8) && (MAXA == 8);
   bool have = false;
-  float cur_next = 0.f;
-  for (int it = it0; it < it1 && !st.done; ++it) {
+  float cur_next = COOP ? st.best_err : 0.f;
+  for (int it = it0; it < it1; ++it) {
+    if (COOP ? !__any(!st.done) : st.done != 0) break;
+    bool live = !COOP || !st.done;
+    float delta[MAXA];
+    float cur = 0.f;
+    Pose P2[MAXA], Tee2[NEE];
+    float r2[6 * NEE];
+    float et = 0.f;
+    if (live) {
     if (!kReuse || !have) {
       node_fk(sh, st.q, P);
       residuals(sh, P, tg, r, Tee);
@@ -606,13 +890,16 @@ __device__ __forceinline__ void lm_iterate(const IkView<MAXA, NEE>& v, const flo
       max_p = fmaxf(max_p, np);
       max_o = fmaxf(max_o, no);
     }
-    if (conv) { st.done = 1; break; }
-
-    float cur = 0.f;
+    if (conv) {
+      st.done = 1;
+      if (!COOP) break;
+      live = false;
+    }
+    if (live) {
     float fw[6 * NEE];
 #pragma unroll
     for (int i = 0; i < 6 * NEE; ++i) { fw[i] = r[i] * W[i % 6]; cur += fw[i] * fw[i]; }
-    if (have) {
+    if (have || COOP) {
       cur = cur_next;  // the same sum (and penalty) the line search evaluated
     } else if (v.coll) {
       // With G lanes per seed every lane computes the same value; the work
@@ -733,7 +1020,6 @@ __device__ __forceinline__ void lm_iterate(const IkView<MAXA, NEE>& v, const flo
       for (int pp = 0; pp < i; ++pp) t -= A[i * (i + 1) / 2 + pp] * y[pp];
       y[i] = t * idg[i];
     }
-    float delta[MAXA];
 #pragma unroll
     for (int i = MAXA - 1; i >= 0; --i) {
       float t = y[i];
@@ -760,6 +1046,40 @@ __device__ __forceinline__ void lm_iterate(const IkView<MAXA, NEE>& v, const flo
       for (int i = 0; i < MAXA; ++i) delta[i] *= sc;
     }
 
+    if (G != 1) {
+      const int ai = min(static_cast<int>(threadIdx.x % G), 4);
+      float qt[MAXA];
+#pragma unroll
+      for (int i = 0; i < MAXA; ++i) qt[i] = fmaxf(sh.lo[i], fminf(sh.hi[i], st.q[i] + ls_alpha(ai) * delta[i]));
+      unsigned wk = 0;
+      if (COOP)
+        et = pose_error(v, tg, W, qt, P2, r2, Tee2);
+      else
+        et = kReuse ? weighted_error(v, tg, W, qt, P2, r2, Tee2, grid, wk)
+                    : weighted_error(v, tg, W, qt, P, r, Tee, grid, wk);
+      if (threadIdx.x % G < 5) st.work += wk;  // lanes 5..7 repeat step 4
+    }
+    }
+    }
+    if (COOP && v.coll) {
+      const unsigned long long lives = __ballot(live);
+      const int g = threadIdx.x / G, k = threadIdx.x % G;
+      float pen = 0.f;
+      for (int j = 0; j < n_groups; ++j) {
+        if (!((lives >> (G * j)) & 1)) continue;
+        wave_sync();
+        if (g == j && k < kLineSteps) {
+#pragma unroll
+          for (int n = 0; n < MAXA; ++n)
+            if (n < sh.n_nodes) pose_to(pl->pose[k][n], P2[n]);
+        }
+        const float p = __shfl(wave_penalty<kLineSteps, MAXA, NEE>(v, *pl, *pc), min(k, kLineSteps - 1), kWave);
+        if (g == j) pen = p;
+      }
+      et += v.wc * pen;
+    }
+    if (!live) continue;
+
     // Line search: evaluate all five steps, keep the best (the first on ties).
     float best_a_err = 1e30f;
     int best_a = 0;
@@ -775,15 +1095,6 @@ __device__ __forceinline__ void lm_iterate(const IkView<MAXA, NEE>& v, const flo
     } else {
       static_assert(G == 1 || G == 8, "line-search groups are 1 or 8 lanes");
       const int ai = min(static_cast<int>(threadIdx.x % G), 4);
-      float qt[MAXA];
-#pragma unroll
-      for (int i = 0; i < MAXA; ++i) qt[i] = fmaxf(sh.lo[i], fminf(sh.hi[i], st.q[i] + ls_alpha(ai) * delta[i]));
-      unsigned wk = 0;
-      Pose P2[MAXA], Tee2[NEE];
-      float r2[6 * NEE];
-      const float et = kReuse ? weighted_error(v, tg, W, qt, P2, r2, Tee2, grid, wk)
-                              : weighted_error(v, tg, W, qt, P, r, Tee, grid, wk);
-      if (threadIdx.x % G < 5) st.work += wk;  // lanes 5..7 repeat step 4
       // Sequential semantics: only errors below 1e30 replace the start value
       // (NaN never does); the first index wins ties.
       float e = (et < 1e30f) ? et : INFINITY;
@@ -841,7 +1152,9 @@ __device__ __forceinline__ IkView<MAXA, NEE> ik_prologue(const IkArgs& a, char* 
   float4* ws = reinterpret_cast<float4*>(base + off.ws);
   const int lane = threadIdx.x;
   stage_joint_records(a.tables, recs, slot_of);
-  if (lane == 0) build_problem<MAXA, NEE>(a, recs, slot_of, sh, anchor, rel, sph, sph_tmp);
+  if (lane == 0) build_problem<MAXA, NEE>(a, recs, slot_of, sh, anchor, rel);
+  __syncthreads();
+  group_spheres<MAXA, NEE>(a, slot_of, sh, anchor, rel, sph, sph_tmp);
   for (int i = lane; i < MAXA; i += kWave) {
     const bool real = i < a.n_act;
     sh.lo[i] = real ? a.lower[i] : 0.f;
@@ -873,7 +1186,8 @@ __device__ __forceinline__ IkView<MAXA, NEE> ik_prologue(const IkArgs& a, char* 
   v.ow.margin = a.collision_margin;
   v.coll = (M > 0 || n_oth > 0) && sh.n_sph > 0;
   v.wc = a.collision_weight;
-  if (lane == 0) sh.static_pen = v.coll ? static_sphere_penalty(sh, sph, ws, M, a.grid, v.ow) : 0.f;
+  const float static_pen = v.coll ? static_sphere_penalty(sh, sph, ws, M, a.grid, v.ow) : 0.f;
+  if (lane == 0) sh.static_pen = static_pen;
   __syncthreads();
   return v;
 }
@@ -887,17 +1201,30 @@ __device__ __forceinline__ void load_targets(const IkArgs& a, long long problem,
       tg[e][c] = (e < a.n_ee) ? a.target_T[(problem * a.n_ee + e) * 7 + c] : (c == 0 ? 1.f : 0.f);
 }
 
+// Offset of the shared penalty's tables in the LDS of ls_ik_kernel, after the
+// problem's.
+template <int MAXA, int NEE>
+__host__ __device__ inline size_t pen_lds_offset(const IkArgs& a) {
+  const int K = a.enable_collision ? a.n_robot_spheres : 0;
+  return align16(ik_lds_layout(sizeof(IkShared<MAXA, NEE>), a.tables.n_joints, K, a.enable_collision ? a.n_world : 0,
+                               ik_other_floats(a)).total);
+}
+
 // G lanes per seed (see lm_iterate); the group's first lane writes the result.
-template <int MAXA, int NEE, int G>
+template <int MAXA, int NEE, int G, bool COOP>
 __global__ __launch_bounds__(64) void ls_ik_kernel(IkArgs a) {
   extern __shared__ float4 smem4[];
   const IkView<MAXA, NEE> v = ik_prologue<MAXA, NEE>(a, reinterpret_cast<char*>(smem4));
   const int lane = threadIdx.x;
   const int p = blockIdx.y;
-  const int s = blockIdx.x * (kWave / G) + lane / G;
-  const bool writer = (lane % G) == 0;
-  if (s >= a.n_seeds) return;
-  const long long gs = static_cast<long long>(p) * a.n_seeds + s;
+  // COOP: grid.x covers the seeds in steps of a.seeds_per_wave, at most 64 / G;
+  // the lanes past them only take part in the shared penalty.
+  const int per_wave = COOP ? a.seeds_per_wave : kWave / G;
+  const int s = blockIdx.x * per_wave + lane / G;
+  const bool valid = s < a.n_seeds && lane / G < per_wave;
+  const bool writer = valid && (lane % G) == 0;
+  if (!COOP && !valid) return;
+  const long long gs = static_cast<long long>(p) * a.n_seeds + (valid ? s : a.n_seeds - 1);
   if (v.sh->too_many_nodes) {  // reported to the caller as NaN errors, seeds unchanged
     if (writer) {
       for (int i = 0; i < a.n_act; ++i) a.out_cfgs[gs * a.n_act + i] = a.seeds[gs * a.n_act + i];
@@ -918,10 +1245,33 @@ __global__ __launch_bounds__(64) void ls_ik_kernel(IkArgs a) {
   Pose Tee[NEE];
   float r[6 * NEE];
   st.work = 0;
-  st.best_err = weighted_error(v, tg, W, st.q, P, r, Tee, a.grid, st.work);
   st.lam = a.lambda_init;
-  st.done = 0;
-  lm_iterate<MAXA, NEE, G>(v, tg, W, a, st, 0, a.max_iter, a.grid);
+  st.done = valid ? 0 : 1;
+  if constexpr (COOP) {
+    PenLds<MAXA>* pl = reinterpret_cast<PenLds<MAXA>*>(reinterpret_cast<char*>(smem4) + pen_lds_offset<MAXA, NEE>(a));
+    const PenClusters pc = pen_clusters<MAXA>(pl, a.enable_collision ? a.n_robot_spheres : 0);
+    const int n_groups = min(per_wave, a.n_seeds - static_cast<int>(blockIdx.x) * per_wave);
+    st.best_err = pose_error(v, tg, W, st.q, P, r, Tee);
+    if (v.coll) {
+      stage_clusters<MAXA, NEE>(v, *pl, pc);
+      float pen = 0.f;
+      for (int j = 0; j < n_groups; ++j) {
+        wave_sync();
+        if (lane == G * j) {
+#pragma unroll
+          for (int n = 0; n < MAXA; ++n)
+            if (n < v.sh->n_nodes) pose_to(pl->pose[0][n], P[n]);
+        }
+        const float x = __shfl(wave_penalty<1, MAXA, NEE>(v, *pl, pc), 0, kWave);
+        if (lane / G == j) pen = x;
+      }
+      st.best_err += v.wc * pen;
+    }
+    lm_iterate<MAXA, NEE, G, true>(v, tg, W, a, st, 0, a.max_iter, a.grid, pl, &pc, n_groups);
+  } else {
+    st.best_err = weighted_error(v, tg, W, st.q, P, r, Tee, a.grid, st.work);
+    lm_iterate<MAXA, NEE, G>(v, tg, W, a, st, 0, a.max_iter, a.grid);
+  }
   if (writer) {
 #pragma unroll
     for (int i = 0; i < MAXA; ++i)
@@ -972,6 +1322,15 @@ inline long long wave_seed_limit() {
   return limit;
 }
 
+// Seeds of one wave when they share the collision penalty, whose cost grows
+// with them while the LM step's does not: as many as keep at most two waves
+// per SIMD, up to the 8 groups of 8 lanes.
+inline int coop_seeds_per_wave(long long n_all) {
+  int n = 1;
+  while (n < 8 && n_all > 2 * wave_seed_limit() * n) n *= 2;
+  return n;
+}
+
 template <int MAXA, int NEE>
 __device__ __forceinline__ void store_iterate(WaveLds<MAXA, NEE>& wl, const Pose* P, const Pose* Tee, const float* r) {
 #pragma unroll
@@ -985,9 +1344,9 @@ __device__ __forceinline__ void store_iterate(WaveLds<MAXA, NEE>& wl, const Pose
 template <int MAXA, int NEE>
 __device__ __forceinline__ void lm_iterate_wave(const IkView<MAXA, NEE>& v, const float (&tg)[NEE][7],
                                                 const float* W, const IkArgs& a, LmState<MAXA>& st,
-                                                WaveLds<MAXA, NEE>& wl, float cur_next) {
+                                                WaveLds<MAXA, NEE>& wl, PenLds<MAXA>* pl, const PenClusters& pc,
+                                                float cur_next) {
   const IkShared<MAXA, NEE>& sh = *v.sh;
-  const GridArgs& grid = a.grid;
   const int lane = threadIdx.x;
   constexpr int NT = MAXA * (MAXA + 1) / 2;
   for (int it = 0; it < a.max_iter && !st.done; ++it) {
@@ -1145,10 +1504,19 @@ __device__ __forceinline__ void lm_iterate_wave(const IkView<MAXA, NEE>& v, cons
       float qt[MAXA];
 #pragma unroll
       for (int i = 0; i < MAXA; ++i) qt[i] = fmaxf(sh.lo[i], fminf(sh.hi[i], st.q[i] + ls_alpha(ai) * delta[i]));
-      unsigned wk = 0;
-      const float et = weighted_error(v, tg, W, qt, P2, r2, Tee2, grid, wk);
-      e = (et < 1e30f) ? et : INFINITY;
+      e = pose_error(v, tg, W, qt, P2, r2, Tee2);
       idx = ai;
+      if (v.coll && lane < kLineSteps) {
+#pragma unroll
+        for (int n = 0; n < MAXA; ++n) pose_to(pl->pose[lane][n], P2[n]);
+      }
+    }
+    if (v.coll) {
+      const float pen = wave_penalty<kLineSteps, MAXA, NEE>(v, *pl, pc);
+      e = (lane < kLineSteps) ? e + v.wc * pen : INFINITY;
+    }
+    if (lane < 8) {
+      e = (e < 1e30f) ? e : INFINITY;
       ls_argmin_step<0xb1>(e, idx);   // quad_perm [1,0,3,2]
       ls_argmin_step<0x4e>(e, idx);   // quad_perm [2,3,0,1]
       ls_argmin_step<0x141>(e, idx);  // row_half_mirror
@@ -1190,6 +1558,8 @@ __global__ __launch_bounds__(64) void ls_ik_wave_kernel(IkArgs a) {
   const IkLds off = ik_lds_layout(sizeof(Sh), a.tables.n_joints, Kin, a.enable_collision ? a.n_world : 0,
                                   ik_other_floats(a));
   WaveLds<MAXA, NEE>& wl = *reinterpret_cast<WaveLds<MAXA, NEE>*>(base + align16(off.total));
+  PenLds<MAXA>* pl = reinterpret_cast<PenLds<MAXA>*>(base + align16(align16(off.total) + sizeof(wl)));
+  const PenClusters pc = pen_clusters<MAXA>(pl, Kin);
   const int lane = threadIdx.x;
   const int p = blockIdx.y;
   const int s = blockIdx.x;
@@ -1222,11 +1592,20 @@ __global__ __launch_bounds__(64) void ls_ik_wave_kernel(IkArgs a) {
   Pose Tee[NEE];
   float r[6 * NEE];
   st.work = 0;
-  st.best_err = weighted_error(v, tg, W, st.q, P, r, Tee, a.grid, st.work);
+  st.best_err = pose_error(v, tg, W, st.q, P, r, Tee);
   if (lane == 0) store_iterate<MAXA, NEE>(wl, P, Tee, r);
+  if (v.coll) {
+    stage_clusters<MAXA, NEE>(v, *pl, pc);
+    if (lane == 0) {
+#pragma unroll
+      for (int n = 0; n < MAXA; ++n) pose_to(pl->pose[0][n], P[n]);
+    }
+    const float pen = wave_penalty<1, MAXA, NEE>(v, *pl, pc);
+    st.best_err += v.wc * __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(pen)));
+  }
   st.lam = a.lambda_init;
   st.done = 0;
-  lm_iterate_wave<MAXA, NEE>(v, tg, W, a, st, wl, st.best_err);
+  lm_iterate_wave<MAXA, NEE>(v, tg, W, a, st, wl, pl, pc, st.best_err);
   if (lane == 0) {
 #pragma unroll
     for (int i = 0; i < MAXA; ++i)
@@ -1332,26 +1711,36 @@ inline int launch_ik(void* stream, const IkArgs& a, bool batched, int grid_waves
   // seed's iterations: the 8-wide instantiations give each seed a wave while
   // every SIMD holds at most one of them, and every instantiation gives
   // each seed 8 lanes (parallel line search) while the lanes still fit one
-  // pass of the CUs at two waves per SIMD.
+  // pass of the CUs at two waves per SIMD.  Both share the collision penalty
+  // over the wave while its tables fit the LDS.
   const long long n_all = static_cast<long long>(a.n_problems) * a.n_seeds;
-  if (MAXA == 8 && n_all <= wave_seed_limit()) {
-    const size_t lds_w = align16(lds) + sizeof(WaveLds<MAXA, NEE>);
-    PK_REQUIRE(lds_w <= 150 * 1024, "IK tables need %zu bytes of LDS (limit 150 KiB)", lds_w);
-    dim3 grid(a.n_seeds, a.n_problems);
-    hipLaunchKernelGGL((ls_ik_wave_kernel<MAXA, NEE>), grid, dim3(kWave), lds_w,
-                       static_cast<hipStream_t>(stream), a);
-    return check_launch("ls_ik_wave_kernel");
+  const bool coll = Kin > 0 && M + a.n_caps + a.n_boxes + a.n_hs > 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if constexpr (MAXA == 8) {
+    const size_t tables = align16(lds) + sizeof(WaveLds<MAXA, NEE>);
+    const size_t lds_w = align16(tables) + (coll ? pen_lds_bytes<MAXA>(Kin) : 0);
+    if (n_all <= wave_seed_limit()) PK_REQUIRE(tables <= 150 * 1024, "IK tables need %zu bytes of LDS (limit 150 KiB)", tables);
+    if (n_all <= wave_seed_limit() && lds_w <= 160 * 1024) {
+      dim3 grid(a.n_seeds, a.n_problems);
+      hipLaunchKernelGGL((ls_ik_wave_kernel<MAXA, NEE>), grid, dim3(kWave), lds_w, s, a);
+      return check_launch("ls_ik_wave_kernel");
+    }
   }
-  const long long lanes8 = n_all * 8;
-  if (lanes8 <= kSmallBatchLanes) {
+  if (n_all * 8 <= kSmallBatchLanes) {
     constexpr int G = 8;
-    dim3 grid((a.n_seeds + kWave / G - 1) / (kWave / G), a.n_problems);
-    hipLaunchKernelGGL((ls_ik_kernel<MAXA, NEE, G>), grid, dim3(kWave), lds,
-                       static_cast<hipStream_t>(stream), a);
+    const size_t lds_c = pen_lds_offset<MAXA, NEE>(a) + pen_lds_bytes<MAXA>(Kin);
+    if (coll && lds_c <= 150 * 1024) {
+      IkArgs b = a;
+      b.seeds_per_wave = coop_seeds_per_wave(n_all);
+      dim3 grid((a.n_seeds + b.seeds_per_wave - 1) / b.seeds_per_wave, a.n_problems);
+      hipLaunchKernelGGL((ls_ik_kernel<MAXA, NEE, G, true>), grid, dim3(kWave), lds_c, s, b);
+    } else {
+      dim3 grid((a.n_seeds + kWave / G - 1) / (kWave / G), a.n_problems);
+      hipLaunchKernelGGL((ls_ik_kernel<MAXA, NEE, G, false>), grid, dim3(kWave), lds, s, a);
+    }
   } else {
     dim3 grid((a.n_seeds + kWave - 1) / kWave, a.n_problems);
-    hipLaunchKernelGGL((ls_ik_kernel<MAXA, NEE, 1>), grid, dim3(kWave), lds,
-                       static_cast<hipStream_t>(stream), a);
+    hipLaunchKernelGGL((ls_ik_kernel<MAXA, NEE, 1, false>), grid, dim3(kWave), lds, s, a);
   }
   return check_launch("ls_ik_kernel");
 }

@@ -1,0 +1,44 @@
+"""The wave-shared collision penalty of the multi-seed LM against the FP64 oracle, where
+its culling can go wrong: world sizes around the 64 obstacles of a pass, obstacles crowded
+round the base (every pair in reach, so the pair list is emptied several times), radii
+that swallow the robot, and robots of six to eight joints."""
+
+import numpy as np
+import pytest
+from conftest import load_robot, random_cfgs
+
+from pyroffi_amd.collision import RobotCollisionSpherized
+from pyroffi_amd.optimization_engines._ls_ik import ee_tables, ls_ik_run, prepare_ls_collision_buffers
+
+pytestmark = pytest.mark.gpu
+
+HAND = {"panda": "panda_hand", "ur5": "ee_link", "fetch": "gripper_link"}
+
+
+@pytest.mark.parametrize("name,m,extent,r_hi", [
+    ("panda", 1, 1.0, 0.15), ("panda", 63, 1.0, 0.15), ("ur5", 64, 1.0, 0.15), ("fetch", 65, 1.0, 0.15),
+    ("fetch", 300, 0.4, 0.1), ("panda", 1000, 0.3, 0.05), ("ur5", 5, 1.0, 3.0), ("panda", 40, 1000.0, 0.1)])
+def test_wave_penalty_matches_oracle(oracle_mod, name, m, extent, r_hi):
+    """Errors of the seeds (one point a wave) and after one step (five points of the line
+    search).  FP32 sums of some thousand hinge terms: 1e-4 relative.  A step whose two best
+    points tie to rounding may pick either, so 1% of the seeds may differ."""
+    robot, path = load_robot(name)
+    links = (robot.links.names.index(HAND[name]),)
+    t = oracle_mod.Tables.of(robot)
+    rng = np.random.default_rng(17)
+    lo, hi = robot.joints.lower_limits, robot.joints.upper_limits
+    tgt = oracle_mod.fk_links(t, random_cfgs(robot, 3, seed=18))[:, list(links)]
+    seeds = rng.uniform(lo, hi, (3, 70, len(lo))).astype(np.float32)
+    world = np.concatenate([rng.uniform(-extent, extent, (m, 3)), rng.uniform(0.02, r_hi, (m, 1))], 1)
+    rs, rj, ws, ok = prepare_ls_collision_buffers(robot, RobotCollisionSpherized.from_urdf(path),
+                                                  world.astype(np.float32))
+    assert ok
+    okw = dict(robot_spheres=rs, sphere_joint=rj, world=ws, enable_collision=True, collision_weight=1e4,
+               collision_margin=0.02)
+    for iters in (0, 1):
+        _, errs = ls_ik_run(robot, seeds, tgt, links, max_iter=iters, lambda_init=1e-2,
+                            collision=(rs, rj, ws, 1e4, 0.02))
+        _, oerrs = oracle_mod.ls_ik(t, seeds, *ee_tables(robot, links), tgt, lo, hi, max_iter=iters,
+                                    lambda_init=1e-2, **okw)
+        close = np.isclose(errs.cpu().numpy(), oerrs, rtol=1e-4, atol=1e-5)
+        assert close.all() if iters == 0 else close.mean() >= 0.99, (iters, close.mean())
