@@ -285,6 +285,18 @@ int pk_sphere_distances_jax_f32(void* stream, const float* link_poses, int64_t b
                                 float* out_self);
 
 /*
+ * The same distances as collision costs: each d is written as
+ *   min(c, 0) * weight,  c = d' - half  (d' < 0)  or  quad * (d' - margin)^2,
+ * d' = min(d, margin) -- colldist_from_sdf with half = margin / 2 and
+ * quad = -0.5 / (margin + 1e-6).
+ */
+int pk_sphere_costs_jax_f32(void* stream, const float* link_poses, int64_t batch, int32_t n_links,
+                            const float* spheres_padded, int32_t s_per_link, const float* world_spheres,
+                            int32_t n_world_spheres, const int32_t* pair_i, const int32_t* pair_j,
+                            int32_t n_pairs, float margin, float half, float quad, float weight,
+                            float* out_world, float* out_self);
+
+/*
  * Fused sphere sweep from link poses (no reference counterpart as one call:
  * it fuses what CUDARobotCollisionChecker does in three steps -- the vmapped
  * sphere transform, AoS->SoA transposes and the two distance kernels

@@ -129,8 +129,8 @@ class CUDARobotCollisionChecker:
             self.set_world(world_geom)
         return self._ws
 
-    def _links_world(self, model, robot, cfg):
-        """Mixed-kind world distances ``(batch, back, (B, L, M), (B,))`` of a spherized model."""
+    def _links_world(self, model, robot, cfg, *, world_min: bool):
+        """Mixed-kind world distances ``(batch, back, (B, L, M), (B,) or None)`` of a spherized model."""
         from .._robot import _to_cuda
         from ..kernels.ops import sphere_world_links
 
@@ -139,7 +139,7 @@ class CUDARobotCollisionChecker:
         batch = tuple(x.shape[:-1])
         poses = robot.forward_kinematics(x.reshape(-1, x.shape[-1]))
         t = model.device_tables(poses.device)
-        ow, om = sphere_world_links(poses, t["spheres_padded"], self._world)
+        ow, om = sphere_world_links(poses, t["spheres_padded"], self._world, world_min=world_min)
         return batch, back, ow, om
 
     def _world_of(self, model, robot, cfg, *, full: bool):
@@ -152,7 +152,7 @@ class CUDARobotCollisionChecker:
             ow = collision_world_capsule(c, w["spheres"], w["capsules"], w["boxes"], w["halfspaces"])
             return batch, back, ow, (None if full else row_min(ow))
         if self._mixed:
-            return self._links_world(model, robot, cfg)
+            return self._links_world(model, robot, cfg, world_min=not full)
         if full:
             batch, back, ow, _, _ = model._sweep(robot, cfg, self._ws, world=True)
             return batch, back, ow, None

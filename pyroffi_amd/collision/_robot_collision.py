@@ -223,7 +223,7 @@ class RobotCollisionSpherized:
             raise ValueError(f"semantics must be one of {self.SEMANTICS}, got {sem!r}")
         return sem
 
-    def _jax_distances(self, robot, cfg, world_arr, *, world: bool, self_pairs: bool):
+    def _jax_distances(self, robot, cfg, world_arr, *, world: bool, self_pairs: bool, cost=None):
         from .._robot import _to_cuda
         from ..kernels.ops import sphere_distances_jax
 
@@ -234,8 +234,25 @@ class RobotCollisionSpherized:
         t = self.device_tables(poses.device)
         ws = world_arr if world_arr is not None else torch.zeros((0, 4), device=poses.device)
         ow, osf = sphere_distances_jax(poses, t["spheres_padded"], ws, t["pair_i"], t["pair_j"], world=world,
-                                       self_pairs=self_pairs)
+                                       self_pairs=self_pairs, cost=cost)
         return batch, back, ow, osf
+
+    def _collision_rows(self, robot, cfg, margin: float, weight: float, world_geom=None):
+        """``colldist_from_sdf(d, margin) * weight`` of every distance d under the JAX conventions, flattened,
+        the distances themselves never leaving the kernel: of the world distances, or without
+        ``world_geom`` of the self distances.  None for a world that is not all spheres."""
+        from ._hip_collision import world_arrays
+
+        ws = None
+        if world_geom is not None:
+            arrs = world_arrays(world_geom)
+            if any(v.shape[0] for k, v in arrs.items() if k != "spheres"):
+                return None
+            ws = torch.as_tensor(arrs["spheres"], device="cuda")
+        _, back, ow, osf = self._jax_distances(robot, cfg, ws, world=ws is not None, self_pairs=ws is None,
+                                               cost=(margin, weight))
+        out = (osf if ws is None else ow).flatten()
+        return back(out) if isinstance(cfg, torch.Tensor) else out
 
     def compute_world_collision_distance(self, robot, cfg, world_geom, semantics: str | None = None):
         """``(*batch, N, M)``: per link, min over its spheres of the sphere-sphere distance."""
@@ -253,7 +270,8 @@ class RobotCollisionSpherized:
             self._check_robot(robot)
             x, back = _to_cuda(cfg)
             poses = robot.forward_kinematics(x.reshape(-1, x.shape[-1]))
-            ow, _ = sphere_world_links(poses, self.device_tables(poses.device)["spheres_padded"], arrs)
+            ow, _ = sphere_world_links(poses, self.device_tables(poses.device)["spheres_padded"], arrs,
+                                       world_min=False)
             return back(ow.reshape(*x.shape[:-1], self.num_links, ow.shape[-1]))
         ws = torch.as_tensor(world_sphere_array(world_geom), device="cuda")
         if sem == "jax":

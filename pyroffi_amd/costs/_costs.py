@@ -31,6 +31,7 @@ import numpy as np
 import torch
 
 from ..collision._collision import colldist_from_sdf
+from ..collision._robot_collision import RobotCollisionSpherized
 
 __all__ = ["pose_cost", "self_collision_cost", "world_collision_cost", "se3_log_t", "JAXLS_FACTORIES"]
 
@@ -115,9 +116,22 @@ def pose_cost(vals, robot, joint_var, target_pose, target_link_index, pos_weight
     return torch.cat([residual[..., :3] * pw, residual[..., 3:] * ow]).flatten()
 
 
+def _fused_rows(robot_coll, robot, cfg, margin, weight, world_geom=None):
+    """The activated distances from the distance kernels themselves, or None where the general path is
+    needed: another model or convention, a margin or weight that is not a plain number."""
+    if type(robot_coll) is not RobotCollisionSpherized or robot_coll.semantics != "jax":
+        return None
+    if not all(isinstance(v, (int, float)) and abs(v) < 1e30 for v in (margin, weight)):
+        return None
+    return robot_coll._collision_rows(robot, cfg, float(margin), float(weight), world_geom)
+
+
 def self_collision_cost(vals, robot, robot_coll, joint_var, margin: float, weight) -> torch.Tensor:
     """``colldist_from_sdf(self distances, margin) * weight``, flattened
     (``src/pyroffi/costs/_costs.py:169-182``)."""
+    rows = _fused_rows(robot_coll, robot, _cfg(vals, joint_var), margin, weight)
+    if rows is not None:
+        return rows
     d = robot_coll.compute_self_collision_distance(robot, _cfg(vals, joint_var))
     d = d if isinstance(d, torch.Tensor) else torch.as_tensor(np.asarray(d), device="cuda")
     return (colldist_from_sdf(d, margin) * weight).flatten()
@@ -126,6 +140,10 @@ def self_collision_cost(vals, robot, robot_coll, joint_var, margin: float, weigh
 def world_collision_cost(vals, robot, robot_coll, joint_var, world_geom, margin: float, weight) -> torch.Tensor:
     """``colldist_from_sdf(world distances, margin) * weight``, flattened
     (``src/pyroffi/costs/_costs.py:185-199``)."""
+    if world_geom is not None:
+        rows = _fused_rows(robot_coll, robot, _cfg(vals, joint_var), margin, weight, world_geom)
+        if rows is not None:
+            return rows
     d = robot_coll.compute_world_collision_distance(robot, _cfg(vals, joint_var), world_geom)
     d = d if isinstance(d, torch.Tensor) else torch.as_tensor(np.asarray(d), device="cuda")
     return (colldist_from_sdf(d, margin) * weight).flatten()

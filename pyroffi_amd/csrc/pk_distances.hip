@@ -11,6 +11,8 @@
 #include "pk_geom.h"
 #include "pk_model.h"
 
+#include <algorithm>
+
 namespace pk {
 
 constexpr float kNoSphere = 1e9f;  // the reference's "no sphere" value
@@ -61,6 +63,332 @@ __global__ __launch_bounds__(256) void world_reduced_mixed_kernel(const float* _
   }
 }
 
+// The JAX distance of two spheres (src/pyroffi/collision/_geometry_pairs.py:59-68
+// with the 1e-6 added to each component inside the norm, _utils.py:45):
+// |(p2 - p1) + 1e-6| - (r1 + r2).  Padding radii (-1e9) take part as they do
+// in JAX and make the distance about +1e9.
+__device__ __forceinline__ float jax_sphere_dist(float x1, float y1, float z1, float r1, float x2, float y2,
+                                                 float z2, float r2) {
+  const float dx = (x2 - x1) + 1e-6f, dy = (y2 - y1) + 1e-6f, dz = (z2 - z1) + 1e-6f;
+  return sqrtf(dx * dx + dy * dy + dz * dz) - (r1 + r2);
+}
+
+// ---------------------------------------------------------------------------
+// Per-link distances from link poses, out[b, l, m] = min over the link's
+// spheres of the distance to obstacle m, in both conventions.
+//
+// An output element takes a handful of sphere tests and four bytes of write,
+// so the work is the tests, not the write.  With one lane per element placing
+// the link's spheres for itself (33 flop a sphere, padding slots included) the
+// placement was most of the kernel: 403 us for 4099 Fetch configurations x 200
+// obstacles (28 slots a link, 6.5 of them real), 410 us for 8191 UR5 ones x 195
+// mixed obstacles.  Here a workgroup sorts the table once (by radius within a
+// link, padding folded), places a configuration's spheres into LDS once, and
+// its lanes run over (link, obstacle) with the spheres as near-broadcast LDS
+// reads; spheres of one radius share a square root (sqrt and the subtraction
+// are monotone, so the minimum is the same).  Obstacle kinds are taken one
+// after the other, so the lanes of a wave test the same kind.  (The calls at
+// those sizes: both collision residuals of Fetch 617 -> 208 us, the distances
+// written as costs; the mixed world of UR5 491 -> 198 us.)
+// ---------------------------------------------------------------------------
+
+constexpr int kRowThreads = 256;
+constexpr int kRowSlots = 2048;  // L * S slots the LDS tables hold (two float4 each)
+
+// Activation of a distance into a collision cost: min(c(d), 0) * weight with
+// c = d - half below zero, else quad (d - margin)^2, d capped at the margin
+// (colldist_from_sdf).
+struct RowCost {
+  int on;
+  float margin, half, quad, weight;
+};
+
+__device__ __forceinline__ float row_cost(const RowCost& c, float dist) {
+  const float d = fminf(dist, c.margin);
+  const float v = d < 0.f ? d - c.half : c.quad * ((d - c.margin) * (d - c.margin));
+  return fminf(v, 0.f) * c.weight;
+}
+
+struct RowArgs {
+  const float* poses;  // (B, L, 7)
+  long long batch;
+  int n_links, s_per_link;
+  const float* table;  // (L, S, 4) link-frame spheres
+  WorldPrims w;
+  int parts;           // workgroups that share one configuration's rows
+  RowCost cost;        // written instead of the distance when on
+  float* out;
+};
+
+// Two floats' minimum that skips NaN, for values that are never negative: as
+// unsigned integers, where every NaN is above +inf.
+__device__ __forceinline__ unsigned min_bits(unsigned m, float v) { return min(m, __float_as_uint(v)); }
+
+// Same-radius runs: the square root and the radius are applied when the radius
+// changes.  `r` of the run that m2 belongs to.
+template <bool JAX>
+__device__ __forceinline__ float row_spheres(const float4* pos, int n, const float* o, float best) {
+  const float ox = o[0], oy = o[1], oz = o[2], orad = o[3];
+  if (n == 0) return best;
+  unsigned m2 = 0x7f800000u;
+  float r = pos[0].w;
+  for (int i = 0; i < n; ++i) {
+    const float4 c = pos[i];
+    if (c.w != r) {
+      best = fminf(best, sqrtf(__uint_as_float(m2)) - (r + orad));
+      m2 = 0x7f800000u;
+      r = c.w;
+    }
+    // The JAX path adds its bias to (obstacle - sphere).
+    const float dx = JAX ? (ox - c.x) + 1e-6f : c.x - ox;
+    const float dy = JAX ? (oy - c.y) + 1e-6f : c.y - oy;
+    const float dz = JAX ? (oz - c.z) + 1e-6f : c.z - oz;
+    m2 = min_bits(m2, dx * dx + dy * dy + dz * dz);
+  }
+  return fminf(best, sqrtf(__uint_as_float(m2)) - (r + orad));
+}
+
+__device__ __forceinline__ float row_capsule(const float4* pos, int n, const float* o, float best) {
+  const float ax = o[0], ay = o[1], az = o[2];
+  const float ux = o[3] - ax, uy = o[4] - ay, uz = o[5] - az, rad = o[6];
+  const float uu = ux * ux + uy * uy + uz * uz;
+  const float inv = uu > 1e-12f ? 1.f / uu : 0.f;  // a point: t = 0
+  if (n == 0) return best;
+  unsigned m2 = 0x7f800000u;
+  float r = pos[0].w;
+  for (int i = 0; i < n; ++i) {
+    const float4 c = pos[i];
+    if (c.w != r) {
+      best = fminf(best, sqrtf(__uint_as_float(m2)) - (r + rad));
+      m2 = 0x7f800000u;
+      r = c.w;
+    }
+    const float wx = c.x - ax, wy = c.y - ay, wz = c.z - az;
+    const float t = fminf(fmaxf((wx * ux + wy * uy + wz * uz) * inv, 0.f), 1.f);
+    const float dx = wx - t * ux, dy = wy - t * uy, dz = wz - t * uz;
+    m2 = min_bits(m2, dx * dx + dy * dy + dz * dz);
+  }
+  return fminf(best, sqrtf(__uint_as_float(m2)) - (r + rad));
+}
+
+// KIND of WorldPrims (0 spheres, 1 capsules, 2 boxes, 3 half-spaces): rows of
+// obstacles [0, count) of that kind, written at column `col` of the M.
+template <int KIND, bool JAX>
+__device__ __forceinline__ void kind_rows(const RowArgs& a, const float4* pos, const int* cnt, int part,
+                                          long long row0, int M, int col) {
+  constexpr int width = KIND == 0 ? 4 : (KIND == 1 ? 7 : (KIND == 2 ? 15 : 6));
+  const float* data = KIND == 0 ? a.w.data[0] : (KIND == 1 ? a.w.data[1] : (KIND == 2 ? a.w.data[2] : a.w.data[3]));
+  const int n_obs = KIND == 0 ? a.w.count[0] : (KIND == 1 ? a.w.count[1] : (KIND == 2 ? a.w.count[2] : a.w.count[3]));
+  if (n_obs == 0) return;
+  const int S = a.s_per_link;
+  // Lane strides of (link, obstacle), without a division in the loop.
+  const int step = kRowThreads * a.parts;
+  const int step_l = step / n_obs, step_m = step - step_l * n_obs;
+  const int f0 = part * kRowThreads + static_cast<int>(threadIdx.x);
+  int l = f0 / n_obs, m = f0 - l * n_obs;
+  while (l < a.n_links) {
+    const float* o = data + static_cast<long long>(width) * m;
+    const float4* p = pos + l * S;
+    const int n = cnt[l];
+    float best = JAX ? INFINITY : kNoSphere;
+    if (KIND == 0) {
+      best = row_spheres<JAX>(p, n, o, best);
+    } else if (KIND == 1) {
+      best = row_capsule(p, n, o, best);
+    } else {
+      float obs[width];
+#pragma unroll
+      for (int i = 0; i < width; ++i) obs[i] = o[i];
+      for (int i = 0; i < n; ++i) {
+        const float4 c = p[i];
+        best = fminf(best, KIND == 2 ? dist_sphere_box(c.x, c.y, c.z, c.w, obs)
+                                     : dist_sphere_halfspace(c.x, c.y, c.z, c.w, obs));
+      }
+    }
+    if (a.cost.on) best = row_cost(a.cost, best);
+    __builtin_nontemporal_store(best, a.out + (row0 + l) * M + col + m);
+    l += step_l;
+    m += step_m;
+    if (m >= n_obs) { m -= n_obs; ++l; }
+  }
+}
+
+template <bool JAX>
+__global__ __launch_bounds__(kRowThreads) void link_rows_kernel(RowArgs a) {
+  extern __shared__ float4 rsmem[];
+  const int L = a.n_links, S = a.s_per_link, LS = L * S;
+  float4* loc = rsmem;                             // sorted link-frame spheres, link l at l * S
+  float4* pos = loc + LS;                          // the same in the world
+  int* cnt = reinterpret_cast<int*>(pos + LS);     // spheres of each link
+  const int tid = threadIdx.x;
+  for (int t = tid; t < LS; t += kRowThreads) {
+    const float* s = a.table + 4LL * t;
+    pos[t] = make_float4(s[0], s[1], s[2], s[3]);  // staged here until sorted
+  }
+  for (int l = tid; l < L; l += kRowThreads) cnt[l] = 0;
+  __syncthreads();
+  // Which slots count.  CUDA conventions: those with r >= 0 (or NaN).  JAX:
+  // padding takes part, but a slot equal to the one before it changes no
+  // minimum, so of a run of padding one is kept.  A kept slot's place: larger
+  // radii first, slot order within a radius (a NaN compares as smallest).
+  for (int t = tid; t < LS; t += kRowThreads) {
+    const int l = t / S, s = t - l * S;
+    auto kept = [&](int i) {
+      const float4 c = pos[l * S + i];
+      if (!JAX) return !(c.w < 0.f);
+      if (i == 0) return true;
+      const float4 p = pos[l * S + i - 1];
+      return !(c.x == p.x && c.y == p.y && c.z == p.z && c.w == p.w);
+    };
+    if (!kept(s)) continue;
+    const float4 c = pos[t];
+    auto above = [](float p, float q) { return p > q || (p == p && q != q); };
+    int rank = 0;
+    for (int i = 0; i < S; ++i) {
+      const float r = pos[l * S + i].w;
+      if ((above(r, c.w) || (!above(c.w, r) && i < s)) && kept(i)) ++rank;
+    }
+    loc[l * S + rank] = c;
+    atomicAdd(&cnt[l], 1);
+  }
+  __syncthreads();
+  const int M = a.w.total();
+  const long long n_items = a.batch * a.parts;
+  for (long long item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const long long b = item / a.parts;
+    const int part = static_cast<int>(item - b * a.parts);
+    for (int t = tid; t < LS; t += kRowThreads) {
+      const int l = t / S;
+      if (t - l * S < cnt[l]) {
+        const float* T = a.poses + (b * L + l) * 7;
+        const float4 c = loc[t];
+        float x, y, z;
+        quat_rotate(T[0], T[1], T[2], T[3], c.x, c.y, c.z, x, y, z);
+        pos[t] = make_float4(x + T[4], y + T[5], z + T[6], c.w);
+      }
+    }
+    __syncthreads();
+    int col = 0;
+    kind_rows<0, JAX>(a, pos, cnt, part, b * L, M, col);
+    if (!JAX) {
+      col += a.w.count[0];
+      kind_rows<1, false>(a, pos, cnt, part, b * L, M, col);
+      col += a.w.count[1];
+      kind_rows<2, false>(a, pos, cnt, part, b * L, M, col);
+      col += a.w.count[2];
+      kind_rows<3, false>(a, pos, cnt, part, b * L, M, col);
+    }
+    __syncthreads();
+  }
+}
+
+// Same-slot self distances (jax_self_kernel's) with each configuration's
+// spheres placed once into LDS: `tile` configurations at a time, lanes over
+// (configuration, pair).  A link's slots past its last distinct one repeat it,
+// so a pair stops at the longer of its two links.  (One lane per pair placing
+// both links' 28 slots took 30 us for 4099 Fetch configurations.)
+struct SelfRowArgs {
+  const float* poses;
+  long long batch;
+  int n_links, s_per_link;
+  const float* table;
+  const int* pair_i;
+  const int* pair_j;
+  int n_pairs, tile;
+  RowCost cost;
+  float* out;
+};
+
+__global__ __launch_bounds__(kRowThreads) void self_rows_kernel(SelfRowArgs a) {
+  extern __shared__ float4 rsmem[];
+  const int L = a.n_links, S = a.s_per_link, LS = L * S, P = a.n_pairs;
+  float4* loc = rsmem;                                    // link-frame slots
+  float4* pos = loc + LS;                                 // tile x LS in the world
+  int* cnt = reinterpret_cast<int*>(pos + a.tile * LS);   // slots of each link up to its last distinct one
+  int* pairs = cnt + L;                                   // link i | link j << 16, -1 invalid
+  const int tid = threadIdx.x;
+  for (int t = tid; t < LS; t += kRowThreads) {
+    const float* s = a.table + 4LL * t;
+    loc[t] = make_float4(s[0], s[1], s[2], s[3]);
+  }
+  for (int l = tid; l < L; l += kRowThreads) cnt[l] = S > 0 ? 1 : 0;
+  for (int p = tid; p < P; p += kRowThreads) {
+    const int i = a.pair_i[p], j = a.pair_j[p];
+    pairs[p] = (i >= 0 && i < L && j >= 0 && j < L) ? (i | (j << 16)) : -1;
+  }
+  __syncthreads();
+  for (int t = tid; t < LS; t += kRowThreads) {
+    const int l = t / S, s = t - l * S;
+    if (s == 0) continue;
+    const float4 c = loc[t], q = loc[t - 1];
+    if (!(c.x == q.x && c.y == q.y && c.z == q.z && c.w == q.w)) atomicMax(&cnt[l], s + 1);
+  }
+  __syncthreads();
+  const long long n_tiles = (a.batch + a.tile - 1) / a.tile;
+  for (long long tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    const long long b0 = tile * a.tile;
+    const int nb = static_cast<int>(min(static_cast<long long>(a.tile), a.batch - b0));
+    for (int t = tid; t < nb * LS; t += kRowThreads) {
+      const int c = t / LS, k = t - c * LS, l = k / S;
+      if (k - l * S >= cnt[l]) continue;
+      const float* T = a.poses + ((b0 + c) * L + l) * 7;
+      const float4 s = loc[k];
+      float x, y, z;
+      quat_rotate(T[0], T[1], T[2], T[3], s.x, s.y, s.z, x, y, z);
+      pos[t] = make_float4(x + T[4], y + T[5], z + T[6], s.w);
+    }
+    __syncthreads();
+    for (int t = tid; t < nb * P; t += kRowThreads) {
+      const int c = t / P, en = pairs[t - c * P];
+      float best = INFINITY;
+      if (en >= 0) {
+        const int li = en & 0xffff, lj = en >> 16;
+        const int ni = cnt[li], nj = cnt[lj];
+        const float4* pi = pos + c * LS + li * S;
+        const float4* pj = pos + c * LS + lj * S;
+        for (int s = 0; s < max(ni, nj); ++s) {
+          const float4 u = pi[min(s, ni - 1)], v = pj[min(s, nj - 1)];
+          best = fminf(best, jax_sphere_dist(u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w));
+        }
+      }
+      if (a.cost.on) best = row_cost(a.cost, best);
+      __builtin_nontemporal_store(best, a.out + b0 * P + t);
+    }
+    __syncthreads();
+  }
+}
+
+// False when the tables do not fit the LDS (jax_self_kernel then takes them).
+static bool launch_self_rows(hipStream_t s, SelfRowArgs a) {
+  const long long LS = static_cast<long long>(a.n_links) * a.s_per_link;
+  if (LS > kRowSlots || a.n_links >= 32768 || a.n_pairs > 8192) return false;
+  // Enough configurations for two rounds of lanes, while their spheres take
+  // at most 32 KiB.
+  a.tile = std::max(1, std::min(2 * kRowThreads / a.n_pairs, LS > 0 ? static_cast<int>(2048 / LS) : 8));
+  const size_t lds = sizeof(float4) * (1 + a.tile) * LS + sizeof(int) * (a.n_links + a.n_pairs);
+  const unsigned grid = static_cast<unsigned>(std::min((a.batch + a.tile - 1) / a.tile, 256LL * 4));
+  hipLaunchKernelGGL(self_rows_kernel, dim3(grid), dim3(kRowThreads), lds, s, a);
+  return true;
+}
+
+// Launch of link_rows_kernel, or false when its tables do not fit the LDS.
+// Four workgroups a CU loop over the configurations, which spreads the table's
+// sorting; fewer configurations than that share each among workgroups.
+template <bool JAX>
+static bool launch_link_rows(hipStream_t s, RowArgs a) {
+  const int LS = a.n_links * a.s_per_link;
+  const long long per = a.n_links * static_cast<long long>(a.w.total());
+  if (static_cast<long long>(a.n_links) * a.s_per_link > kRowSlots || per > 0x3fffffffLL) return false;
+  constexpr long long kGroups = 256LL * 4;
+  long long parts = 1;
+  if (a.batch < kGroups) parts = std::min((kGroups + a.batch - 1) / a.batch, (per + kRowThreads - 1) / kRowThreads);
+  a.parts = static_cast<int>(parts);
+  const size_t lds = sizeof(float4) * 2 * LS + sizeof(int) * a.n_links;
+  const unsigned grid = static_cast<unsigned>(std::min(kGroups, a.batch * parts));
+  hipLaunchKernelGGL((link_rows_kernel<JAX>), dim3(grid), dim3(kRowThreads), lds, s, a);
+  return true;
+}
+
 // Centre of sphere slot s of link l for configuration b: T_l applied to the
 // link-frame centre of the padded (L, S, 4) table.
 __device__ __forceinline__ void placed(const float* __restrict__ poses, const float* __restrict__ table,
@@ -75,22 +403,12 @@ __device__ __forceinline__ void placed(const float* __restrict__ poses, const fl
   r = c[3];
 }
 
-// The JAX distance of two spheres (src/pyroffi/collision/_geometry_pairs.py:59-68
-// with the 1e-6 added to each component inside the norm, _utils.py:45):
-// |(p2 - p1) + 1e-6| - (r1 + r2).  Padding radii (-1e9) take part as they do
-// in JAX and make the distance about +1e9.
-__device__ __forceinline__ float jax_sphere_dist(float x1, float y1, float z1, float r1, float x2, float y2,
-                                                 float z2, float r2) {
-  const float dx = (x2 - x1) + 1e-6f, dy = (y2 - y1) + 1e-6f, dz = (z2 - z1) + 1e-6f;
-  return sqrtf(dx * dx + dy * dy + dz * dz) - (r1 + r2);
-}
-
 // out[b, l, m] = min over slots s of jax_sphere_dist(sphere (l, s), world m)
 // (RobotCollisionSpherized.compute_world_collision_distance,
 // src/pyroffi/collision/_robot_collision.py:830-895).
 __global__ __launch_bounds__(256) void jax_world_kernel(const float* __restrict__ poses, long long B, int L,
                                                         const float* __restrict__ table, int S,
-                                                        const float* __restrict__ world, int M,
+                                                        const float* __restrict__ world, int M, RowCost cost,
                                                         float* __restrict__ out) {
   const long long total = B * L * static_cast<long long>(M);
   const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
@@ -106,6 +424,7 @@ __global__ __launch_bounds__(256) void jax_world_kernel(const float* __restrict_
       placed(poses, table, b, L, S, l, s, x, y, z, r);
       best = fminf(best, jax_sphere_dist(x, y, z, r, o[0], o[1], o[2], o[3]));
     }
+    if (cost.on) best = row_cost(cost, best);
     __builtin_nontemporal_store(best, out + f);
   }
 }
@@ -117,7 +436,7 @@ __global__ __launch_bounds__(256) void jax_world_kernel(const float* __restrict_
 __global__ __launch_bounds__(256) void jax_self_kernel(const float* __restrict__ poses, long long B, int L,
                                                        const float* __restrict__ table, int S,
                                                        const int* __restrict__ pair_i,
-                                                       const int* __restrict__ pair_j, int P,
+                                                       const int* __restrict__ pair_j, int P, RowCost cost,
                                                        float* __restrict__ out) {
   const long long total = B * static_cast<long long>(P);
   const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
@@ -134,6 +453,7 @@ __global__ __launch_bounds__(256) void jax_self_kernel(const float* __restrict__
         best = fminf(best, jax_sphere_dist(xi, yi, zi, ri, xj, yj, zj, rj));
       }
     }
+    if (cost.on) best = row_cost(cost, best);
     __builtin_nontemporal_store(best, out + f);
   }
 }
@@ -309,12 +629,12 @@ extern "C" int pk_collision_world_sphere_f32(void* stream, const float* sphere_c
   return pk::check_launch("world_sphere_full_kernel");
 }
 
-extern "C" int pk_sphere_distances_jax_f32(void* stream, const float* link_poses, int64_t batch,
-                                           int32_t n_links, const float* spheres_padded,
-                                           int32_t s_per_link, const float* world_spheres,
-                                           int32_t n_world_spheres, const int32_t* pair_i,
-                                           const int32_t* pair_j, int32_t n_pairs, float* out_world,
-                                           float* out_self) {
+namespace {
+
+int distances_jax(void* stream, const float* link_poses, int64_t batch, int32_t n_links, const float* spheres_padded,
+                  int32_t s_per_link, const float* world_spheres, int32_t n_world_spheres, const int32_t* pair_i,
+                  const int32_t* pair_j, int32_t n_pairs, const pk::RowCost& cost, float* out_world,
+                  float* out_self) {
   PK_REQUIRE(batch >= 0 && n_links >= 0 && s_per_link >= 0 && n_world_spheres >= 0 && n_pairs >= 0,
              "negative size");
   if (batch == 0 || n_links == 0) return PK_OK;
@@ -322,22 +642,70 @@ extern "C" int pk_sphere_distances_jax_f32(void* stream, const float* link_poses
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (out_world && n_world_spheres > 0) {
     PK_REQUIRE(world_spheres != nullptr, "null world");
-    const long long total = batch * n_links * static_cast<long long>(n_world_spheres);
-    hipLaunchKernelGGL(pk::jax_world_kernel, dim3(pk::flat_blocks(total)), dim3(256), 0, s, link_poses,
-                       static_cast<long long>(batch), n_links, spheres_padded, s_per_link, world_spheres,
-                       n_world_spheres, out_world);
-    const int st = pk::check_launch("jax_world_kernel");
+    pk::RowArgs a{};
+    a.poses = link_poses;
+    a.batch = batch;
+    a.n_links = n_links;
+    a.s_per_link = s_per_link;
+    a.table = spheres_padded;
+    a.w.data[0] = world_spheres;
+    a.w.count[0] = n_world_spheres;
+    a.cost = cost;
+    a.out = out_world;
+    if (!pk::launch_link_rows<true>(s, a)) {
+      const long long total = batch * n_links * static_cast<long long>(n_world_spheres);
+      hipLaunchKernelGGL(pk::jax_world_kernel, dim3(pk::flat_blocks(total)), dim3(256), 0, s, link_poses,
+                         static_cast<long long>(batch), n_links, spheres_padded, s_per_link, world_spheres,
+                         n_world_spheres, cost, out_world);
+    }
+    const int st = pk::check_launch("link_rows_kernel");
     if (st != PK_OK) return st;
   }
   if (out_self && n_pairs > 0) {
     PK_REQUIRE(pair_i && pair_j, "null pair list");
-    const long long total = batch * static_cast<long long>(n_pairs);
-    hipLaunchKernelGGL(pk::jax_self_kernel, dim3(pk::flat_blocks(total)), dim3(256), 0, s, link_poses,
-                       static_cast<long long>(batch), n_links, spheres_padded, s_per_link, pair_i, pair_j,
-                       n_pairs, out_self);
-    return pk::check_launch("jax_self_kernel");
+    pk::SelfRowArgs a{};
+    a.poses = link_poses;
+    a.batch = batch;
+    a.n_links = n_links;
+    a.s_per_link = s_per_link;
+    a.table = spheres_padded;
+    a.pair_i = pair_i;
+    a.pair_j = pair_j;
+    a.n_pairs = n_pairs;
+    a.cost = cost;
+    a.out = out_self;
+    if (!pk::launch_self_rows(s, a)) {
+      const long long total = batch * static_cast<long long>(n_pairs);
+      hipLaunchKernelGGL(pk::jax_self_kernel, dim3(pk::flat_blocks(total)), dim3(256), 0, s, link_poses,
+                         static_cast<long long>(batch), n_links, spheres_padded, s_per_link, pair_i, pair_j,
+                         n_pairs, cost, out_self);
+    }
+    return pk::check_launch("self_rows_kernel");
   }
   return PK_OK;
+}
+
+}  // namespace
+
+extern "C" int pk_sphere_distances_jax_f32(void* stream, const float* link_poses, int64_t batch,
+                                           int32_t n_links, const float* spheres_padded,
+                                           int32_t s_per_link, const float* world_spheres,
+                                           int32_t n_world_spheres, const int32_t* pair_i,
+                                           const int32_t* pair_j, int32_t n_pairs, float* out_world,
+                                           float* out_self) {
+  return distances_jax(stream, link_poses, batch, n_links, spheres_padded, s_per_link, world_spheres,
+                       n_world_spheres, pair_i, pair_j, n_pairs, pk::RowCost{}, out_world, out_self);
+}
+
+extern "C" int pk_sphere_costs_jax_f32(void* stream, const float* link_poses, int64_t batch, int32_t n_links,
+                                       const float* spheres_padded, int32_t s_per_link,
+                                       const float* world_spheres, int32_t n_world_spheres,
+                                       const int32_t* pair_i, const int32_t* pair_j, int32_t n_pairs,
+                                       float margin, float half, float quad, float weight, float* out_world,
+                                       float* out_self) {
+  return distances_jax(stream, link_poses, batch, n_links, spheres_padded, s_per_link, world_spheres,
+                       n_world_spheres, pair_i, pair_j, n_pairs, pk::RowCost{1, margin, half, quad, weight},
+                       out_world, out_self);
 }
 
 extern "C" int pk_collision_world_capsule_f32(void* stream, const float* caps, int64_t batch, int32_t n_links,
@@ -398,10 +766,20 @@ extern "C" int pk_sphere_world_links_f32(void* stream, const float* link_poses, 
     const int ws = pk::world_prims(w, world_spheres, n_world_spheres, world_capsules, n_world_capsules,
                                    world_boxes, n_world_boxes, world_halfspaces, n_world_halfspaces);
     if (ws != PK_OK) return ws;
-    const long long total = batch * n_links * M;
-    hipLaunchKernelGGL(pk::world_links_mixed_kernel, dim3(pk::flat_blocks(total)), dim3(256), 0, st, link_poses,
-                       static_cast<long long>(batch), n_links, spheres_padded, s_per_link, w, out_world);
-    const int e = pk::check_launch("world_links_mixed_kernel");
+    pk::RowArgs a{};
+    a.poses = link_poses;
+    a.batch = batch;
+    a.n_links = n_links;
+    a.s_per_link = s_per_link;
+    a.table = spheres_padded;
+    a.w = w;
+    a.out = out_world;
+    if (!pk::launch_link_rows<false>(st, a)) {
+      const long long total = batch * n_links * M;
+      hipLaunchKernelGGL(pk::world_links_mixed_kernel, dim3(pk::flat_blocks(total)), dim3(256), 0, st, link_poses,
+                         static_cast<long long>(batch), n_links, spheres_padded, s_per_link, w, out_world);
+    }
+    const int e = pk::check_launch("link_rows_kernel");
     if (e != PK_OK) return e;
   }
   if (out_world_min) {

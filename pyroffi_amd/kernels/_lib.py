@@ -121,6 +121,7 @@ _SIGNATURES = {
     ),
     "pk_collision_self_sphere_f32": (_i32, [_p, _p, _p, _i64, _i32, _i32, _p, _p, _i32, _p]),
     "pk_sphere_distances_jax_f32": (_i32, [_p, _p, _i64, _i32, _p, _i32, _p, _i32, _p, _p, _i32, _p, _p]),
+    "pk_sphere_costs_jax_f32": (_i32, [_p, _p, _i64, _i32, _p, _i32, _p, _i32, _p, _p, _i32, _f32, _f32, _f32, _f32, _p, _p]),
     "pk_collision_world_capsule_f32": (_i32, [_p, _p, _i64, _i32, _p, _i32, _p, _i32, _p, _i32, _p, _i32, _p]),
     "pk_collision_self_capsule_f32": (_i32, [_p, _p, _i64, _i32, _p, _p, _i32, _p]),
     "pk_capsules_place_f32": (_i32, [_p, _p, _i64, _i32, _p, _p, _p]),

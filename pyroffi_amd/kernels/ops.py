@@ -220,9 +220,9 @@ def collision_self_capsule(caps, pair_i, pair_j) -> torch.Tensor:
     return out
 
 
-def sphere_world_links(link_poses, spheres_padded, world: dict, *, per_link: bool = True):
+def sphere_world_links(link_poses, spheres_padded, world: dict, *, per_link: bool = True, world_min: bool = True):
     """World distances of a spherized robot over the four obstacle kinds with the CUDA
-    kernels' semantics: ``(out (B, L, M), out_min (B,))`` from link poses ``(B, L, 7)``,
+    kernels' semantics: ``(out (B, L, M), out_min (B,) | None)`` from link poses ``(B, L, 7)``,
     the padded ``(L, S, 4)`` link-frame sphere table and ``world`` = packed arrays by kind
     (``spheres (Ms,4)``, ``capsules (Mc,7)``, ``boxes (Mb,15)``, ``halfspaces (Mh,6)``)."""
     lp = _dev(link_poses, torch.float32)
@@ -233,7 +233,7 @@ def sphere_world_links(link_poses, spheres_padded, world: dict, *, per_link: boo
          for k, n in (("spheres", 4), ("capsules", 7), ("boxes", 15), ("halfspaces", 6))}
     M = sum(v.shape[0] for v in w.values())
     out = torch.empty((B, L, M), dtype=torch.float32, device=dev)
-    out_min = torch.empty((B,), dtype=torch.float32, device=dev)
+    out_min = torch.empty((B,), dtype=torch.float32, device=dev) if world_min else None
     st = lib().pk_sphere_world_links_f32(
         _stream(), _ptr(lp), B, L, _ptr(sp), sp.shape[1],
         _ptr(w["spheres"]), w["spheres"].shape[0], _ptr(w["capsules"]), w["capsules"].shape[0],
@@ -245,9 +245,11 @@ def sphere_world_links(link_poses, spheres_padded, world: dict, *, per_link: boo
 
 
 def sphere_distances_jax(link_poses, spheres_padded, world_spheres, pair_i, pair_j, *, world: bool = True,
-                         self_pairs: bool = True):
+                         self_pairs: bool = True, cost: tuple[float, float] | None = None):
     """The JAX path's conventions: ``(out_world (B, L, M) | None, out_self (B, P) | None)``
-    from link poses ``(B, L, 7)`` and the padded ``(L, S, 4)`` link-frame sphere table."""
+    from link poses ``(B, L, 7)`` and the padded ``(L, S, 4)`` link-frame sphere table.
+    With ``cost = (margin, weight)`` each distance d is written as
+    ``colldist_from_sdf(d, margin) * weight``."""
     lp = _dev(link_poses, torch.float32)
     dev = lp.device
     B, L, _ = lp.shape
@@ -257,11 +259,13 @@ def sphere_distances_jax(link_poses, spheres_padded, world_spheres, pair_i, pair
     pj = _dev(pair_j, torch.int32, dev)
     ow = torch.empty((B, L, ws.shape[0]), dtype=torch.float32, device=dev) if world else None
     osf = torch.empty((B, pi.shape[0]), dtype=torch.float32, device=dev) if self_pairs else None
-    st = lib().pk_sphere_distances_jax_f32(
-        _stream(), _ptr(lp), B, L, _ptr(sp), sp.shape[1], _ptr(ws), ws.shape[0], _ptr(pi), _ptr(pj),
-        pi.shape[0], _ptr(ow), _ptr(osf),
-    )
-    check(st, "pk_sphere_distances_jax_f32")
+    args = (_stream(), _ptr(lp), B, L, _ptr(sp), sp.shape[1], _ptr(ws), ws.shape[0], _ptr(pi), _ptr(pj), pi.shape[0])
+    if cost is None:
+        check(lib().pk_sphere_distances_jax_f32(*args, _ptr(ow), _ptr(osf)), "pk_sphere_distances_jax_f32")
+    else:
+        margin, weight = cost
+        check(lib().pk_sphere_costs_jax_f32(*args, margin, 0.5 * margin, -0.5 / (margin + 1e-6), weight, _ptr(ow),
+                                            _ptr(osf)), "pk_sphere_costs_jax_f32")
     return ow, osf
 
 
