@@ -664,11 +664,10 @@ struct PenLds {
   int n_clusters, pad[3];
 };
 
-// The tables behind it, one entry per cluster (at: one per point and cluster).
+// The tables behind it, one entry per cluster.
 struct PenClusters {
   float4* bound;  // bounding sphere, node frame
-  float4* hull;   // ball around `at` of all the points
-  float4* at;     // the bounding sphere in the world at each point
+  float4* hull;   // ball around the bounding sphere's places at the points
   int* node;
   int* first;     // first sphere; the cluster ends at the next one's or its node's
   int max;
@@ -676,7 +675,7 @@ struct PenClusters {
 
 template <int MAXA>
 __host__ __device__ inline size_t pen_lds_bytes(int K) {
-  return sizeof(PenLds<MAXA>) + (sizeof(float4) * (2 + kLineSteps) + 2 * sizeof(int)) * max_clusters(K, MAXA);
+  return sizeof(PenLds<MAXA>) + (sizeof(float4) * 2 + sizeof(int) * 2) * max_clusters(K, MAXA);
 }
 
 template <int MAXA>
@@ -685,8 +684,7 @@ __device__ __forceinline__ PenClusters pen_clusters(PenLds<MAXA>* pl, int K) {
   o.max = max_clusters(K, MAXA);
   o.bound = reinterpret_cast<float4*>(pl + 1);
   o.hull = o.bound + o.max;
-  o.at = o.hull + o.max;
-  o.node = reinterpret_cast<int*>(o.at + kLineSteps * o.max);
+  o.node = reinterpret_cast<int*>(o.hull + o.max);
   o.first = o.node + o.max;
   return o;
 }
@@ -788,6 +786,11 @@ __device__ __forceinline__ float wave_penalty(const IkView<MAXA, NEE>& v, PenLds
     pc.hull[c] = h;
   }
   wave_sync();
+  // The first 64 kHeld obstacles stay in registers for all clusters.
+  constexpr int kHeld = 4;
+  float4 held[kHeld];
+#pragma unroll
+  for (int h = 0; h < kHeld; ++h) held[h] = v.ws[max(min(h * kWave + lane, v.M - 1), 0)];
   float total = sh.static_pen;
   for (int c = 0; c < n_cl; ++c) {
     const int n = __builtin_amdgcn_readfirstlane(pc.node[c]);
@@ -808,10 +811,9 @@ __device__ __forceinline__ float wave_penalty(const IkView<MAXA, NEE>& v, PenLds
       placed = true;
     };
     if (n_other > 0) place();
-    for (int m0 = 0; m0 < v.M; m0 += kWave) {
-      const float4 o = v.ws[min(m0 + lane, v.M - 1)];
+    auto pass = [&](int m0, const float4& o) {
       const unsigned long long mask = __ballot(m0 + lane < v.M && in_reach(hull, o));
-      if (mask == 0) continue;
+      if (mask == 0) return;
       if (!placed) place();
       auto one = [&](int j, float& p) {
         const float ax = cx - __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o.x), j));
@@ -823,15 +825,28 @@ __device__ __forceinline__ float wave_penalty(const IkView<MAXA, NEE>& v, PenLds
       };
       for (unsigned long long m = mask & 0x5555555555555555ull; m != 0; m &= m - 1) one(__builtin_ctzll(m), p0);
       for (unsigned long long m = mask & 0xaaaaaaaaaaaaaaaaull; m != 0; m &= m - 1) one(__builtin_ctzll(m), p1);
-    }
+    };
+#pragma unroll
+    for (int h = 0; h < kHeld; ++h)
+      if (h * kWave < v.M) pass(h * kWave, held[h]);
+    for (int m0 = kHeld * kWave; m0 < v.M; m0 += kWave) pass(m0, v.ws[min(m0 + lane, v.M - 1)]);
     if (!placed) continue;  // every term is zero
     pl.term[lane] = p0 + p1;
     if (n_other > 0) pl.other[lane] = other_penalty(cx, cy, cz, r, v.ow);
     wave_sync();
     if (lane < NP) {
-      for (int i = lane; i < cnt; i += NP) {
-        total += pl.term[i];
-        if (n_other > 0) total += pl.other[i];
+      if (n_other > 0) {
+        for (int i = lane; i < cnt; i += NP) {
+          total += pl.term[i];
+          total += pl.other[i];
+        }
+      } else {
+        // All reads first; a slot past the cluster adds zero, which changes nothing.
+        float t[kCluster];
+#pragma unroll
+        for (int i = 0; i < kCluster; ++i) t[i] = pl.term[lane + NP * i];
+#pragma unroll
+        for (int i = 0; i < kCluster; ++i) total += (lane + NP * i < cnt) ? t[i] : 0.f;
       }
     }
     wave_sync();
@@ -1212,7 +1227,7 @@ __host__ __device__ inline size_t pen_lds_offset(const IkArgs& a) {
 
 // G lanes per seed (see lm_iterate); the group's first lane writes the result.
 template <int MAXA, int NEE, int G, bool COOP>
-__global__ __launch_bounds__(64) void ls_ik_kernel(IkArgs a) {
+__global__ __launch_bounds__(64, COOP && MAXA == 8 ? 2 : 1) void ls_ik_kernel(IkArgs a) {
   extern __shared__ float4 smem4[];
   const IkView<MAXA, NEE> v = ik_prologue<MAXA, NEE>(a, reinterpret_cast<char*>(smem4));
   const int lane = threadIdx.x;
