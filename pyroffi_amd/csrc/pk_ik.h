@@ -644,8 +644,8 @@ __device__ __forceinline__ void jac_column(const Pose& Pn, const float* ax, int 
 //      lane that holds them, in index order (even and odd ones summed apart,
 //      as world_penalty_all does);
 //   3. lane i adds point i's terms in sphere order.
-// 61 problems x 32 seeds of Fetch, 40 iterations, 256 obstacles: 41.6 -> 2.55
-// ms a call (2.78 with one bounding sphere per node).
+// 61 problems x 32 seeds of Fetch, 40 iterations, 256 obstacles: 41.6 -> 1.47
+// ms a call.
 // The bounds carry slack for rounding, so a dropped pair's term is zero; the
 // tests are phrased so that a NaN keeps its pair.
 constexpr int kLineSteps = 5;

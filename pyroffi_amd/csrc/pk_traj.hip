@@ -174,6 +174,25 @@ struct TrajLds {
   float4* gc;   // per group: world sphere centres + radius (K), link bounding spheres (L)
 };
 
+// out[0 .. n] = the running maximum of in[0 .. n - 1] and, last, of `last`, each
+// clamped to [0, last]; out[0] = 0.  One wave.
+__device__ __forceinline__ void stage_offsets(const int* in, int n, int last, int* out) {
+  const int lane = threadIdx.x % kWave;
+  int carry = 0;
+  for (int base = 0; base <= n; base += kWave) {
+    const int i = base + lane;
+    int v = (i < n) ? min(max(in[i], 0), last) : (i == n ? last : 0);
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int u = __shfl_up(v, off, kWave);
+      if (lane >= off) v = max(v, u);
+    }
+    v = max(v, carry);
+    if (i <= n) out[i] = (i == 0) ? 0 : v;
+    carry = __shfl(v, kWave - 1, kWave);
+  }
+}
+
 // Cooperative copy of the model into LDS, with every index clamped into range.
 __device__ __forceinline__ TrajLds stage_traj_model(const TrajModelDev& md, int max_len, char* base) {
   const int N = md.n_nodes, L = md.n_links, K = md.n_spheres, P = md.n_pairs, Q = md.n_items;
@@ -210,19 +229,13 @@ __device__ __forceinline__ TrajLds stage_traj_model(const TrajModelDev& md, int 
     const int n = md.link_node[l];
     link_node[l] = (n >= 0 && n < N) ? n : -1;
   }
-  if (tid == 0) {
-    int prev = 0;
-    for (int l = 0; l <= L; ++l) {
-      const int v = (l == L) ? K : md.link_sph_start[l];
-      prev = max(prev, min(max(v, 0), K));
-      link_sph[l] = (l == 0) ? 0 : prev;
-    }
-    prev = 0;
-    for (int p = 0; p <= P; ++p) {
-      const int v = (p == P) ? Q : md.pair_start[p];
-      prev = max(prev, min(max(v, 0), Q));
-      pair_start[p] = (p == 0) ? 0 : prev;
-    }
+  // CSR offsets clamped into monotone [0, K] and [0, Q] sequences, one wave
+  // each (on one thread the chain of table loads took 20 us).
+  if (tid < 2 * kWave) {
+    if (tid < kWave)
+      stage_offsets(md.link_sph_start, L, K, link_sph);
+    else
+      stage_offsets(md.pair_start, P, Q, pair_start);
   }
   for (int k = tid; k < K; k += blockDim.x) {
     const float* s = md.spheres + 4 * k;
@@ -434,6 +447,36 @@ __device__ __forceinline__ void waypoint_centres(const TrajModelDev& md, const T
   }
 }
 
+// Obstacle indices of one robot sphere: items[0 .. count), or 0 .. count - 1
+// (every world sphere) when items is null.
+struct GridCell {
+  const int* items;
+  int count;
+};
+constexpr int kItems = 8;
+
+__device__ __forceinline__ GridCell grid_cell_of(const GridArgs& grid, int n_world, const float4& c, bool valid) {
+  GridCell o;
+  o.items = nullptr;
+  o.count = 0;
+  if (valid) {
+    const int level = grid_level(grid, c.w);
+    if (level >= 0)
+      grid_cell_list(grid, level, c.x, c.y, c.z, o.items, o.count);
+    else
+      o.count = n_world;  // no level serves this radius
+  }
+  return o;
+}
+
+__device__ __forceinline__ void grid_items(const GridCell& cell, int i0, int (&m)[kItems]) {
+#pragma unroll
+  for (int u = 0; u < kItems; ++u) {
+    m[u] = i0 + u;
+    if (cell.items != nullptr && i0 + u < cell.count) m[u] = cell.items[i0 + u];
+  }
+}
+
 // Collision cost of one waypoint, evaluated by the kGroup lanes of a group
 // (lane g = threadIdx.x % kGroup) from the centres in gc, and with GRAD the
 // group's dcost/dq_node (per node, before the mimic map).  Every lane of the
@@ -450,28 +493,53 @@ __device__ __forceinline__ float group_waypoint_coll(const TrajModelDev& md, con
 #pragma unroll
   for (int a = 0; a < MAXN; ++a) gn[a] = 0.f;
 
-  // World: spheres s = g, g + kGroup, ... of the waypoint.
+  // World: spheres s = g, g + kGroup, ... of the waypoint.  A sphere's lookup
+  // is a chain of global loads (the cell's entry, then its obstacle indices),
+  // which one wave cannot hide: the entry is read two spheres ahead and the
+  // first kItems indices one sphere ahead, and further ones kItems at a time.
+  // (Read one by one, the chain was most of a pass: Panda, 1024 obstacles, one
+  // path of 128 waypoints, cost and gradient 371 us.)
+  GridCell next, after;
+  int ahead[kItems];
+  next = grid_cell_of(md.grid, md.n_world, gc[min(g, Ks - 1)], g < Ks);
+  grid_items(next, 0, ahead);
+  after = grid_cell_of(md.grid, md.n_world, gc[max(min(g + kGroup, Ks - 1), 0)], g + kGroup < Ks);
   for (int s = g; s < Ks; s += kGroup) {
     const float4 c = gc[s];
-    const int level = grid_level(md.grid, c.w);
-    const int* items = nullptr;
-    int count = 0;
-    if (level >= 0) grid_cell_list(md.grid, level, c.x, c.y, c.z, items, count);
-    const bool brute = level < 0;  // no level serves this radius: every world sphere
-    const int total = brute ? md.n_world : count;
+    const GridCell cell = next;
+    int m8[kItems];
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) m8[u] = ahead[u];
+    next = after;
+    grid_items(next, 0, ahead);
+    after = grid_cell_of(md.grid, md.n_world, gc[min(s + 2 * kGroup, Ks - 1)], s + 2 * kGroup < Ks);
+    const int total = cell.count;
     if (total == 0) continue;
     const int l = L.sph_link[s];
     const int k0 = L.link_sph[l], k1 = L.link_sph[l + 1];
     const int node = L.link_node[l];
     const int mask = node >= 0 ? L.anc[node] : 0;
-    for (int i = 0; i < total; ++i) {
-      const int m = brute ? i : items[i];
-      if (m < 0 || m >= md.n_world) continue;
+    for (int i0 = 0; i0 < total; i0 += kItems) {
+    if (i0 > 0) grid_items(cell, i0, m8);
+    unsigned near = 0;  // obstacles of this batch within the margin
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+      const int m = m8[u];
+      if (i0 + u >= total || m < 0 || m >= md.n_world) continue;
+      const float4 o = L.world[m];
+      const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
+      if (sqrtf(dx * dx + dy * dy + dz * dz) - c.w - o.w < margin) near |= 1u << u;
+    }
+    for (; near != 0; near &= near - 1) {
+      const int u0 = __builtin_ctz(near);
+      int m = m8[0];
+#pragma unroll
+      for (int u = 1; u < kItems; ++u)
+        if (u == u0) m = m8[u];
       const float4 o = L.world[m];
       const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
       const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
       const float d = dist - c.w - o.w;
-      if (!(d < margin)) continue;
       // The (link, world sphere) term is owned by the link's lowest-index
       // sphere within the margin; the owner takes the minimum over the link.
       bool owner = true;
@@ -496,6 +564,7 @@ __device__ __forceinline__ float group_waypoint_coll(const TrajModelDev& md, con
         const float k = -df / bdist;
         pull_point<MAXN, GRAD>(K, mask, bcx, bcy, bcz, k * bx, k * by, k * bz, gn);
       }
+    }
     }
   }
 
