@@ -1,0 +1,45 @@
+"""The trajectory cost's shared world search (paths of 24 waypoints and more) against the
+same waypoints evaluated as short paths, which look every sphere up in the grid: path lengths
+around the threshold, a wave's eight waypoints and a workgroup's rounds, world sizes around
+a pass of 64 obstacles, and obstacles crowded round the robot so that the lists overflow."""
+
+import numpy as np
+import pytest
+import torch
+from conftest import load_robot, random_cfgs
+
+from pyroffi_amd.collision import RobotCollisionSpherized
+from pyroffi_amd.optimization_engines._lbfgs_trajopt_optimization import TrajModel, flatten_trajs, traj_cost
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("name,T,M,extent,mode", [
+    ("panda", 24, 1, 1.0, 1), ("panda", 25, 63, 1.0, 0), ("ur5", 33, 64, 1.0, 1), ("fetch", 65, 65, 1.0, 1),
+    ("panda", 130, 300, 1.0, 0), ("panda", 40, 700, 0.4, 1), ("baxter", 31, 200, 0.6, 1), ("panda", 47, 0, 1.0, 1)])
+def test_long_path_equals_its_pieces(name, T, M, extent, mode):
+    """Collision terms only.  Both sides add the same FP32 terms in another order: 1e-5 of the
+    cost, 1e-4 of the gradient (whose terms cancel)."""
+    robot, path = load_robot(name)
+    coll = RobotCollisionSpherized.from_urdf(path)
+    rng = np.random.default_rng(T + M)
+    world = np.concatenate([rng.uniform(-extent, extent, (M, 3)), rng.uniform(0.02, 0.1, (M, 1))], 1)
+    model = TrajModel(robot, coll, world.astype(np.float32), 0.05, mode)
+    paths = []
+    for s in range(3):
+        a, b = random_cfgs(robot, 2, seed=s)
+        t = np.linspace(0, 1, T)[:, None]
+        paths.append(((1 - t) * a + t * b).astype(np.float32))
+    w = (0.0, 0.0, 0.0, 0.0, 0.0, 2.0)
+    x, start, n = flatten_trajs(paths, model.device)
+    comps, grad = traj_cost(model, x, start, n, w)
+    alone, none = traj_cost(model, x, start, n, w, grad=False)
+    assert none is None
+    torch.testing.assert_close(alone[:, 2], comps[:, 2], rtol=1e-5, atol=1e-6)
+    pieces = [p[i:i + 20] for p in paths for i in range(0, T, 20)]
+    xs, ss, ns = flatten_trajs(pieces, model.device)
+    pc, pg = traj_cost(model, xs, ss, ns, w)
+    per = -(-T // 20)
+    torch.testing.assert_close(comps[:, 2], pc[:, 2].reshape(3, per).sum(1), rtol=1e-5, atol=1e-6)
+    assert torch.equal(x, xs)
+    assert (grad - pg).norm() <= 1e-4 * pg.norm() + 1e-6
