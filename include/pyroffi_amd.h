@@ -125,6 +125,20 @@ int pk_fk_vjp_f32(void* stream, const float* cfg, int64_t batch, int32_t n_act,
                   int32_t n_links, const float* cot_links, float* out_dq);
 
 /*
+ * The same with a bound on the moving joints (actuated, mimic or with an
+ * offset; at most n_joints), which sizes the kernel's tables: with it more
+ * configurations are in flight.  A table with more moving joints gives NaN.
+ */
+int pk_fk_vjp_moving_f32(void* stream, const float* cfg, int64_t batch, int32_t n_act,
+                         const float* twists, const float* parent_tf,
+                         const int32_t* parent_idx, const int32_t* act_idx,
+                         const float* mimic_mul, const float* mimic_off,
+                         const int32_t* mimic_act_idx, const int32_t* topo_inv,
+                         int32_t n_joints, const int32_t* link_parent_joint,
+                         int32_t n_links, int32_t max_moving, const float* cot_links,
+                         float* out_dq);
+
+/*
  * World collision per robot sphere: out[b, k, m] = signed distance of sphere k
  * (centre c[:, b, k], radius r[b, k]) to obstacle m of the packed world, 1e9
  * for a padding slot (r < 0).  Obstacles are indexed spheres first, then

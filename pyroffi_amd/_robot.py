@@ -42,6 +42,10 @@ class _DeviceTables:
         self.link_parent_joint = i(links.parent_joint_indices)
         self.lower = f(joints.lower_limits)
         self.upper = f(joints.upper_limits)
+        # Joints whose transform is not constant (the kernels' rule).
+        self.n_moving = int(np.sum((np.asarray(joints.mimic_act_indices) >= 0)
+                                   | (np.asarray(joints.actuated_indices) >= 0)
+                                   | (np.asarray(joints.mimic_offset, dtype=np.float32) != 0)))
         self._derived: dict = {}
 
     def derived(self, key, make):
@@ -102,7 +106,8 @@ class _LinkPosesFn(torch.autograd.Function):
 
         (x,) = ctx.saved_tensors
         t = ctx.tables
-        return fk_vjp(x.detach(), g.contiguous(), *t.robot_buffers(), t.link_parent_joint), None
+        return fk_vjp(x.detach(), g.contiguous(), *t.robot_buffers(), t.link_parent_joint,
+                      max_moving=t.n_moving), None
 
 
 class Robot:

@@ -514,61 +514,162 @@ static int launch_fk(void* stream, const float* cfg, int64_t batch, int32_t n_ac
 // So a link's cotangent (g_q = (g_w, g_u), g_t) acts on q_j through the wrench
 //   F = g_t,   tau = t x g_t + 1/2 (w g_u - g_w u + u x g_u)   (quat = (w, u)),
 // and dL/dq_j = v_s . F_sub + w_s . tau_sub with the wrench summed over the
-// subtree below j.  Each lane recomputes its configuration's FK (no pose
-// residual in HBM), adds every link's wrench to its parent joint, then walks
-// the slots in reverse topological order: a slot's wrench is complete when it
-// is reached, is projected on the slot's twist (times the mimic multiplier,
-// into the actuated source), and is passed to the parent slot.
-__global__ __launch_bounds__(64) void fk_vjp_kernel(
-    const float* __restrict__ cfg, long long batch, int n_act, RobotTables tables,
-    const int* __restrict__ link_parent_joint, int n_links, const float* __restrict__ cot,
-    float* __restrict__ out_dq) {
-  extern __shared__ float smem[];
-  const int J = tables.n_joints;
-  JointRec* recs = reinterpret_cast<JointRec*>(smem);
-  int* slot_of = reinterpret_cast<int*>(recs + J);
-  float* cfg_tile = reinterpret_cast<float*>(slot_of + J);   // [a][lane], stride 65
-  float* poses = cfg_tile + n_act * kLaneStride;             // [slot*7+c][lane]
-  float* wrench = poses + 7 * J * kLaneStride;               // [slot*6+c][lane]
+// subtree below j.
+//
+// What bounds it is the chain of one configuration and the LDS its lanes share.
+// With a lane walking all joints of a configuration and a pose and a wrench per
+// joint in LDS, Baxter (43 joints, 14 of them moving) took 145 KiB a wave, one
+// wave a CU: 111 us for 30011 configurations.  Here the constant joints are
+// folded into the moving ones (each lane of the prologue composes its joint's
+// constant chain), so a workgroup of four waves keeps pose and wrench of the
+// moving joints only for its 64 configurations (lanes): the first wave walks
+// them, then every wave takes the links of every fourth moving joint (the
+// wrenches of one joint stay in one wave's registers: no race, a fixed order),
+// then the subtree sums and projections of every fourth joint: 28 us.
+constexpr int kVjpWaves = 4;
 
-  const int lane = threadIdx.x;
+// One moving joint: its record with the constant joints above folded into ptf.
+struct VjpNode {
+  JointRec r;                  // parent_slot = parent node, joint = slot
+  unsigned long long subtree;  // nodes at or below it
+};
+
+// LDS image; nodes = moving joints the tables may have (J at most).
+struct VjpLds {
+  int recs, nodes, rel, anchor, slot_of, lnode, cfg, pose, wrench, total;
+};
+// The joint records are only needed before the first pose is written and share
+// the poses' place.
+__host__ __device__ inline VjpLds vjp_lds(int J, int L, int n_act, int nodes) {
+  VjpLds o;
+  o.nodes = 0;
+  o.rel = o.nodes + static_cast<int>(sizeof(VjpNode)) * nodes;  // constant chain above each slot
+  o.anchor = o.rel + 28 * J;                                // node at or above each slot, -1 none
+  o.slot_of = o.anchor + 4 * J;
+  o.lnode = o.slot_of + 4 * J;                              // node of each link
+  o.cfg = o.lnode + 4 * L;                                  // [a][lane], stride 65
+  o.pose = o.cfg + 4 * n_act * kLaneStride;                 // [node * 7 + c][lane]
+  o.recs = o.pose;
+  o.wrench = o.pose + 4 * 7 * nodes * kLaneStride;          // [node * 6 + c][lane]
+  const int end = o.wrench + 4 * 6 * nodes * kLaneStride, recs_end = o.recs + static_cast<int>(sizeof(JointRec)) * J;
+  o.total = end > recs_end ? end : recs_end;
+  return o;
+}
+
+__global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
+    const float* __restrict__ cfg, long long batch, int n_act, RobotTables tables,
+    const int* __restrict__ link_parent_joint, int n_links, int max_nodes, const float* __restrict__ cot,
+    float* __restrict__ out_dq) {
+  extern __shared__ char vsmem[];
+  const int J = tables.n_joints;
+  const VjpLds lay = vjp_lds(J, n_links, n_act, max_nodes);
+  VjpNode* nodes = reinterpret_cast<VjpNode*>(vsmem + lay.nodes);
+  JointRec* recs = reinterpret_cast<JointRec*>(vsmem + lay.recs);
+  float* rel = reinterpret_cast<float*>(vsmem + lay.rel);
+  int* anchor = reinterpret_cast<int*>(vsmem + lay.anchor);
+  int* slot_of = reinterpret_cast<int*>(vsmem + lay.slot_of);
+  int* lnode = reinterpret_cast<int*>(vsmem + lay.lnode);
+  float* cfg_tile = reinterpret_cast<float*>(vsmem + lay.cfg);
+  float* poses = reinterpret_cast<float*>(vsmem + lay.pose);
+  float* wrench = reinterpret_cast<float*>(vsmem + lay.wrench);
+
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave, wave = uniform_i(tid / kWave);
   const long long b0 = static_cast<long long>(blockIdx.x) * kWave;
   const int n_valid = static_cast<int>(min(static_cast<long long>(kWave), batch - b0));
   const float* cfg_blk = cfg + b0 * n_act;
-  const int n_cfg = n_valid * n_act;
-  stage_joint_records(tables, recs, slot_of);
-  for (int f = lane; f < n_cfg; f += kWave) {
+  for (int f = tid; f < n_valid * n_act; f += kWave * kVjpWaves) {
     const int l = f / n_act, a = f - l * n_act;
     cfg_tile[a * kLaneStride + l] = cfg_blk[f];
   }
-  for (int i = 0; i < 6 * J; ++i) wrench[i * kLaneStride + lane] = 0.f;
-  __syncthreads();
-  if (lane >= n_valid) return;  // no barrier below
-  fk_walk(recs, J, [&](int a) { return cfg_tile[a * kLaneStride + lane]; }, poses, lane);
-
-  const float* g = cot + (b0 + lane) * static_cast<long long>(n_links) * 7;
-  for (int l = 0; l < n_links; ++l) {
-    const int pj = link_parent_joint[l];
-    const int s = (pj >= 0 && pj < J) ? slot_of[pj] : -1;
-    if (s < 0) continue;  // a root link's pose is the constant identity
-    const Pose T = lds_get_pose(poses, s, lane);
-    const float gw = g[7 * l], gx = g[7 * l + 1], gy = g[7 * l + 2], gz = g[7 * l + 3];
-    const float fx = g[7 * l + 4], fy = g[7 * l + 5], fz = g[7 * l + 6];
-    const float tau_x = (T.ty * fz - T.tz * fy) + 0.5f * (T.w * gx - gw * T.x + (T.y * gz - T.z * gy));
-    const float tau_y = (T.tz * fx - T.tx * fz) + 0.5f * (T.w * gy - gw * T.y + (T.z * gx - T.x * gz));
-    const float tau_z = (T.tx * fy - T.ty * fx) + 0.5f * (T.w * gz - gw * T.z + (T.x * gy - T.y * gx));
-    float* W = wrench + s * 6 * kLaneStride + lane;
-    W[0] += fx; W[kLaneStride] += fy; W[2 * kLaneStride] += fz;
-    W[3 * kLaneStride] += tau_x; W[4 * kLaneStride] += tau_y; W[5 * kLaneStride] += tau_z;
+  for (int l = tid; l < n_links; l += kWave * kVjpWaves) lnode[l] = link_parent_joint[l];
+  stage_joint_records(tables, recs, slot_of);
+  // Every wave counts the moving slots for itself (J <= 64: one per lane).
+  const bool moving = lane < J && recs[min(lane, J - 1)].kind != 0;
+  const unsigned long long moves = J > 0 ? __ballot(moving) : 0ull;
+  const int n_nodes = __popcll(moves);
+  if (n_nodes > max_nodes) {  // the caller's bound does not hold: reported as NaN
+    for (int f = tid; f < n_valid * n_act; f += kWave * kVjpWaves) out_dq[b0 * n_act + f] = __builtin_nanf("");
+    return;
   }
-  // dq accumulates in the (no longer needed) configuration tile column.
-  for (int a = 0; a < n_act; ++a) cfg_tile[a * kLaneStride + lane] = 0.f;
-  for (int i = J - 1; i >= 0; --i) {
-    const JointRec& r = recs[i];
-    const float* W = wrench + i * 6 * kLaneStride + lane;
-    const float F[3] = {W[0], W[kLaneStride], W[2 * kLaneStride]};
-    const float tau[3] = {W[3 * kLaneStride], W[4 * kLaneStride], W[5 * kLaneStride]};
-    if (r.src >= 0 && r.kind != 0) {
+  auto node_of = [&](int slot) { return __popcll(moves & ((1ull << slot) - 1ull)); };
+  if (wave == 0 && lane < J) {
+    // A parent's slot is below its child's, so the walk up ends.
+    Pose T = load_pose(recs[lane].ptf);
+    int p = recs[lane].parent_slot;
+    while (p >= 0 && recs[p].kind == 0) {
+      T = compose(load_pose(recs[p].ptf), T);
+      p = recs[p].parent_slot;
+    }
+    const int par = p >= 0 ? node_of(p) : -1;
+    float* d = rel + 7 * lane;
+    if (moving) {
+      VjpNode& n = nodes[node_of(lane)];
+      n.r = recs[lane];
+      n.r.ptf[0] = T.w; n.r.ptf[1] = T.x; n.r.ptf[2] = T.y; n.r.ptf[3] = T.z;
+      n.r.ptf[4] = T.tx; n.r.ptf[5] = T.ty; n.r.ptf[6] = T.tz;
+      n.r.parent_slot = par;
+      n.subtree = 0;
+      T = pose_identity();
+    }
+    anchor[lane] = moving ? node_of(lane) : par;
+    d[0] = T.w; d[1] = T.x; d[2] = T.y; d[3] = T.z; d[4] = T.tx; d[5] = T.ty; d[6] = T.tz;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    if (lane < n_nodes)
+      for (int p = lane; p >= 0; p = nodes[p].r.parent_slot) atomicOr(&nodes[p].subtree, 1ull << lane);
+    if (lane < n_valid) {
+      for (int n = 0; n < n_nodes; ++n) {
+        const JointRec& r = nodes[n].r;
+        const float q = ((r.src >= 0) ? cfg_tile[r.src * kLaneStride + lane] : 0.f) * r.mul + r.off;
+        Pose T = joint_local(r, q);
+        if (r.parent_slot >= 0) T = compose(lds_get_pose(poses, r.parent_slot, lane), T);
+        lds_put_pose(poses, n, lane, T);
+      }
+    }
+  } else {
+    // Meanwhile: each link's slot, and from it its node (-1: a link that does not move).
+    for (int l = tid - kWave; l < n_links; l += kWave * (kVjpWaves - 1)) {
+      const int pj = lnode[l];
+      lnode[l] = (pj >= 0 && pj < J) ? slot_of[pj] : -1;
+    }
+  }
+  __syncthreads();
+
+  const float* g = cot + (b0 + min(lane, n_valid - 1)) * static_cast<long long>(n_links) * 7;
+  for (int n = wave; n < n_nodes; n += kVjpWaves) {
+    float W[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const Pose N = lds_get_pose(poses, n, lane);
+    for (int l0 = 0; l0 < n_links; l0 += kWave) {
+      const int ls = l0 + lane < n_links ? lnode[l0 + lane] : -1;
+      for (unsigned long long m = __ballot(ls >= 0 && anchor[max(ls, 0)] == n); m != 0; m &= m - 1ull) {
+        const int l = l0 + __builtin_ctzll(m);
+        const float gw = g[7 * l], gx = g[7 * l + 1], gy = g[7 * l + 2], gz = g[7 * l + 3];
+        const float fx = g[7 * l + 4], fy = g[7 * l + 5], fz = g[7 * l + 6];
+        const Pose T = compose(N, load_pose(rel + 7 * lnode[l]));
+        W[0] += fx; W[1] += fy; W[2] += fz;
+        W[3] += (T.ty * fz - T.tz * fy) + 0.5f * (T.w * gx - gw * T.x + (T.y * gz - T.z * gy));
+        W[4] += (T.tz * fx - T.tx * fz) + 0.5f * (T.w * gy - gw * T.y + (T.z * gx - T.x * gz));
+        W[5] += (T.tx * fy - T.ty * fx) + 0.5f * (T.w * gz - gw * T.z + (T.x * gy - T.y * gx));
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 6; ++c) wrench[(6 * n + c) * kLaneStride + lane] = W[c];
+  }
+  __syncthreads();
+  // Subtree sums and projections; a node's dq contribution replaces the first
+  // component of its pose, which no other node reads here.
+  for (int n = wave; n < n_nodes; n += kVjpWaves) {
+    const JointRec& r = nodes[n].r;
+    float d = 0.f;
+    if (r.src >= 0) {
+      float W[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (unsigned long long m = nodes[n].subtree; m != 0; m &= m - 1ull) {
+        const float* w = wrench + 6 * __builtin_ctzll(m) * kLaneStride + lane;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) W[c] += w[c * kLaneStride];
+      }
       float v[3] = {0.f, 0.f, 0.f}, w[3] = {0.f, 0.f, 0.f};
       if (r.kind == 4) {
         w[0] = r.ang[0] * r.lin[0]; w[1] = r.ang[1] * r.lin[0]; w[2] = r.ang[2] * r.lin[0];
@@ -576,33 +677,63 @@ __global__ __launch_bounds__(64) void fk_vjp_kernel(
         v[0] = r.lin[0]; v[1] = r.lin[1]; v[2] = r.lin[2];
         if (r.kind == 3) { w[0] = r.ang[0]; w[1] = r.ang[1]; w[2] = r.ang[2]; }
       }
-      const Pose T = lds_get_pose(poses, i, lane);
+      const Pose T = lds_get_pose(poses, n, lane);
       float ws[3], vs[3];
       quat_rotate(T.w, T.x, T.y, T.z, w[0], w[1], w[2], ws[0], ws[1], ws[2]);
       quat_rotate(T.w, T.x, T.y, T.z, v[0], v[1], v[2], vs[0], vs[1], vs[2]);
       vs[0] += T.ty * ws[2] - T.tz * ws[1];
       vs[1] += T.tz * ws[0] - T.tx * ws[2];
       vs[2] += T.tx * ws[1] - T.ty * ws[0];
-      const float d = vs[0] * F[0] + vs[1] * F[1] + vs[2] * F[2] + ws[0] * tau[0] + ws[1] * tau[1] +
-                      ws[2] * tau[2];
-      cfg_tile[r.src * kLaneStride + lane] += r.mul * d;
+      d = r.mul * (vs[0] * W[0] + vs[1] * W[1] + vs[2] * W[2] + ws[0] * W[3] + ws[1] * W[4] + ws[2] * W[5]);
     }
-    if (r.parent_slot >= 0) {
-      float* P = wrench + r.parent_slot * 6 * kLaneStride + lane;
-      P[0] += F[0]; P[kLaneStride] += F[1]; P[2 * kLaneStride] += F[2];
-      P[3 * kLaneStride] += tau[0]; P[4 * kLaneStride] += tau[1]; P[5 * kLaneStride] += tau[2];
-    }
+    poses[7 * n * kLaneStride + lane] = d;
   }
-  float* o = out_dq + (b0 + lane) * n_act;
-  for (int a = 0; a < n_act; ++a) o[a] = cfg_tile[a * kLaneStride + lane];
-}
-
-static size_t fk_vjp_lds_bytes(int J, int n_act) {
-  return sizeof(JointRec) * J + sizeof(int) * J +
-         sizeof(float) * (static_cast<size_t>(n_act) + 13 * J) * kLaneStride;
+  __syncthreads();
+  for (int a = wave; a < n_act; a += kVjpWaves) {
+    float d = 0.f;
+    for (int n = n_nodes - 1; n >= 0; --n)
+      if (nodes[n].r.src == a) d += poses[7 * n * kLaneStride + lane];
+    cfg_tile[a * kLaneStride + lane] = d;
+  }
+  __syncthreads();
+  for (int f = tid; f < n_valid * n_act; f += kWave * kVjpWaves) {
+    const int l = f / n_act, a = f - l * n_act;
+    out_dq[b0 * n_act + f] = cfg_tile[a * kLaneStride + l];
+  }
 }
 
 }  // namespace pk
+
+namespace {
+
+// max_moving: a bound on the moving joints (actuated, mimic or with an offset),
+// which sizes the LDS.
+int launch_fk_vjp(void* stream, const float* cfg, int64_t batch, int32_t n_act, const pk::RobotTables& t,
+                  const int32_t* link_parent_joint, int32_t n_links, int32_t max_moving, const float* cot_links,
+                  float* out_dq) {
+  PK_REQUIRE(batch >= 0, "batch must be >= 0 (got %lld)", (long long)batch);
+  PK_REQUIRE(t.n_joints >= 0 && t.n_joints <= pk::kMaxJoints, "n_joints=%d outside [0, %d]", t.n_joints,
+             pk::kMaxJoints);
+  PK_REQUIRE(n_act >= 0 && n_act <= pk::kMaxAct, "n_act=%d outside [0, %d]", n_act, pk::kMaxAct);
+  PK_REQUIRE(n_links >= 0 && n_links <= pk::kMaxJoints + 1, "n_links=%d too large", n_links);
+  PK_REQUIRE(max_moving >= 0 && max_moving <= t.n_joints, "max_moving=%d outside [0, %d]", max_moving, t.n_joints);
+  if (batch == 0 || n_act == 0) return PK_OK;
+  PK_REQUIRE(cfg && out_dq && (n_links == 0 || (cot_links && link_parent_joint)), "null pointer");
+  if (t.n_joints > 0)
+    PK_REQUIRE(t.twists && t.parent_tf && t.parent_idx && t.act_idx && t.mimic_mul && t.mimic_off &&
+                   t.mimic_act_idx && t.topo_inv,
+               "null robot table pointer");
+  const long long blocks = (batch + pk::kWave - 1) / pk::kWave;
+  PK_REQUIRE(blocks <= 0x7fffffffLL, "batch too large");
+  const size_t lds = static_cast<size_t>(pk::vjp_lds(t.n_joints, n_links, n_act, max_moving).total);
+  PK_REQUIRE(lds <= 160 * 1024, "FK adjoint needs %zu bytes of LDS", lds);
+  hipLaunchKernelGGL(pk::fk_vjp_kernel, dim3(static_cast<unsigned>(blocks)), dim3(pk::kWave * pk::kVjpWaves), lds,
+                     static_cast<hipStream_t>(stream), cfg, static_cast<long long>(batch), n_act, t,
+                     link_parent_joint, n_links, max_moving, cot_links, out_dq);
+  return pk::check_launch("fk_vjp_kernel");
+}
+
+}  // namespace
 
 extern "C" int pk_fk_vjp_f32(void* stream, const float* cfg, int64_t batch, int32_t n_act,
                              const float* twists, const float* parent_tf,
@@ -611,27 +742,28 @@ extern "C" int pk_fk_vjp_f32(void* stream, const float* cfg, int64_t batch, int3
                              const int32_t* mimic_act_idx, const int32_t* topo_inv,
                              int32_t n_joints, const int32_t* link_parent_joint,
                              int32_t n_links, const float* cot_links, float* out_dq) {
-  PK_REQUIRE(batch >= 0, "batch must be >= 0 (got %lld)", (long long)batch);
-  PK_REQUIRE(n_joints >= 0 && n_joints <= pk::kMaxJoints, "n_joints=%d outside [0, %d]", n_joints,
-             pk::kMaxJoints);
-  PK_REQUIRE(n_act >= 0 && n_act <= pk::kMaxAct, "n_act=%d outside [0, %d]", n_act, pk::kMaxAct);
-  PK_REQUIRE(n_links >= 0 && n_links <= pk::kMaxJoints + 1, "n_links=%d too large", n_links);
-  if (batch == 0 || n_act == 0) return PK_OK;
-  PK_REQUIRE(cfg && out_dq && (n_links == 0 || (cot_links && link_parent_joint)), "null pointer");
-  if (n_joints > 0)
-    PK_REQUIRE(twists && parent_tf && parent_idx && act_idx && mimic_mul && mimic_off &&
-                   mimic_act_idx && topo_inv,
-               "null robot table pointer");
-  const long long blocks = (batch + pk::kWave - 1) / pk::kWave;
-  PK_REQUIRE(blocks <= 0x7fffffffLL, "batch too large");
-  const size_t lds = pk::fk_vjp_lds_bytes(n_joints, n_act);
-  PK_REQUIRE(lds <= 160 * 1024, "FK adjoint needs %zu bytes of LDS", lds);
-  pk::RobotTables t{twists, parent_tf, parent_idx, act_idx, mimic_mul,
-                    mimic_off, mimic_act_idx, topo_inv, n_joints, n_act};
-  hipLaunchKernelGGL(pk::fk_vjp_kernel, dim3(static_cast<unsigned>(blocks)), dim3(pk::kWave), lds,
-                     static_cast<hipStream_t>(stream), cfg, static_cast<long long>(batch), n_act, t,
-                     link_parent_joint, n_links, cot_links, out_dq);
-  return pk::check_launch("fk_vjp_kernel");
+  const pk::RobotTables t{twists, parent_tf, parent_idx, act_idx, mimic_mul,
+                          mimic_off, mimic_act_idx, topo_inv, n_joints, n_act};
+  // Any joint may move; a table of 46 joints that all do is one too many for the
+  // LDS and reported as NaN, as a broken bound is.
+  int32_t moving = n_joints;
+  if (n_joints == 46 && n_links >= 0 && n_links <= pk::kMaxJoints + 1 &&
+      pk::vjp_lds(n_joints, n_links, n_act, moving).total > 160 * 1024)
+    --moving;
+  return launch_fk_vjp(stream, cfg, batch, n_act, t, link_parent_joint, n_links, moving, cot_links, out_dq);
+}
+
+extern "C" int pk_fk_vjp_moving_f32(void* stream, const float* cfg, int64_t batch, int32_t n_act,
+                                    const float* twists, const float* parent_tf,
+                                    const int32_t* parent_idx, const int32_t* act_idx,
+                                    const float* mimic_mul, const float* mimic_off,
+                                    const int32_t* mimic_act_idx, const int32_t* topo_inv,
+                                    int32_t n_joints, const int32_t* link_parent_joint,
+                                    int32_t n_links, int32_t max_moving, const float* cot_links,
+                                    float* out_dq) {
+  const pk::RobotTables t{twists, parent_tf, parent_idx, act_idx, mimic_mul,
+                          mimic_off, mimic_act_idx, topo_inv, n_joints, n_act};
+  return launch_fk_vjp(stream, cfg, batch, n_act, t, link_parent_joint, n_links, max_moving, cot_links, out_dq);
 }
 
 extern "C" int pk_fk_f32(void* stream, const float* cfg, int64_t batch, int32_t n_act,

@@ -111,6 +111,7 @@ _SIGNATURES = {
     "pk_fk_f32": (_i32, [_p, _p, _i64, _i32] + [_p] * 10 + [_i32, _i32, _p]),
     "pk_fk_links_f32": (_i32, [_p, _p, _i64, _i32] + [_p] * 8 + [_i32, _p, _i32, _p]),
     "pk_fk_vjp_f32": (_i32, [_p, _p, _i64, _i32] + [_p] * 8 + [_i32, _p, _i32, _p, _p]),
+    "pk_fk_vjp_moving_f32": (_i32, [_p, _p, _i64, _i32] + [_p] * 8 + [_i32, _p, _i32, _i32, _p, _p]),
     "pk_collision_world_sphere_reduced_f32": (
         _i32,
         [_p, _p, _p, _i64, _i32, _p, _i32, _p, _i32, _p, _i32, _p, _i32, _i32, _p],

@@ -102,8 +102,9 @@ def fk_links(cfg, twists, parent_tf, parent_idx, act_idx, mimic_mul, mimic_off, 
 
 
 def fk_vjp(cfg, cot_links, twists, parent_tf, parent_idx, act_idx, mimic_mul, mimic_off, mimic_act_idx,
-           topo_inv, link_parent_joint) -> torch.Tensor:
-    """``(*batch, n_act)``: the FK adjoint, J^T of the link poses applied to ``cot_links``."""
+           topo_inv, link_parent_joint, max_moving: int | None = None) -> torch.Tensor:
+    """``(*batch, n_act)``: the FK adjoint, J^T of the link poses applied to ``cot_links``.
+    ``max_moving`` bounds the joints that move (all of them by default)."""
     cfg = _dev(cfg, torch.float32)
     dev = cfg.device
     batch_axes = tuple(cfg.shape[:-1])
@@ -116,11 +117,11 @@ def fk_vjp(cfg, cot_links, twists, parent_tf, parent_idx, act_idx, mimic_mul, mi
     if tuple(cot.shape) != batch_axes + (n_links, 7):
         raise ValueError(f"cotangent shape {tuple(cot.shape)} != {batch_axes + (n_links, 7)}")
     out = torch.empty((batch, n_act), dtype=torch.float32, device=dev)
-    st = lib().pk_fk_vjp_f32(
-        _stream(), _ptr(cfg), batch, n_act, *[_ptr(t) for t in tb], tb[0].shape[0], _ptr(lpj),
-        n_links, _ptr(cot), _ptr(out),
-    )
-    check(st, "pk_fk_vjp_f32")
+    args = (_stream(), _ptr(cfg), batch, n_act, *[_ptr(t) for t in tb], tb[0].shape[0], _ptr(lpj), n_links)
+    if max_moving is None:
+        check(lib().pk_fk_vjp_f32(*args, _ptr(cot), _ptr(out)), "pk_fk_vjp_f32")
+    else:
+        check(lib().pk_fk_vjp_moving_f32(*args, int(max_moving), _ptr(cot), _ptr(out)), "pk_fk_vjp_moving_f32")
     return out.reshape(*batch_axes, n_act)
 
 
