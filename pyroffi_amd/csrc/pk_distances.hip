@@ -88,7 +88,7 @@ __device__ __forceinline__ float jax_sphere_dist(float x1, float y1, float z1, f
 // reads; spheres of one radius share a square root (sqrt and the subtraction
 // are monotone, so the minimum is the same).  Obstacle kinds are taken one
 // after the other, so the lanes of a wave test the same kind.  (The calls at
-// those sizes: both collision residuals of Fetch 617 -> 208 us, the distances
+// those sizes: both collision residuals of Fetch 617 -> 163 us, the distances
 // written as costs; the mixed world of UR5 491 -> 198 us.)
 // ---------------------------------------------------------------------------
 
@@ -213,6 +213,111 @@ __device__ __forceinline__ void kind_rows(const RowArgs& a, const float4* pos, c
   }
 }
 
+// The same rows with a wave per (link, 64 T obstacles): each lane keeps T
+// obstacles in registers and every sphere is one broadcast LDS read for all of
+// them, where kind_rows reads it per element and loads the obstacle per link.
+// Links are taken by falling number of spheres, so the waves' shares are even.
+template <int KIND, bool JAX, int T>
+__device__ __forceinline__ void wave_rows(const RowArgs& a, const float4* pos, const int* cnt, const int* order,
+                                          int part, long long row0, int M, int col) {
+  constexpr int width = KIND == 0 ? 4 : (KIND == 1 ? 7 : 15);
+  const float* data = KIND == 0 ? a.w.data[0] : (KIND == 1 ? a.w.data[1] : a.w.data[2]);
+  const int n_obs = KIND == 0 ? a.w.count[0] : (KIND == 1 ? a.w.count[1] : a.w.count[2]);
+  const int lane = threadIdx.x % kWave;
+  const int worker = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) + part * (kRowThreads / kWave);
+  const int n_workers = a.parts * (kRowThreads / kWave);
+  const int S = a.s_per_link, L = a.n_links;
+  const int n_chunks = (n_obs + kWave * T - 1) / (kWave * T);
+  float o[T][width], inv[T];
+  int held = -1;
+  for (int task = worker; task < L * n_chunks; task += n_workers) {
+    const int chunk = task / L;  // few chunks: the obstacles stay for most tasks
+    const int l = __builtin_amdgcn_readfirstlane(order[task - chunk * L]);
+    if (chunk != held) {
+      held = chunk;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const float* p = data + static_cast<long long>(width) * min((chunk * T + t) * kWave + lane, n_obs - 1);
+#pragma unroll
+        for (int c = 0; c < width; ++c) o[t][c] = p[c];
+        if (KIND == 1) {  // segment end b -> direction, and 1 / |b - a|^2 (0 for a point)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) o[t][3 + c] -= o[t][c];
+          const float uu = o[t][3] * o[t][3] + o[t][4] * o[t][4] + o[t][5] * o[t][5];
+          inv[t] = uu > 1e-12f ? 1.f / uu : 0.f;
+        }
+      }
+    }
+    const int n = __builtin_amdgcn_readfirstlane(cnt[l]);
+    const float4* p = pos + l * S;
+    float best[T];
+    unsigned m2[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) { best[t] = JAX ? INFINITY : kNoSphere; m2[t] = 0x7f800000u; }
+    float r = n > 0 ? p[0].w : 0.f;
+    auto close_run = [&]() {  // a run of equal radii ends: its square roots
+      if (KIND == 2) return;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        best[t] = fminf(best[t], sqrtf(__uint_as_float(m2[t])) - (r + o[t][KIND == 1 ? 6 : 3]));
+        m2[t] = 0x7f800000u;
+      }
+    };
+    for (int i = 0; i < n; ++i) {
+      const float4 c = p[i];
+      if (KIND != 2 && __builtin_amdgcn_readfirstlane(__float_as_int(c.w)) !=
+                           __builtin_amdgcn_readfirstlane(__float_as_int(r))) {
+        close_run();
+        r = c.w;
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        if (KIND == 0) {
+          const float dx = JAX ? (o[t][0] - c.x) + 1e-6f : c.x - o[t][0];
+          const float dy = JAX ? (o[t][1] - c.y) + 1e-6f : c.y - o[t][1];
+          const float dz = JAX ? (o[t][2] - c.z) + 1e-6f : c.z - o[t][2];
+          m2[t] = min_bits(m2[t], dx * dx + dy * dy + dz * dz);
+        } else if (KIND == 1) {
+          const float wx = c.x - o[t][0], wy = c.y - o[t][1], wz = c.z - o[t][2];
+          const float s = fminf(fmaxf((wx * o[t][3] + wy * o[t][4] + wz * o[t][5]) * inv[t], 0.f), 1.f);
+          const float dx = wx - s * o[t][3], dy = wy - s * o[t][4], dz = wz - s * o[t][5];
+          m2[t] = min_bits(m2[t], dx * dx + dy * dy + dz * dz);
+        } else {
+          best[t] = fminf(best[t], dist_sphere_box(c.x, c.y, c.z, c.w, o[t]));
+        }
+      }
+    }
+    if (n > 0) close_run();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int m = (chunk * T + t) * kWave + lane;
+      if (a.cost.on) best[t] = row_cost(a.cost, best[t]);
+      if (m < n_obs) __builtin_nontemporal_store(best[t], a.out + (row0 + l) * M + col + m);
+    }
+  }
+}
+
+// Rows of one obstacle kind.  A wave per link pays where it has two obstacles
+// a lane (200 spheres, 111 robot spheres, both collision residuals of 4099
+// configurations: 208 -> 163 us); with 48 to 96 of a kind and two spheres a link
+// it is slower than lane by lane (210 against 197 us), which also takes the
+// half-spaces, of which a scene has a handful.
+constexpr int kWaveRowsMin = 65;
+
+template <int KIND, bool JAX>
+__device__ __forceinline__ void rows_of_kind(const RowArgs& a, const float4* pos, const int* cnt, const int* order,
+                                             int part, long long row0, int M, int col) {
+  const int n = KIND == 0 ? a.w.count[0] : (KIND == 1 ? a.w.count[1] : (KIND == 2 ? a.w.count[2] : a.w.count[3]));
+  if constexpr (KIND < 3) {
+    if (n >= kWaveRowsMin) {
+      if (KIND != 0 || n <= 2 * kWave) wave_rows<KIND, JAX, 2>(a, pos, cnt, order, part, row0, M, col);
+      else wave_rows<KIND, JAX, KIND == 0 ? 4 : 2>(a, pos, cnt, order, part, row0, M, col);
+      return;
+    }
+  }
+  kind_rows<KIND, JAX>(a, pos, cnt, part, row0, M, col);
+}
+
 template <bool JAX>
 __global__ __launch_bounds__(kRowThreads) void link_rows_kernel(RowArgs a) {
   extern __shared__ float4 rsmem[];
@@ -220,6 +325,7 @@ __global__ __launch_bounds__(kRowThreads) void link_rows_kernel(RowArgs a) {
   float4* loc = rsmem;                             // sorted link-frame spheres, link l at l * S
   float4* pos = loc + LS;                          // the same in the world
   int* cnt = reinterpret_cast<int*>(pos + LS);     // spheres of each link
+  int* order = cnt + L;                            // links by falling number of spheres
   const int tid = threadIdx.x;
   for (int t = tid; t < LS; t += kRowThreads) {
     const float* s = a.table + 4LL * t;
@@ -252,6 +358,12 @@ __global__ __launch_bounds__(kRowThreads) void link_rows_kernel(RowArgs a) {
     atomicAdd(&cnt[l], 1);
   }
   __syncthreads();
+  for (int l = tid; l < L; l += kRowThreads) {
+    int rank = 0;
+    for (int i = 0; i < L; ++i) rank += cnt[i] > cnt[l] || (cnt[i] == cnt[l] && i < l);
+    order[rank] = l;
+  }
+  __syncthreads();
   const int M = a.w.total();
   const long long n_items = a.batch * a.parts;
   for (long long item = blockIdx.x; item < n_items; item += gridDim.x) {
@@ -269,14 +381,14 @@ __global__ __launch_bounds__(kRowThreads) void link_rows_kernel(RowArgs a) {
     }
     __syncthreads();
     int col = 0;
-    kind_rows<0, JAX>(a, pos, cnt, part, b * L, M, col);
+    rows_of_kind<0, JAX>(a, pos, cnt, order, part, b * L, M, col);
     if (!JAX) {
       col += a.w.count[0];
-      kind_rows<1, false>(a, pos, cnt, part, b * L, M, col);
+      rows_of_kind<1, false>(a, pos, cnt, order, part, b * L, M, col);
       col += a.w.count[1];
-      kind_rows<2, false>(a, pos, cnt, part, b * L, M, col);
+      rows_of_kind<2, false>(a, pos, cnt, order, part, b * L, M, col);
       col += a.w.count[2];
-      kind_rows<3, false>(a, pos, cnt, part, b * L, M, col);
+      rows_of_kind<3, false>(a, pos, cnt, order, part, b * L, M, col);
     }
     __syncthreads();
   }
@@ -381,9 +493,10 @@ static bool launch_link_rows(hipStream_t s, RowArgs a) {
   if (static_cast<long long>(a.n_links) * a.s_per_link > kRowSlots || per > 0x3fffffffLL) return false;
   constexpr long long kGroups = 256LL * 4;
   long long parts = 1;
-  if (a.batch < kGroups) parts = std::min((kGroups + a.batch - 1) / a.batch, (per + kRowThreads - 1) / kRowThreads);
+  if (a.batch < kGroups)
+    parts = std::min((kGroups + a.batch - 1) / a.batch, (per + 4 * kRowThreads - 1) / (4 * kRowThreads));
   a.parts = static_cast<int>(parts);
-  const size_t lds = sizeof(float4) * 2 * LS + sizeof(int) * a.n_links;
+  const size_t lds = sizeof(float4) * 2 * LS + sizeof(int) * 2 * a.n_links;
   const unsigned grid = static_cast<unsigned>(std::min(kGroups, a.batch * parts));
   hipLaunchKernelGGL((link_rows_kernel<JAX>), dim3(grid), dim3(kRowThreads), lds, s, a);
   return true;
