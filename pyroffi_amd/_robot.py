@@ -46,6 +46,7 @@ class _DeviceTables:
         self.n_moving = int(np.sum((np.asarray(joints.mimic_act_indices) >= 0)
                                    | (np.asarray(joints.actuated_indices) >= 0)
                                    | (np.asarray(joints.mimic_offset, dtype=np.float32) != 0)))
+        self.n_links = int(self.link_parent_joint.shape[0])
         self._derived: dict = {}
 
     def derived(self, key, make):
@@ -62,6 +63,13 @@ class _DeviceTables:
                 self._derived.clear()
             v = self._derived[key] = make()
         return v
+
+    def fk_args(self) -> tuple[int, ...]:
+        """The table arguments of the FK launches (the buffers have the kernels' types and layout)."""
+        return (self.twists.data_ptr(), self.parent_tf.data_ptr(), self.parent_idx.data_ptr(),
+                self.act_idx.data_ptr(), self.mimic_mul.data_ptr(), self.mimic_off.data_ptr(),
+                self.mimic_act_idx.data_ptr(), self.topo_inv.data_ptr(), self.twists.shape[0],
+                self.link_parent_joint.data_ptr(), self.n_links)
 
     def robot_buffers(self) -> tuple[torch.Tensor, ...]:
         """The 8 robot buffers of the reference FFI calls, in order."""
@@ -94,20 +102,20 @@ class _LinkPosesFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, tables):
-        from .kernels.ops import fk_links
+        from .kernels.ops import fk_links_of
 
         ctx.tables = tables
         ctx.save_for_backward(x)
-        return fk_links(x.detach(), *tables.robot_buffers(), tables.link_parent_joint)
+        return fk_links_of(x, tables)
 
     @staticmethod
     def backward(ctx, g):
-        from .kernels.ops import fk_vjp
+        from .kernels.ops import _dev, fk_vjp_of
 
+        # Saved-tensor hooks may hand back another layout, type or device.
         (x,) = ctx.saved_tensors
-        t = ctx.tables
-        return fk_vjp(x.detach(), g.contiguous(), *t.robot_buffers(), t.link_parent_joint,
-                      max_moving=t.n_moving), None
+        x = _dev(x, torch.float32, g.device)
+        return fk_vjp_of(x, _dev(g, torch.float32, x.device), ctx.tables), None
 
 
 class Robot:
@@ -149,7 +157,7 @@ class Robot:
         adjoint kernel (``pk_fk_vjp_f32``).
         """
         del unroll_fk, use_cuda
-        from .kernels.ops import fk_links
+        from .kernels.ops import fk_links_of
 
         x, back = _to_cuda(cfg)
         assert x.shape[-1] == self.joints.num_actuated_joints, (
@@ -158,8 +166,7 @@ class Robot:
         t = self.device_tables(x.device)
         if isinstance(cfg, torch.Tensor) and cfg.requires_grad and torch.is_grad_enabled():
             return back(_LinkPosesFn.apply(x, t))
-        out = fk_links(x, *t.robot_buffers(), t.link_parent_joint)
-        return back(out)
+        return back(fk_links_of(x, t))
 
     def forward_kinematics_joints(self, cfg):
         """World pose of each joint, ``(*batch, n_joints, 7)`` (the FK kernel's raw output)."""

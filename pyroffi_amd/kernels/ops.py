@@ -101,6 +101,30 @@ def fk_links(cfg, twists, parent_tf, parent_idx, act_idx, mimic_mul, mimic_off, 
     return out.reshape(*batch_axes, n_links, 7)
 
 
+def fk_links_of(cfg: torch.Tensor, tables) -> torch.Tensor:
+    """``fk_links`` for a contiguous float32 GPU configuration tensor and a robot's device tables
+    (``_DeviceTables``), which need no look at their types and layout (at 1000 configurations that
+    was half of the call's 16 us)."""
+    n_act = cfg.shape[-1]
+    out = torch.empty((*cfg.shape[:-1], tables.n_links, 7), dtype=torch.float32, device=cfg.device)
+    st = lib().pk_fk_links_f32(torch.cuda.current_stream().cuda_stream, cfg.data_ptr(),
+                               cfg.numel() // n_act if n_act else math.prod(cfg.shape[:-1]), n_act,
+                               *tables.fk_args(), out.data_ptr())
+    check(st, "pk_fk_links_f32")
+    return out
+
+
+def fk_vjp_of(cfg: torch.Tensor, cot: torch.Tensor, tables) -> torch.Tensor:
+    """``fk_vjp`` for the tensors and tables of ``fk_links_of``; ``cot`` contiguous float32 of the output's shape."""
+    n_act = cfg.shape[-1]
+    out = torch.empty_like(cfg)
+    st = lib().pk_fk_vjp_moving_f32(torch.cuda.current_stream().cuda_stream, cfg.data_ptr(),
+                                    cfg.numel() // n_act if n_act else math.prod(cfg.shape[:-1]), n_act,
+                                    *tables.fk_args(), tables.n_moving, cot.data_ptr(), out.data_ptr())
+    check(st, "pk_fk_vjp_moving_f32")
+    return out
+
+
 def fk_vjp(cfg, cot_links, twists, parent_tf, parent_idx, act_idx, mimic_mul, mimic_off, mimic_act_idx,
            topo_inv, link_parent_joint, max_moving: int | None = None) -> torch.Tensor:
     """``(*batch, n_act)``: the FK adjoint, J^T of the link poses applied to ``cot_links``.
