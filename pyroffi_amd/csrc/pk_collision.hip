@@ -9,6 +9,8 @@
 //   * lanes run across world obstacles -- each lane keeps T obstacles in
 //     registers for the whole launch -- and every robot sphere is read once
 //     from LDS as a broadcast and tested against the lane's T obstacles;
+//   * where only the configuration minimum is wanted, link balls rule out most
+//     pairs first (world_min_culled);
 //   * per-link minima are written as coalesced rows (lanes = obstacles), the
 //     per-configuration minimum is a wavefront min-reduction, and self pairs
 //     are reduced in registers along each lane's run of the entry list and
@@ -22,6 +24,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace pk {
@@ -168,6 +171,141 @@ __device__ __forceinline__ void link_sweep(int n, int g0, int g1, const float4* 
   }
 }
 
+// The candidates of the configuration minimum: (link, obstacle) pairs that a
+// link's bounding ball cannot rule out.  A wave holds at most one per lane.
+constexpr int kCandidates = kWave;
+constexpr int kCullMinSpheres = 12;  // see launch_sweep
+
+// LDS of one wave: the world spheres and a blank, then the expanded entries (rows)
+// or the placed balls and the candidates (minimum only); pose tile, pair minima.
+__host__ __device__ inline int sweep_float4_per_wave(int src, bool min_only, int K, int L) {
+  return (K + 1) + (src != 0 ? 0 : min_only ? L + kCandidates : K);
+}
+__host__ __device__ inline int sweep_words_per_wave(int src, bool min_only, int L, int P) {
+  return (src == 0 ? 7 * L : 0) + P + (min_only ? kCandidates : 0);
+}
+
+// Bounding ball of one link's spheres in the link frame: xyz = centre (of the
+// spheres' box), w = radius, and `near` = min_k(|c_k - centre| - r_k).  For an
+// obstacle o of radius R with s = |o - centre| - R, the link's distance lies in
+// [s - w, s + near].  Spheres that no minimum takes (a NaN or infinite centre, a
+// radius of -inf) are left out; a radius of +inf gives w = near = +inf about the
+// origin, which rules nothing out.
+__device__ __forceinline__ float4 link_ball(const float4* sl, int k0, int k1, float& near) {
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  bool any = false, sane = true;
+  auto counted = [](const float4& s) {
+    return fabsf(s.x) < INFINITY && fabsf(s.y) < INFINITY && fabsf(s.z) < INFINITY && s.w != -INFINITY;
+  };
+  for (int k = k0; k < k1; ++k) {
+    const float4 s = sl[k];
+    if (!counted(s)) continue;
+    any = true;
+    sane = sane && s.w < INFINITY;
+    const float c[3] = {s.x, s.y, s.z};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      lo[j] = fminf(lo[j], c[j] - s.w);
+      hi[j] = fmaxf(hi[j], c[j] + s.w);
+    }
+  }
+  const float bx = 0.5f * lo[0] + 0.5f * hi[0], by = 0.5f * lo[1] + 0.5f * hi[1], bz = 0.5f * lo[2] + 0.5f * hi[2];
+  float rb = -INFINITY;
+  near = INFINITY;
+  for (int k = k0; k < k1; ++k) {
+    const float4 s = sl[k];
+    if (!counted(s)) continue;
+    const float dx = s.x - bx, dy = s.y - by, dz = s.z - bz;
+    const float d = sqrtf(dx * dx + dy * dy + dz * dz);
+    rb = fmaxf(rb, d + s.w);
+    near = fminf(near, d - s.w);
+  }
+  sane = sane && fabsf(rb) < 1e6f;
+  // Slack for the rounding of the placed centre and of the distances.
+  near = any && sane ? near + 1e-5f : INFINITY;
+  if (!any) return make_float4(0.f, 0.f, 0.f, -INFINITY);
+  return sane ? make_float4(bx, by, bz, rb + 1e-5f) : make_float4(0.f, 0.f, 0.f, INFINITY);
+}
+
+// Exact minimum of the wave's `count` candidates (one per lane), into gmin.
+__device__ __forceinline__ void candidate_min(int lane, int count, const float4* cand, const unsigned* crange,
+                                              const float4* sc, float& gmin) {
+  wave_sync();
+  if (lane < count) {
+    const float4 o = cand[lane];
+    const unsigned r = crange[lane];
+    const int k1 = static_cast<int>(r >> 16);
+    float best = INFINITY;
+    for (int k = static_cast<int>(r & 0xffffu); k < k1; ++k) {
+      const float4 s = sc[k];
+      const float dx = s.x - o.x, dy = s.y - o.y, dz = s.z - o.z;
+      best = fminf(best, fast_sqrt(dx * dx + dy * dy + dz * dz) - s.w);
+    }
+    gmin = fminf(gmin, fminf(kBig, best - o.w));
+  }
+  wave_sync();
+}
+
+// Minimum distance of one configuration to a lane's T obstacles of this chunk,
+// where nothing but the minimum is wanted.  The sweep over every sphere is bound by
+// VALU issue, so the way to less time is fewer pairs: link by link, the least s over the
+// wave's obstacles gives bounds from below and above (link_ball); the least
+// upper bound U over links and obstacles (and earlier chunks) rules out every
+// pair that starts above it, and the few that are left (on Panda among 256
+// obstacles a few dozen of 2816) are collected, one per lane, and measured.
+// Lane i keeps the least s of link i, so at most 64 links are taken at a time.
+// Panda, 65536 configurations x 256 obstacles with poses and self pairs: 273 -> 220 us.
+template <int T>
+__device__ __forceinline__ void world_min_culled(int lane, int n_balls, const float4* ball, const float4* local_ball,
+                                                 const unsigned* brange, const float4* sc, float4* cand,
+                                                 unsigned* crange, const float (&ox)[T], const float (&oy)[T],
+                                                 const float (&oz)[T], const float (&orad)[T], float& upper,
+                                                 float& gmin) {
+  auto clear = [&](const float4& b, int t) {
+    const float dx = b.x - ox[t], dy = b.y - oy[t], dz = b.z - oz[t];
+    return fast_sqrt(dx * dx + dy * dy + dz * dz) - orad[t];
+  };
+  float first = INFINITY;  // least s of ball `lane`
+  for (int i = 0; i < n_balls; ++i) {
+    const float4 b = ball[i];
+    float s = clear(b, 0);
+#pragma unroll
+    for (int t = 1; t < T; ++t) s = fminf(s, clear(b, t));
+    s = wave_min(fminf(s, INFINITY));
+    if (lane == i) first = s;
+    upper = fminf(upper, s + b.w);
+  }
+  int count = 0;
+  unsigned long long hits =
+      __ballot(lane < n_balls && !(first - local_ball[min(lane, n_balls - 1)].w > upper));
+  while (hits) {
+    const int i = __builtin_ctzll(hits);
+    hits &= hits - 1;
+    const float4 b = ball[i];
+    const float rb = local_ball[i].w;
+    const unsigned range = brange[i];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const float s = clear(b, t);
+      const bool in = s == s && !(s - rb > upper);
+      const unsigned long long m = __ballot(in);
+      if (m == 0) continue;
+      const int add = __popcll(m);
+      if (count + add > kCandidates) {
+        candidate_min(lane, count, cand, crange, sc, gmin);
+        count = 0;
+      }
+      if (in) {
+        const int at = count + __popcll(m & ((1ull << lane) - 1));
+        cand[at] = make_float4(ox[t], oy[t], oz[t], orad[t]);
+        crange[at] = range;
+      }
+      count += add;
+    }
+  }
+  if (count) candidate_min(lane, count, cand, crange, sc, gmin);
+}
+
 // Waves per sweep workgroup.  They share the per-launch tables (local
 // spheres, self entries, groups) in LDS and each works through its own block
 // of configurations with private sphere, pose and pair-minimum buffers, so a
@@ -178,7 +316,8 @@ constexpr int kSweepWaves = 4;
 // world-frame sphere slots (the reference FFI layout).  T = obstacles per lane.
 // Six waves per SIMD (at most 80 VGPRs) for up to four obstacles per lane,
 // three with eight, which need the registers.
-template <int SRC, int T>
+// CULL: SRC 0 with no rows wanted, the minimum by world_min_culled.
+template <int SRC, int T, bool CULL>
 __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_kernel(SweepArgs a) {
   extern __shared__ float smem[];
   const int tid = threadIdx.x;
@@ -191,20 +330,27 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
   const int E = a.n_entries;
   const int P = a.n_pairs;
   // LDS carve-up: shared tables, then one float4 block and one word block per wave.
-  const int f4_per_wave = (K + 1) + (SRC == 0 ? K : 0);
-  const int words_per_wave = (SRC == 0 ? 7 * L : 0) + P;
+  static_assert(!CULL || SRC == 0, "link balls come from the local spheres");
+  const int f4_per_wave = sweep_float4_per_wave(SRC, CULL, K, L);
+  const int words_per_wave = sweep_words_per_wave(SRC, CULL, L, P);
   float4* sl = reinterpret_cast<float4*>(smem);                          // K local spheres (SRC 0)
   float4* sc = sl + (SRC == 0 ? K : 0) + wave * f4_per_wave;            // K world spheres + 1 blank
-  float4* se = sc + (K + 1);                                             // K expanded entries (SRC 0)
+  float4* se = sc + (K + 1);                                             // K expanded entries (SRC 0, rows)
+  float4* ball = sc + (K + 1);                                           // L placed balls (minimum only) ...
+  float4* cand = ball + L;                                               // ... and the candidates' obstacles
   const int n_it = (E + kWave - 1) / kWave;                             // self steps per lane
-  unsigned* sent = reinterpret_cast<unsigned*>(sl + (SRC == 0 ? K : 0) + kSweepWaves * f4_per_wave);  // n_it * 64
+  float4* lball = sl + (SRC == 0 ? K : 0) + kSweepWaves * f4_per_wave;   // L balls in link frames (minimum only)
+  unsigned* sent = reinterpret_cast<unsigned*>(lball + (CULL ? L : 0));  // n_it * 64
   int* lstart = reinterpret_cast<int*>(sent + n_it * kWave);             // L + 1
   int* slink = lstart + (L + 1);                                         // K: link of sphere (SRC 0)
   int* gstart = slink + (SRC == 0 ? K : 0);                              // K + 1: sphere groups
   int* lgroup = gstart + (K + 1);                                        // L + 1: groups of each link
   float* lrad2 = reinterpret_cast<float*>(lgroup + (L + 1));             // L: bound of |offset|^2 (SRC 0)
+  float* bnear = lrad2;                                                  // L: the balls' near bounds (minimum only)
   float* ptile = lrad2 + (SRC == 0 ? L : 0) + wave * words_per_wave;     // L * 7 poses (SRC 0)
   float* pmin = ptile + (SRC == 0 ? 7 * L : 0);                          // P
+  unsigned* crange = reinterpret_cast<unsigned*>(pmin + P);              // the candidates' spheres (minimum only)
+  unsigned* brange = reinterpret_cast<unsigned*>(gstart);                // L: the balls' spheres (minimum only)
 
   // Per-launch tables, staged by the whole workgroup.
   const int nt = kWave * kSweepWaves;
@@ -254,8 +400,9 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
   if (SRC == 0) {
     for (int n = tid; n < L; n += nt) {
       float r2 = 0.f;
+      for (int k = lstart[n]; k < lstart[n + 1]; ++k) slink[k] = n;
+      if constexpr (CULL) continue;
       for (int k = lstart[n]; k < lstart[n + 1]; ++k) {
-        slink[k] = n;
         const float4 s = sl[k];
         r2 = fmaxf(r2, s.x * s.x + s.y * s.y + s.z * s.z);
       }
@@ -267,7 +414,19 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
   // slots (SRC 1, whose radii are per configuration).  For one obstacle,
   // min_k(|c_k - o|) - r = sqrt(min_k |c_k - o|^2) - r inside a group, so a
   // group costs one square root per obstacle.
-  if (tid == 0) {
+  // Where only the minimum is wanted, the links with spheres and their balls instead.
+  if constexpr (CULL) {
+    if (tid == 0) {
+      int nb = 0;
+      for (int n = 0; n < L; ++n)
+        if (lstart[n] < lstart[n + 1])
+          brange[nb++] = static_cast<unsigned>(lstart[n]) | (static_cast<unsigned>(lstart[n + 1]) << 16);
+      lgroup[0] = nb;
+    }
+    __syncthreads();
+    for (int i = tid; i < lgroup[0]; i += nt)
+      lball[i] = link_ball(sl, static_cast<int>(brange[i] & 0xffffu), static_cast<int>(brange[i] >> 16), bnear[i]);
+  } else if (tid == 0) {
     int g = 0;
     for (int n = 0; n < L; ++n) {
       lgroup[n] = g;
@@ -305,6 +464,7 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
   const long long per = (a.batch + n_waves - 1) / n_waves;
   const long long b_begin = (static_cast<long long>(blockIdx.x) * kSweepWaves + wave) * per;
   const long long b_end = min(a.batch, b_begin + per);
+  const int n_balls = CULL ? __builtin_amdgcn_readfirstlane(lgroup[0]) : 0;
   for (long long b = b_begin; b < b_end; ++b) {
     // 1. Robot spheres of configuration b in the world frame -> LDS.
     if (SRC == 0) {
@@ -317,7 +477,16 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
         float wx, wy, wz;
         quat_rotate(p[0], p[1], p[2], p[3], s.x, s.y, s.z, wx, wy, wz);
         sc[k] = make_float4(wx + p[4], wy + p[5], wz + p[6], s.w);
-        se[k] = make_float4(-2.f * wx, -2.f * wy, -2.f * wz, wx * wx + wy * wy + wz * wz);
+        if (!CULL) se[k] = make_float4(-2.f * wx, -2.f * wy, -2.f * wz, wx * wx + wy * wy + wz * wz);
+      }
+      if constexpr (CULL) {
+        for (int i = lane; i < n_balls; i += kWave) {
+          const float* p = ptile + 7 * slink[brange[i] & 0xffffu];
+          const float4 s = lball[i];
+          float wx, wy, wz;
+          quat_rotate(p[0], p[1], p[2], p[3], s.x, s.y, s.z, wx, wy, wz);
+          ball[i] = make_float4(wx + p[4], wy + p[5], wz + p[6], bnear[i]);
+        }
       }
     } else {
       const long long BK = a.batch * K;
@@ -335,11 +504,17 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
     wave_sync();
 
     // 2. World sweep.
-    float gmin = INFINITY;
+    float gmin = INFINITY, upper = INFINITY;
     if (a.out_world != nullptr || a.out_min != nullptr) {
       for (int c = 0; c < n_chunks; ++c) {
         if (T == 8 && c > 0) load_obstacles(c);
-        if (SRC == 0 && a.out_world == nullptr) {
+        if constexpr (CULL) {
+          for (int i = 0; i < n_balls; i += kWave)
+            world_min_culled<T>(lane, min(kWave, n_balls - i), ball + i, lball + i, brange + i, sc, cand, crange, ox,
+                                oy, oz, orad, upper, gmin);
+          continue;
+        }
+        if (SRC == 0 && !CULL && a.out_world == nullptr) {
           // Only the configuration minimum is wanted.  Subtracting r_o is
           // monotone, so min_n fminf(kBig, acc_n - r_o) equals
           // fminf(kBig, min_n acc_n - r_o) (NaN and infinite cases included):
@@ -494,7 +669,7 @@ static long long resident_groups(const void* fn, int block, size_t lds, int max_
   return groups;
 }
 
-// One launch of sweep_kernel<SRC, T>: at least eight configurations per wave,
+// One launch of sweep_kernel<SRC, T, CULL>: at least eight configurations per wave,
 // and no more workgroups than are resident at once (each wave loops over its
 // block of configurations, so a second, partial round would only run at low
 // occupancy).  Residency is capped at six workgroups per CU (six waves per
@@ -502,35 +677,56 @@ static long long resident_groups(const void* fn, int block, size_t lds, int max_
 // 72 VGPRs -- made the launch 12% slower, the self phase included.
 constexpr int kSweepGroupsPerCu = 6;
 
-template <int SRC, int T>
+template <int SRC, int T, bool CULL>
 static void launch_sweep_t(hipStream_t s, const SweepArgs& a, size_t lds) {
-  const void* fn = reinterpret_cast<const void*>(&sweep_kernel<SRC, T>);
+  const void* fn = reinterpret_cast<const void*>(&sweep_kernel<SRC, T, CULL>);
   const long long want = (a.batch + 8 * kSweepWaves - 1) / (8 * kSweepWaves);
   long long cap = resident_groups(fn, kWave * kSweepWaves, lds, kSweepGroupsPerCu);
   if (cap <= 0) cap = 8192 / kSweepWaves;
   const unsigned grid = static_cast<unsigned>(std::max(1LL, std::min(want, cap)));
-  hipLaunchKernelGGL((sweep_kernel<SRC, T>), dim3(grid), dim3(kWave * kSweepWaves), lds, s, a);
+  hipLaunchKernelGGL((sweep_kernel<SRC, T, CULL>), dim3(grid), dim3(kWave * kSweepWaves), lds, s, a);
 }
 
 template <int SRC>
 static int launch_sweep(void* stream, const SweepArgs& a) {
   const int K = a.n_spheres, L = a.n_links;
-  const size_t per_wave = sizeof(float4) * ((K + 1) + (SRC == 0 ? K : 0)) +
-                          sizeof(float) * ((SRC == 0 ? 7 * L : 0) + a.n_pairs);
   const size_t n_slots = static_cast<size_t>((a.n_entries + kWave - 1) / kWave) * kWave;
-  size_t lds = sizeof(float4) * (SRC == 0 ? K : 0) + sizeof(unsigned) * n_slots +
-               sizeof(int) * ((L + 1) + (SRC == 0 ? K : 0) + (K + 1) + (L + 1)) +
-               sizeof(float) * (SRC == 0 ? L : 0) + per_wave * kSweepWaves;
+  auto lds_bytes = [&](bool min_only) {
+    const size_t per_wave = sizeof(float4) * sweep_float4_per_wave(SRC, min_only, K, L) +
+                            sizeof(float) * sweep_words_per_wave(SRC, min_only, L, a.n_pairs);
+    return sizeof(float4) * ((SRC == 0 ? K : 0) + (min_only ? L : 0)) + sizeof(unsigned) * n_slots +
+           sizeof(int) * ((L + 1) + (SRC == 0 ? K : 0) + (K + 1) + (L + 1)) +
+           sizeof(float) * (SRC == 0 ? L : 0) + per_wave * kSweepWaves;
+  };
+  // The bounds cost a fixed part of each configuration, which a robot of very few
+  // spheres does not win back.  32768 configurations, every pair / culled, us: 2 links
+  // x 2 spheres 19 / 23 (64 obstacles), 42 / 53 (512); 2 x 4, 27 / 29 (128), 65 / 58;
+  // 11 x 1, 43 / 38, 110 / 90; 2 x 8, 39 / 30, 111 / 54; 11 x 5, 114 / 58, 343 / 199.
+  // A very long entry list can also need more LDS with the candidates' buffers than
+  // without: such a launch sweeps every pair.
+  const bool cull = SRC == 0 && a.out_world == nullptr && a.out_min != nullptr && K >= kCullMinSpheres &&
+                    lds_bytes(true) <= 150 * 1024;
+  const size_t lds = lds_bytes(cull);
   PK_REQUIRE(a.n_entries == 0 || K < 1024, "self entries address at most 1023 spheres (got %d)", K);
   PK_REQUIRE(a.n_entries == 0 || a.n_pairs < 2048, "self entries address at most 2047 pairs (got %d)", a.n_pairs);
   PK_REQUIRE(lds <= 150 * 1024, "sphere tables need %zu bytes of LDS (limit 150 KiB)", lds);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (pick_t(a.n_world)) {
-    case 1: launch_sweep_t<SRC, 1>(s, a, lds); break;
-    case 2: launch_sweep_t<SRC, 2>(s, a, lds); break;
-    case 4: launch_sweep_t<SRC, 4>(s, a, lds); break;
-    default: launch_sweep_t<SRC, 8>(s, a, lds); break;
+  auto launch = [&](auto culled) {
+    constexpr bool kCull = decltype(culled)::value;
+    switch (pick_t(a.n_world)) {
+      case 1: launch_sweep_t<SRC, 1, kCull>(s, a, lds); break;
+      case 2: launch_sweep_t<SRC, 2, kCull>(s, a, lds); break;
+      case 4: launch_sweep_t<SRC, 4, kCull>(s, a, lds); break;
+      default: launch_sweep_t<SRC, 8, kCull>(s, a, lds); break;
+    }
+  };
+  if constexpr (SRC == 0) {
+    if (cull) {
+      launch(std::true_type{});
+      return check_launch("sweep_kernel");
+    }
   }
+  launch(std::false_type{});
   return check_launch("sweep_kernel");
 }
 
