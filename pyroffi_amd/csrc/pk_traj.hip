@@ -432,11 +432,11 @@ __device__ __forceinline__ void pull_point(const WaypointNodes<MAXN, GRAD>& K, i
 // waypoint with node poses K.P, this lane's share, into the group's LDS slot
 // gc = [K spheres | L link bounds].  Links are visited in table order and a
 // node's rotation is rebuilt only when the node changes (the host sorts links
-// by node).
-template <int MAXN, bool GRAD>
+// by node).  GROUP: lanes that share the waypoint.
+template <int MAXN, bool GRAD, int GROUP = kGroup>
 __device__ __forceinline__ void waypoint_centres(const TrajModelDev& md, const TrajLds& L,
                                                  const WaypointNodes<MAXN, GRAD>& K, float4* gc) {
-  const int g = threadIdx.x % kGroup;
+  const int g = threadIdx.x % GROUP;
   const int Ks = md.n_spheres;
   int prev = -2;
   Pose T = pose_identity();
@@ -449,13 +449,13 @@ __device__ __forceinline__ void waypoint_centres(const TrajModelDev& md, const T
       prev = node;
     }
     const int k0 = L.link_sph[l], k1 = L.link_sph[l + 1];
-    for (int s = k0 + g; s < k1; s += kGroup) {
+    for (int s = k0 + g; s < k1; s += GROUP) {
       const float4 sp = L.sph[s];
       gc[s] = make_float4(R.m00 * sp.x + R.m01 * sp.y + R.m02 * sp.z + T.tx,
                           R.m10 * sp.x + R.m11 * sp.y + R.m12 * sp.z + T.ty,
                           R.m20 * sp.x + R.m21 * sp.y + R.m22 * sp.z + T.tz, sp.w);
     }
-    if (g == l % kGroup) {
+    if (g == l % GROUP) {
       const float4 b = L.lb[l];
       gc[Ks + l] = make_float4(R.m00 * b.x + R.m01 * b.y + R.m02 * b.z + T.tx,
                                R.m10 * b.x + R.m11 * b.y + R.m12 * b.z + T.ty,
@@ -1418,11 +1418,27 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_chomp_kernel(ChompArgs a
 // gradients are accumulated per link as a wrench (F, c x F) and pulled back to
 // the link's ancestor nodes once per link: dq_a += v_a . F + w_a . (tau - p_a x F).
 constexpr int kMaxScoGroups = 8;
+constexpr int kScoWaveThreads = 256;  // of the whole-wave linearisation
 
-__device__ __forceinline__ float group8_min(float v) {
-  v = fminf(v, __shfl_xor(v, 1, kWave));
-  v = fminf(v, __shfl_xor(v, 2, kWave));
-  return fminf(v, __shfl_xor(v, 4, kWave));
+// Whether the linearisation gives each waypoint a whole wave.  Panda, eight lanes /
+// a wave, us: 6144 waypoints among 512 spheres 536 / 179, among 32 150 / 100; 8192,
+// 548 / 228 and 153 / 132; 16384, 624 / 430 and 174 / 250; 32768, 649 / 820.  A wave
+// repeats the waypoint's kinematics in every lane, which few obstacles do not repay.
+inline bool sco_wave_per_waypoint(long long n_waypoints, int n_world) {
+  return n_waypoints <= (n_world >= 256 ? 16384 : 8192);
+}
+
+template <int GROUP>
+__device__ __forceinline__ float lanes_min(float v) {
+#pragma unroll
+  for (int off = 1; off < GROUP; off <<= 1) v = fminf(v, __shfl_xor(v, off, kWave));
+  return v;
+}
+
+template <int GROUP>
+__device__ __forceinline__ float lanes_sum(float v) {
+  static_assert(GROUP == kGroup || GROUP == kWave, "no reduction for this group");
+  return GROUP == kWave ? traj_wave_sum(v) : group_sum(v);
 }
 
 template <int MAXN>
@@ -1476,12 +1492,12 @@ __device__ __forceinline__ float pair_dist(const TrajLds& L, const float4* gc, i
   return best;
 }
 
-template <int MAXN>
+template <int MAXN, int GROUP>
 __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const TrajLds& L,
                                                  const WaypointNodes<MAXN, true>& K, const float4* gc,
                                                  const int* gstart, int gi, float tau, float& dk,
                                                  float (&gn)[MAXN]) {
-  const int g = threadIdx.x % kGroup;
+  const int g = threadIdx.x % GROUP;
 #pragma unroll
   for (int a = 0; a < MAXN; ++a) gn[a] = 0.f;
   float bx, by, bz, bn;
@@ -1490,13 +1506,13 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
   if (gi == 0) {
     // Self pairs (a few dozen): pass 1 the group minimum, pass 2 the weights.
     dmin = INFINITY;
-    for (int p = g; p < md.n_pairs; p += kGroup) dmin = fminf(dmin, pair_dist(L, gc, p, bx, by, bz, bn, bc, bc2));
-    dmin = group8_min(dmin);
+    for (int p = g; p < md.n_pairs; p += GROUP) dmin = fminf(dmin, pair_dist(L, gc, p, bx, by, bz, bn, bc, bc2));
+    dmin = lanes_min<GROUP>(dmin);
     if (!(dmin < INFINITY)) {  // empty group
       dk = INFINITY;
       return;
     }
-    for (int p = g; p < md.n_pairs; p += kGroup) {
+    for (int p = g; p < md.n_pairs; p += GROUP) {
       const float d = pair_dist(L, gc, p, bx, by, bz, bn, bc, bc2);
       const float w = __expf(-(d - dmin) / tau);
       if (!(w > 0.f)) continue;
@@ -1526,14 +1542,15 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
       // obstacle order, the order of one obstacle at a time.  Sixteen per pass
       // measured 3% faster than eight and 27% faster than four (112 VGPRs,
       // no spills).
-      constexpr int kObs = 16;
-      for (int mb = m0 + g; mb < m1; mb += kGroup * kObs) {
+      // A whole wave has at most a few obstacles a lane: four.
+      constexpr int kObs = GROUP == kWave ? 4 : 16;
+      for (int mb = m0 + g; mb < m1; mb += GROUP * kObs) {
         float4 o[kObs];
         float best[kObs];
         int bs[kObs];
 #pragma unroll
         for (int u = 0; u < kObs; ++u) {
-          const int m = mb + u * kGroup;
+          const int m = mb + u * GROUP;
           const float4 w = L.world[m < m1 ? m : mb];
           o[u] = make_float4(w.x + 1e-6f, w.y + 1e-6f, w.z + 1e-6f, w.w);  // centre + e
           best[u] = INFINITY;
@@ -1549,7 +1566,7 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
         }
 #pragma unroll
         for (int u = 0; u < kObs; ++u) {
-          if (mb + u * kGroup >= m1) break;
+          if (mb + u * GROUP >= m1) break;
           const float d = best[u] - o[u].w;
           if (bs[u] >= 0) closest_dir(gc[bs[u]], o[u], bx, by, bz, bn, bc);
           if (d < mloc) {
@@ -1576,7 +1593,7 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
       const int node = L.link_node[l];
       pull_wrench<MAXN>(K, node >= 0 ? L.anc[node] : 0, F, tq, gn);
     }
-    dmin = group8_min(mloc);
+    dmin = lanes_min<GROUP>(mloc);
     if (!(dmin < INFINITY)) {  // empty group
       dk = INFINITY;
       return;
@@ -1586,11 +1603,11 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
 #pragma unroll
     for (int a = 0; a < MAXN; ++a) gn[a] *= r;
   }
-  z = group_sum(z);
+  z = lanes_sum<GROUP>(z);
   dk = dmin - tau * __logf(z);
   const float inv = 1.f / z;
 #pragma unroll
-  for (int a = 0; a < MAXN; ++a) gn[a] = group_sum(gn[a]) * inv;
+  for (int a = 0; a < MAXN; ++a) gn[a] = lanes_sum<GROUP>(gn[a]) * inv;
 }
 
 struct ScoLinArgs {
@@ -1604,25 +1621,32 @@ struct ScoLinArgs {
   float tau;
   float* out_d;  // (W, G)
   float* out_J;  // (W, G, A)
+  int lds_len;   // trajectory length of the LDS layout
 };
 
-template <int MAXN>
-__global__ __launch_bounds__(kMaxTrajThreads) void traj_sco_linearize_kernel(ScoLinArgs a) {
+// GROUP lanes share a waypoint.  Eight (one workgroup a trajectory) put the least
+// work into a waypoint, which counts once the chip is full; with few waypoints they
+// leave it idle (96 paths of 24 to 64 waypoints: 528 waves on 96 of 256 CUs), and a
+// whole wave takes each, workgroups along y sharing a trajectory's waypoints: 536 -> 179
+// us a launch among 512 spheres (four of them in a solve of 3435 -> 1867 us).
+template <int MAXN, int GROUP>
+__global__ __launch_bounds__(GROUP == kWave ? kScoWaveThreads : kMaxTrajThreads) void traj_sco_linearize_kernel(ScoLinArgs a) {
   extern __shared__ float4 smem4[];
-  const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4));
   const int b = blockIdx.x;
   if (b >= a.n_traj) return;  // uniform per block
   const long long w0 = a.start[b], w1 = a.start[b + 1];
   if (w0 < 0 || w1 < w0 || w1 > a.n_waypoints || w1 - w0 > a.max_len) return;  // uniform per block
   const int T = static_cast<int>(w1 - w0);
+  const int n_groups = blockDim.x / GROUP;
+  const int rounds = (T + n_groups - 1) / n_groups;
+  if (static_cast<int>(blockIdx.y) >= rounds) return;  // uniform per block
+  const TrajLds L = stage_traj_model(a.md, a.lds_len, reinterpret_cast<char*>(smem4));
   const int A = a.md.n_act;
   const int G = 1 + a.n_wg;
-  const int grp = threadIdx.x / kGroup;
-  const int g = threadIdx.x % kGroup;
+  const int grp = threadIdx.x / GROUP;
+  const int g = threadIdx.x % GROUP;
   float4* gc = L.gc + grp * (a.md.n_spheres + a.md.n_links);
-  const int n_groups = blockDim.x / kGroup;
-  const int rounds = (T + n_groups - 1) / n_groups;
-  for (int rd = 0; rd < rounds; ++rd) {
+  for (int rd = blockIdx.y; rd < rounds; rd += gridDim.y) {
     const int t = rd * n_groups + grp;
     const bool active = t < T;
     WaypointNodes<MAXN, true> K;
@@ -1631,13 +1655,13 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_sco_linearize_kernel(Sco
 #pragma unroll
       for (int c = 0; c < MAXN; ++c) q[c] = (c < A) ? a.x[(w0 + t) * A + c] : 0.f;
       waypoint_fk<MAXN, true>(a.md, L, q, K);
-      waypoint_centres<MAXN, true>(a.md, L, K, gc);
+      waypoint_centres<MAXN, true, GROUP>(a.md, L, K, gc);
     }
     __syncthreads();
     if (active) {
       for (int gi = 0; gi < G; ++gi) {
         float dk, gn[MAXN], gq[MAXN];
-        group_smooth_min<MAXN>(a.md, L, K, gc, a.gstart, gi, a.tau, dk, gn);
+        group_smooth_min<MAXN, GROUP>(a.md, L, K, gc, a.gstart, gi, a.tau, dk, gn);
         if (!(dk < INFINITY)) {
 #pragma unroll
           for (int c = 0; c < MAXN; ++c) gq[c] = 0.f;
@@ -1648,7 +1672,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_sco_linearize_kernel(Sco
         if (g == 0) a.out_d[row] = dk;
 #pragma unroll
         for (int c = 0; c < MAXN; ++c)
-          if (c < A && c % kGroup == g) a.out_J[row * A + c] = gq[c];
+          if (c < A && c % GROUP == g) a.out_J[row * A + c] = gq[c];
       }
     }
     __syncthreads();
@@ -2152,6 +2176,7 @@ extern "C" int pk_traj_sco_linearize_f32(void* stream, const pk_traj_model* mode
   a.start = reinterpret_cast<const long long*>(traj_start);
   a.n_traj = n_traj;
   a.max_len = max_len;
+  a.lds_len = max_len;
   a.n_waypoints = n_waypoints;
   a.gstart = world_group_start;
   a.n_wg = n_world_groups;
@@ -2159,10 +2184,24 @@ extern "C" int pk_traj_sco_linearize_f32(void* stream, const pk_traj_model* mode
   a.out_d = out_d;
   a.out_J = out_J;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (pk::sco_wave_per_waypoint(n_waypoints, d.n_world)) {
+    constexpr int kWaves = pk::kScoWaveThreads / pk::kWave;
+    a.lds_len = 1;  // no trajectory vectors in the LDS
+    const pk::TrajLdsLayout lay = traj_lds(d, 1, pk::kScoWaveThreads, false);
+    const size_t wave_lds = lay.gc + sizeof(float4) * kWaves * static_cast<size_t>(d.n_spheres + d.n_links);
+    const long long len = std::min<long long>(n_waypoints, max_len);  // of a trajectory, at most
+    const dim3 grid(n_traj, static_cast<unsigned>(std::max(1LL, (len + kWaves - 1) / kWaves)));
+    if (maxn == 8)
+      hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<8, pk::kWave>), grid, dim3(pk::kScoWaveThreads), wave_lds, s, a);
+    else
+      hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<16, pk::kWave>), grid, dim3(pk::kScoWaveThreads), wave_lds, s,
+                         a);
+    return pk::check_launch("traj_sco_linearize_kernel");
+  }
   if (maxn == 8)
-    hipLaunchKernelGGL(pk::traj_sco_linearize_kernel<8>, dim3(n_traj), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<8, pk::kGroup>), dim3(n_traj), dim3(threads), lds, s, a);
   else
-    hipLaunchKernelGGL(pk::traj_sco_linearize_kernel<16>, dim3(n_traj), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<16, pk::kGroup>), dim3(n_traj), dim3(threads), lds, s, a);
   return pk::check_launch("traj_sco_linearize_kernel");
 }
 
