@@ -1002,11 +1002,20 @@ struct CostArgs {
   float w_coll;
   float* out_comps;   // (B, 3)
   float* out_grad;    // (W, A) or null
-  bool hulls;         // wave_world_coll's buffers fit the LDS
+  bool hulls;         // use_hulls, and wave_world_coll's buffers fit the LDS
 };
 
 // Waypoints from which the cost kernel takes the world term by wave_world_coll.
 constexpr int kHullWaypoints = 24;
+
+// A wave tests every obstacle against every link, where the grid looks up every
+// sphere and few obstacles leave its cells nearly empty.  150 paths of 48 waypoints,
+// cost and gradient, grid / hulls, us: Panda (59 spheres on 13 links) 88 / 88 among
+// 32 obstacles, 137 / 96 among 128, 357 / 192 among 1024; UR5 (40 spheres, 17 links
+// with any) 145 / 158 among 128, 275 / 308 among 1024.
+inline bool use_hulls(const TrajModelDev& md) {
+  return md.n_world >= 128 && md.n_spheres >= 4 * md.n_links;
+}
 
 template <int MAXN>
 __global__ __launch_bounds__(kMaxTrajThreads) void traj_cost_kernel(CostArgs a) {
@@ -2016,7 +2025,7 @@ extern "C" int pk_traj_cost_grad_f32(void* stream, const pk_traj_model* model, c
   if (blocks == 0) return PK_OK;
   const pk::TrajLdsLayout lay = traj_lds(d, max_len, threads, true);
   PK_REQUIRE(lay.tables <= 150 * 1024, "trajectory model needs %zu bytes of LDS (limit 150 KiB)", lay.tables);
-  const bool hulls = lay.total <= 160 * 1024;  // a CU's LDS
+  const bool hulls = lay.total <= 160 * 1024 && pk::use_hulls(d);  // a CU's LDS
   const size_t lds = hulls ? lay.total : traj_lds_bytes(d, max_len, threads);
   pk::CostArgs a{};
   a.md = d;

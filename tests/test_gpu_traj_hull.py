@@ -1,7 +1,8 @@
-"""The trajectory cost's shared world search (paths of 24 waypoints and more) against the
+"""The trajectory cost's shared world search (paths of 24 waypoints and more,
+128 obstacles and more, four spheres a link and more: the rest keeps the grid) against the
 same waypoints evaluated as short paths, which look every sphere up in the grid: path lengths
 around the threshold, a wave's eight waypoints and a workgroup's rounds, world sizes around
-a pass of 64 obstacles, and obstacles crowded round the robot so that the lists overflow."""
+the threshold and a pass of 64 obstacles, and obstacles crowded round the robot so that the lists overflow."""
 
 import numpy as np
 import pytest
@@ -16,6 +17,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("name,T,M,extent,mode", [
     ("panda", 24, 1, 1.0, 1), ("panda", 25, 63, 1.0, 0), ("ur5", 33, 64, 1.0, 1), ("fetch", 65, 65, 1.0, 1),
+    ("panda", 24, 128, 1.0, 1), ("panda", 33, 129, 1.0, 0), ("panda", 65, 193, 0.5, 1),
     ("panda", 130, 300, 1.0, 0), ("panda", 40, 700, 0.4, 1), ("baxter", 31, 200, 0.6, 1), ("panda", 47, 0, 1.0, 1)])
 def test_long_path_equals_its_pieces(name, T, M, extent, mode):
     """Collision terms only.  Both sides add the same FP32 terms in another order: 1e-5 of the
