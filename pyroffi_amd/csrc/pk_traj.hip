@@ -1002,7 +1002,6 @@ struct CostArgs {
   float w_coll;
   float* out_comps;   // (B, 3)
   float* out_grad;    // (W, A) or null
-  bool hulls;         // use_hulls, and wave_world_coll's buffers fit the LDS
 };
 
 // Waypoints from which the cost kernel takes the world term by wave_world_coll.
@@ -1017,10 +1016,11 @@ inline bool use_hulls(const TrajModelDev& md) {
   return md.n_world >= 128 && md.n_spheres >= 4 * md.n_links;
 }
 
-template <int MAXN>
+// HULLS: launched with use_hulls (a kernel of its own, so that the other keeps its registers).
+template <int MAXN, bool HULLS>
 __global__ __launch_bounds__(kMaxTrajThreads) void traj_cost_kernel(CostArgs a) {
   extern __shared__ float4 smem4[];
-  const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4), a.hulls);
+  const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4), HULLS);
   const int b = a.subset ? a.subset[blockIdx.x] : static_cast<int>(blockIdx.x);
   if (b < 0 || b >= a.n_traj) return;  // uniform per block
   const long long w0 = a.start[b], w1 = a.start[b + 1];
@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_cost_kernel(CostArgs a) 
   // Neighbouring waypoints of a short path are too far apart to share a search
   // (1024 obstacles, 150 paths, cost and gradient, grid against hulls: 8
   // waypoints 161 / 261 us, 32: 307 / 230, 128: 293 / 181).
-  if (a.hulls && T >= kHullWaypoints) {
+  if (HULLS && T >= kHullWaypoints) {
     if (a.out_grad != nullptr)
       traj_value_grad<MAXN, true, true>(a.md, L, L.vx, T, a.w, a.w_coll, false, comps);
     else
@@ -2029,7 +2029,6 @@ extern "C" int pk_traj_cost_grad_f32(void* stream, const pk_traj_model* model, c
   const size_t lds = hulls ? lay.total : traj_lds_bytes(d, max_len, threads);
   pk::CostArgs a{};
   a.md = d;
-  a.hulls = hulls;
   a.x = x;
   a.start = reinterpret_cast<const long long*>(traj_start);
   a.subset = traj_subset;
@@ -2041,10 +2040,14 @@ extern "C" int pk_traj_cost_grad_f32(void* stream, const pk_traj_model* model, c
   a.out_comps = out_comps;
   a.out_grad = out_grad;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (maxn == 8)
-    hipLaunchKernelGGL(pk::traj_cost_kernel<8>, dim3(blocks), dim3(threads), lds, s, a);
+  if (maxn == 8 && hulls)
+    hipLaunchKernelGGL((pk::traj_cost_kernel<8, true>), dim3(blocks), dim3(threads), lds, s, a);
+  else if (maxn == 8)
+    hipLaunchKernelGGL((pk::traj_cost_kernel<8, false>), dim3(blocks), dim3(threads), lds, s, a);
+  else if (hulls)
+    hipLaunchKernelGGL((pk::traj_cost_kernel<16, true>), dim3(blocks), dim3(threads), lds, s, a);
   else
-    hipLaunchKernelGGL(pk::traj_cost_kernel<16>, dim3(blocks), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_cost_kernel<16, false>), dim3(blocks), dim3(threads), lds, s, a);
   return pk::check_launch("traj_cost_kernel");
 }
 
