@@ -52,6 +52,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace pk {
 
@@ -1429,25 +1430,19 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_chomp_kernel(ChompArgs a
 constexpr int kMaxScoGroups = 8;
 constexpr int kScoWaveThreads = 256;  // of the whole-wave linearisation
 
-// Whether the linearisation gives each waypoint a whole wave.  Panda, eight lanes /
-// a wave, us: 6144 waypoints among 512 spheres 536 / 179, among 32 150 / 100; 8192,
-// 548 / 228 and 153 / 132; 16384, 624 / 430 and 174 / 250; 32768, 649 / 820.  A wave
-// repeats the waypoint's kinematics in every lane, which few obstacles do not repay.
+// Whether the linearisation gives each waypoint a whole wave (same bits).  Panda,
+// eight lanes / a wave, us: 4224 waypoints among 512 spheres 544 / 241, among 32
+// 152 / 101; 8192 among 512 545 / 385, 256 319 / 243, 96 187 / 173, 32 156 / 159; past
+// that eight lanes have more than a wave a SIMD to hide latency with and a wave does
+// their sums eight times over: 12000 among 512 598 / 567, 256 341 / 357, 16000 639 / 705.
 inline bool sco_wave_per_waypoint(long long n_waypoints, int n_world) {
-  return n_waypoints <= (n_world >= 256 ? 16384 : 8192);
+  return n_waypoints <= (n_world >= 256 ? 10240 : 8192);
 }
 
-template <int GROUP>
-__device__ __forceinline__ float lanes_min(float v) {
-#pragma unroll
-  for (int off = 1; off < GROUP; off <<= 1) v = fminf(v, __shfl_xor(v, off, kWave));
-  return v;
-}
-
-template <int GROUP>
-__device__ __forceinline__ float lanes_sum(float v) {
-  static_assert(GROUP == kGroup || GROUP == kWave, "no reduction for this group");
-  return GROUP == kWave ? traj_wave_sum(v) : group_sum(v);
+__device__ __forceinline__ float group8_min(float v) {
+  v = fminf(v, __shfl_xor(v, 1, kWave));
+  v = fminf(v, __shfl_xor(v, 2, kWave));
+  return fminf(v, __shfl_xor(v, 4, kWave));
 }
 
 template <int MAXN>
@@ -1470,10 +1465,11 @@ __device__ __forceinline__ void pull_wrench(const WaypointNodes<MAXN, true>& K, 
 // shifted by e = 1e-6 per component (the world sphere's radius is subtracted
 // once the closest robot sphere is known).  The hardware square root (at most
 // 1 ulp) instead of the correctly rounded one: this runs for every (link
-// sphere, world sphere) pair of every waypoint.
+// sphere, world sphere) pair of every waypoint.  Roundings are spelled out here
+// and in sco_moment, so that every kernel that takes a pair gets the same bits.
 __device__ __forceinline__ float sphere_world_dist(const float4& c, const float4& oe) {
   const float dx = oe.x - c.x, dy = oe.y - c.y, dz = oe.z - c.z;
-  return __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz) - c.w;  // v_sqrt_f32, <= 1 ulp
+  return __builtin_amdgcn_sqrtf(fmaf(dz, dz, fmaf(dx, dx, dy * dy))) - c.w;  // v_sqrt_f32, <= 1 ulp
 }
 
 // Direction o_e - c from sphere c to the shifted obstacle centre, its length
@@ -1481,8 +1477,17 @@ __device__ __forceinline__ float sphere_world_dist(const float4& c, const float4
 __device__ __forceinline__ void closest_dir(const float4& c, const float4& oe, float& bx, float& by, float& bz,
                                             float& bn, float4& bc) {
   bx = oe.x - c.x; by = oe.y - c.y; bz = oe.z - c.z;
-  bn = __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz);
+  bn = __builtin_amdgcn_sqrtf(fmaf(bz, bz, fmaf(bx, bx, by * by)));
   bc = c;
+}
+
+// Moment c x (k b) of the distance gradient k b at sphere centre c.
+__device__ __forceinline__ void sco_moment(const float4& c, float k, float bx, float by, float bz, float& tx, float& ty,
+                                           float& tz) {
+  const float gx = k * bx, gy = k * by, gz = k * bz;
+  tx = fmaf(c.y, gz, -(c.z * gy));
+  ty = fmaf(c.z, gx, -(c.x * gz));
+  tz = fmaf(c.x, gy, -(c.y * gx));
 }
 
 // Closest same-slot pair of active pair p: distance, direction cj - ci + e, its length, the centres.
@@ -1501,12 +1506,12 @@ __device__ __forceinline__ float pair_dist(const TrajLds& L, const float4* gc, i
   return best;
 }
 
-template <int MAXN, int GROUP>
+template <int MAXN>
 __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const TrajLds& L,
                                                  const WaypointNodes<MAXN, true>& K, const float4* gc,
                                                  const int* gstart, int gi, float tau, float& dk,
                                                  float (&gn)[MAXN]) {
-  const int g = threadIdx.x % GROUP;
+  const int g = threadIdx.x % kGroup;
 #pragma unroll
   for (int a = 0; a < MAXN; ++a) gn[a] = 0.f;
   float bx, by, bz, bn;
@@ -1515,13 +1520,13 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
   if (gi == 0) {
     // Self pairs (a few dozen): pass 1 the group minimum, pass 2 the weights.
     dmin = INFINITY;
-    for (int p = g; p < md.n_pairs; p += GROUP) dmin = fminf(dmin, pair_dist(L, gc, p, bx, by, bz, bn, bc, bc2));
-    dmin = lanes_min<GROUP>(dmin);
+    for (int p = g; p < md.n_pairs; p += kGroup) dmin = fminf(dmin, pair_dist(L, gc, p, bx, by, bz, bn, bc, bc2));
+    dmin = group8_min(dmin);
     if (!(dmin < INFINITY)) {  // empty group
       dk = INFINITY;
       return;
     }
-    for (int p = g; p < md.n_pairs; p += GROUP) {
+    for (int p = g; p < md.n_pairs; p += kGroup) {
       const float d = pair_dist(L, gc, p, bx, by, bz, bn, bc, bc2);
       const float w = __expf(-(d - dmin) / tau);
       if (!(w > 0.f)) continue;
@@ -1551,15 +1556,14 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
       // obstacle order, the order of one obstacle at a time.  Sixteen per pass
       // measured 3% faster than eight and 27% faster than four (112 VGPRs,
       // no spills).
-      // A whole wave has at most a few obstacles a lane: four.
-      constexpr int kObs = GROUP == kWave ? 4 : 16;
-      for (int mb = m0 + g; mb < m1; mb += GROUP * kObs) {
+      constexpr int kObs = 16;
+      for (int mb = m0 + g; mb < m1; mb += kGroup * kObs) {
         float4 o[kObs];
         float best[kObs];
         int bs[kObs];
 #pragma unroll
         for (int u = 0; u < kObs; ++u) {
-          const int m = mb + u * GROUP;
+          const int m = mb + u * kGroup;
           const float4 w = L.world[m < m1 ? m : mb];
           o[u] = make_float4(w.x + 1e-6f, w.y + 1e-6f, w.z + 1e-6f, w.w);  // centre + e
           best[u] = INFINITY;
@@ -1575,7 +1579,7 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
         }
 #pragma unroll
         for (int u = 0; u < kObs; ++u) {
-          if (mb + u * GROUP >= m1) break;
+          if (mb + u * kGroup >= m1) break;
           const float d = best[u] - o[u].w;
           if (bs[u] >= 0) closest_dir(gc[bs[u]], o[u], bx, by, bz, bn, bc);
           if (d < mloc) {
@@ -1591,18 +1595,17 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
           if (w > 0.f) {
             z += w;
             const float k = -w * __builtin_amdgcn_rcpf(bn);  // d(distance)/dc = -(o - c + e) / |o - c + e|
-            const float gx = k * bx, gy = k * by, gz = k * bz;
-            F[0] += gx; F[1] += gy; F[2] += gz;
-            tq[0] += bc.y * gz - bc.z * gy;
-            tq[1] += bc.z * gx - bc.x * gz;
-            tq[2] += bc.x * gy - bc.y * gx;
+            float tx, ty, tz;
+            sco_moment(bc, k, bx, by, bz, tx, ty, tz);
+            F[0] = fmaf(bx, k, F[0]); F[1] = fmaf(by, k, F[1]); F[2] = fmaf(bz, k, F[2]);
+            tq[0] += tx; tq[1] += ty; tq[2] += tz;
           }
         }
       }
       const int node = L.link_node[l];
       pull_wrench<MAXN>(K, node >= 0 ? L.anc[node] : 0, F, tq, gn);
     }
-    dmin = lanes_min<GROUP>(mloc);
+    dmin = group8_min(mloc);
     if (!(dmin < INFINITY)) {  // empty group
       dk = INFINITY;
       return;
@@ -1612,12 +1615,294 @@ __device__ __forceinline__ void group_smooth_min(const TrajModelDev& md, const T
 #pragma unroll
     for (int a = 0; a < MAXN; ++a) gn[a] *= r;
   }
-  z = lanes_sum<GROUP>(z);
+  z = group_sum(z);
   dk = dmin - tau * __logf(z);
   const float inv = 1.f / z;
 #pragma unroll
-  for (int a = 0; a < MAXN; ++a) gn[a] = lanes_sum<GROUP>(gn[a]) * inv;
+  for (int a = 0; a < MAXN; ++a) gn[a] = group_sum(gn[a]) * inv;
 }
+
+// a * b, not to be fused into a sum that follows.
+__device__ __forceinline__ float mul_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+// Node a's pose translation and world twist, of the nodes a lane serves.
+struct NodeTwist {
+  float px, py, pz, wx, wy, wz, vx, vy, vz;
+};
+
+// One waypoint's groups by a whole wave, to the bit what its eight lanes get from
+// group_smooth_min, so that a path's result does not depend on how many others
+// share its launch.  What costs time and has no order (distances, the exact minima,
+// weights and directions) takes 64 pairs or obstacles at once.  The sums, whose
+// order counts, are eight per quantity (lane g of eight has items g, g + 8, ... in
+// order), and there are eight quantities (force, moment, weight) and nodes to a
+// register: lane g + 8 s keeps quantity s and the gradients of nodes s, s + 8.
+template <int MAXN>
+struct ScoWave {
+  static constexpr int kNodes = MAXN / kGroup;
+  static constexpr int kObs = 4;                       // obstacles of a lane that share each sphere read
+  static constexpr int kItems = 2;                     // of them whose terms are in the LDS at a time
+  static constexpr int kRow = kItems * kWave + kGroup;  // words from quantity to quantity: no bank twice
+  static constexpr int kPairWords = 12;
+  static constexpr int kWords = kRow * kGroup + 2 * kItems * kWave;  // LDS of a wave
+  static_assert(kPairWords * kWave <= kWords && MAXN <= kWords, "pairs and gradients fit the obstacles' place");
+
+  const TrajModelDev& md;
+  const TrajLds& L;
+  const float4* gc;
+  float* buf;
+  NodeTwist node[kNodes];
+  float gn[kNodes];
+  int lane, g, s;
+
+  __device__ __forceinline__ ScoWave(const TrajModelDev& m, const TrajLds& lds, const WaypointNodes<MAXN, true>& K,
+                                     const float4* centres, float* words)
+      : md(m), L(lds), gc(centres), buf(words) {
+    lane = threadIdx.x % kWave;
+    g = lane % kGroup;
+    s = lane / kGroup;
+#pragma unroll
+    for (int a = 0; a < MAXN; ++a)
+      if (a % kGroup == s)
+        node[a / kGroup] = {K.P[a].tx, K.P[a].ty, K.P[a].tz, K.w[a][0], K.w[a][1], K.w[a][2],
+                            K.v[a][0], K.v[a][1], K.v[a][2]};
+  }
+
+  // pull_point and pull_wrench for this lane's nodes, roundings as the compiler places them there.
+  __device__ __forceinline__ void point(int mask, float cx, float cy, float cz, float gx, float gy, float gz) {
+#pragma unroll
+    for (int i = 0; i < kNodes; ++i) {
+      if (mask & (1 << (s + kGroup * i))) {
+        const NodeTwist& n = node[i];
+        const float rx = cx - n.px, ry = cy - n.py, rz = cz - n.pz;
+        const float dx = fmaf(n.wy, rz, -(n.wz * ry)) + n.vx;
+        const float dy = fmaf(n.wz, rx, -(n.wx * rz)) + n.vy;
+        const float dz = fmaf(n.wx, ry, -(n.wy * rx)) + n.vz;
+        gn[i] += fmaf(gz, dz, fmaf(gx, dx, gy * dy));
+      }
+    }
+  }
+  __device__ __forceinline__ void wrench(int mask, const float (&F)[3], const float (&tq)[3]) {
+#pragma unroll
+    for (int i = 0; i < kNodes; ++i) {
+      if (mask & (1 << (s + kGroup * i))) {
+        const NodeTwist& n = node[i];
+        const float mx = tq[0] - fmaf(n.py, F[2], -(n.pz * F[1]));
+        const float my = tq[1] - fmaf(n.pz, F[0], -(n.px * F[2]));
+        const float mz = tq[2] - fmaf(n.px, F[1], -(n.py * F[0]));
+        gn[i] += fmaf(n.wz, mz, fmaf(n.wy, my, fmaf(n.wx, mx, fmaf(n.vz, F[2], fmaf(n.vx, F[0], n.vy * F[1])))));
+      }
+    }
+  }
+
+  // Every node's gradient, the lanes' sums over 1 / z, in every lane.
+  __device__ __forceinline__ void gather(float inv, float (&all)[MAXN]) {
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < kNodes; ++i) {
+      const float v = group_sum(gn[i]) * inv;
+      if (g == 0) buf[s + kGroup * i] = v;
+    }
+    wave_sync();
+#pragma unroll
+    for (int a = 0; a < MAXN; ++a) all[a] = buf[a];
+    wave_sync();
+  }
+
+  // Self pairs.  Sums run over entries of 64 pairs.
+  __device__ __forceinline__ void self_group(float tau, float& dk, float (&all)[MAXN]) {
+    float bx, by, bz, bn;
+    float4 ci, cj;
+#pragma unroll
+    for (int i = 0; i < kNodes; ++i) gn[i] = 0.f;
+    float dmin = INFINITY;
+    for (int p = lane; p < md.n_pairs; p += kWave) dmin = fminf(dmin, pair_dist(L, gc, p, bx, by, bz, bn, ci, cj));
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) dmin = fminf(dmin, __shfl_xor(dmin, off, kWave));
+    if (!(dmin < INFINITY)) {
+      dk = INFINITY;
+      return;
+    }
+    float z = 0.f;
+    for (int p0 = 0; p0 < md.n_pairs; p0 += kWave) {
+      const int n = min(md.n_pairs - p0, kWave);
+      if (lane < n) {
+        const int p = p0 + lane;
+        const float d = pair_dist(L, gc, p, bx, by, bz, bn, ci, cj);
+        const float w = __expf(-(d - dmin) / tau);
+        const bool counts = w > 0.f;
+        const float k = w / bn;
+        const int ni = L.link_node[L.pair_links[2 * p]], nj = L.link_node[L.pair_links[2 * p + 1]];
+        const int masks = (ni >= 0 ? L.anc[ni] : 0) | ((nj >= 0 ? L.anc[nj] : 0) << 16);
+        const float e[kPairWords] = {counts ? w : 0.f, __int_as_float(masks), k * bx, k * by, k * bz, ci.x,
+                                     ci.y, ci.z, cj.x, cj.y, cj.z, 0.f};
+#pragma unroll
+        for (int c = 0; c < kPairWords - 1; ++c) buf[c * kWave + lane] = e[c];
+      }
+      wave_sync();
+      for (int j = g; j < n; j += kGroup) {
+        const float* e = buf + j;
+        const float w = e[0];
+        if (!(w > 0.f)) continue;
+        z += w;
+        const int masks = __float_as_int(e[kWave]);
+        const float gx = e[2 * kWave], gy = e[3 * kWave], gz = e[4 * kWave];
+        point(static_cast<int>(static_cast<unsigned>(masks) >> 16), e[8 * kWave], e[9 * kWave], e[10 * kWave], gx, gy, gz);
+        point(masks & 0xffff, e[5 * kWave], e[6 * kWave], e[7 * kWave], -gx, -gy, -gz);
+      }
+      wave_sync();
+    }
+    z = group_sum(z);
+    dk = dmin - tau * __logf(z);
+    gather(1.f / z, all);
+  }
+
+  // World group of obstacles [m0, m1).  Of each 128, lane g + 8 s has items
+  // per * s + v of lane g of eight: obstacles mb + 8 (per * s + v) + g.
+  __device__ __forceinline__ void world_group(int m0, int m1, float tau, float& dk, float (&all)[MAXN]) {
+    float* x = buf;                          // [quantity][v][lane]: direction, moment, weight, 0
+    float* factor = buf + kRow * kGroup;     // of the direction: -w / |o - c + e|
+    float* scale = factor + kItems * kWave;  // of the sums before the term: the running minimum drops here
+    const float inv_tau = 1.f / tau;
+#pragma unroll
+    for (int i = 0; i < kNodes; ++i) gn[i] = 0.f;
+    float z = 0.f, mloc = INFINITY;
+    // A NaN never lowers the minimum.
+    auto lower = [](float before, float v) { return v < before ? v : before; };
+    for (int l = 0; l < md.n_links; ++l) {
+      const int k0 = L.link_sph[l], k1 = L.link_sph[l + 1];
+      if (k0 >= k1) continue;
+      float sum = s == 6 ? z : 0.f;
+      for (int mp = m0; mp < m1; mp += kWave * kObs) {
+        float4 o[kObs];
+        float best[kObs];
+        int bs[kObs];
+        auto per_of = [&](int mb) { return m1 - mb <= kWave ? 1 : kItems; };
+#pragma unroll
+        for (int u = 0; u < kObs; ++u) {
+          const int mb = mp + u / kItems * kItems * kWave;
+          const float4 w = L.world[min(mb + kGroup * (per_of(mb) * s + u % kItems) + g, m1 - 1)];
+          o[u] = make_float4(w.x + 1e-6f, w.y + 1e-6f, w.z + 1e-6f, w.w);
+          best[u] = INFINITY;
+          bs[u] = -1;
+        }
+        auto distances = [&](auto count) {
+          for (int sp = k0; sp < k1; ++sp) {
+            const float4 c = gc[sp];
+#pragma unroll
+            for (int u = 0; u < decltype(count)::value; ++u) {
+              const float d = sphere_world_dist(c, o[u]);
+              if (d < best[u]) { best[u] = d; bs[u] = sp; }
+            }
+          }
+        };
+        if (m1 - mp > kItems * kWave)
+          distances(std::integral_constant<int, kObs>{});
+        else
+          distances(std::integral_constant<int, kItems>{});
+#pragma unroll
+        for (int h = 0; h < kObs / kItems; ++h) {
+          const int mb = mp + h * kItems * kWave;
+          if (mb >= m1) break;
+          const int per = per_of(mb);
+          // Running minimum up to each item: within the lane, then over the lanes of g before it.
+          float upto[kItems], d[kItems];
+          bool in[kItems];
+          float own = INFINITY;
+#pragma unroll
+          for (int v = 0; v < kItems; ++v) {
+            d[v] = best[h * kItems + v] - o[h * kItems + v].w;
+            in[v] = v < per && mb + kGroup * (per * s + v) + g < m1;
+            if (in[v]) own = lower(own, d[v]);
+            upto[v] = own;
+          }
+          float through = own;
+#pragma unroll
+          for (int off = kGroup; off < kWave; off <<= 1) {
+            const float t = __shfl_up(through, off, kWave);
+            if (lane >= off) through = lower(t, through);
+          }
+          through = lower(mloc, through);
+          float before = __shfl_up(through, kGroup, kWave);
+          if (lane < kGroup) before = mloc;
+          mloc = __shfl(through, kWave - kGroup + g, kWave);
+          unsigned long long drops_at[kItems];
+#pragma unroll
+          for (int v = 0; v < kItems; ++v) {
+            const int u = h * kItems + v;
+            const float excl = v == 0 ? before : lower(before, upto[v > 0 ? v - 1 : 0]);
+            const bool drops = in[v] && d[v] < excl;
+            const float w = __expf((lower(before, upto[v]) - d[v]) * inv_tau);
+            float bx = 0.f, by = 0.f, bz = 0.f, k = -0.f, tx = -0.f, ty = -0.f, tz = -0.f, tw = -0.f;  // adds nothing
+            if (in[v] && bs[u] >= 0 && w > 0.f) {
+              float4 c;
+              float bn;
+              closest_dir(gc[bs[u]], o[u], bx, by, bz, bn, c);
+              asm("" : "+v"(bn));  // the reciprocal of the rounded root, not one v_rsq_f32
+              k = -w * __builtin_amdgcn_rcpf(bn);
+              sco_moment(c, k, bx, by, bz, tx, ty, tz);
+              tw = w;
+            }
+            const float t[kGroup] = {bx, by, bz, tx, ty, tz, tw, -0.f};
+#pragma unroll
+            for (int c = 0; c < kGroup; ++c) x[c * kRow + v * kWave + lane] = t[c];
+            factor[v * kWave + lane] = k;
+            drops_at[v] = __ballot(drops);
+            if (drops_at[v])
+              scale[v * kWave + lane] = drops ? (excl < INFINITY ? __expf((d[v] - excl) * inv_tau) : 0.f) : 1.f;
+          }
+          wave_sync();
+          const float* xs = x + s * kRow + g;
+#pragma unroll
+          for (int j = 0; j < kGroup; ++j) {
+            if (mb + kGroup * per * j >= m1) break;
+            float xv[kItems], fv[kItems];
+#pragma unroll
+            for (int v = 0; v < kItems; ++v) {
+              xv[v] = xs[v * kWave + j * kGroup];
+              fv[v] = factor[v * kWave + j * kGroup + g];
+            }
+#pragma unroll
+            for (int v = 0; v < kItems; ++v) {
+              if (v >= per) break;
+              if ((drops_at[v] >> (j * kGroup)) & 0xffull) {
+                const float r = scale[v * kWave + j * kGroup + g];
+                sum = mul_rounded(sum, r);
+#pragma unroll
+                for (int i = 0; i < kNodes; ++i) gn[i] = mul_rounded(gn[i], r);
+              }
+              sum = fmaf(xv[v], s < 3 ? fv[v] : 1.f, sum);
+            }
+          }
+          wave_sync();
+        }
+      }
+      z = sum;  // of quantity 6
+      float F[3], tq[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        F[c] = __shfl(sum, c * kGroup + g, kWave);
+        tq[c] = __shfl(sum, (3 + c) * kGroup + g, kWave);
+      }
+      const int node_of = L.link_node[l];
+      wrench(node_of >= 0 ? L.anc[node_of] : 0, F, tq);
+    }
+    const float dmin = group8_min(mloc);
+    if (!(dmin < INFINITY)) {  // empty group
+      dk = INFINITY;
+      return;
+    }
+    const float r = (mloc < INFINITY) ? __expf(-(mloc - dmin) / tau) : 0.f;
+    z = __shfl(group_sum(mul_rounded(z, r)), 6 * kGroup, kWave);
+    dk = dmin - tau * __logf(z);
+#pragma unroll
+    for (int i = 0; i < kNodes; ++i) gn[i] = mul_rounded(gn[i], r);
+    gather(1.f / z, all);
+  }
+};
 
 struct ScoLinArgs {
   TrajModelDev md;
@@ -1630,32 +1915,26 @@ struct ScoLinArgs {
   float tau;
   float* out_d;  // (W, G)
   float* out_J;  // (W, G, A)
-  int lds_len;   // trajectory length of the LDS layout
 };
 
-// GROUP lanes share a waypoint.  Eight (one workgroup a trajectory) put the least
-// work into a waypoint, which counts once the chip is full; with few waypoints they
-// leave it idle (96 paths of 24 to 64 waypoints: 528 waves on 96 of 256 CUs), and a
-// whole wave takes each, workgroups along y sharing a trajectory's waypoints: 536 -> 179
-// us a launch among 512 spheres (four of them in a solve of 3435 -> 1867 us).
-template <int MAXN, int GROUP>
-__global__ __launch_bounds__(GROUP == kWave ? kScoWaveThreads : kMaxTrajThreads) void traj_sco_linearize_kernel(ScoLinArgs a) {
+// Eight lanes share a waypoint, one workgroup a trajectory.
+template <int MAXN>
+__global__ __launch_bounds__(kMaxTrajThreads) void traj_sco_linearize_kernel(ScoLinArgs a) {
   extern __shared__ float4 smem4[];
+  const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4));
   const int b = blockIdx.x;
   if (b >= a.n_traj) return;  // uniform per block
   const long long w0 = a.start[b], w1 = a.start[b + 1];
   if (w0 < 0 || w1 < w0 || w1 > a.n_waypoints || w1 - w0 > a.max_len) return;  // uniform per block
   const int T = static_cast<int>(w1 - w0);
-  const int n_groups = blockDim.x / GROUP;
-  const int rounds = (T + n_groups - 1) / n_groups;
-  if (static_cast<int>(blockIdx.y) >= rounds) return;  // uniform per block
-  const TrajLds L = stage_traj_model(a.md, a.lds_len, reinterpret_cast<char*>(smem4));
   const int A = a.md.n_act;
   const int G = 1 + a.n_wg;
-  const int grp = threadIdx.x / GROUP;
-  const int g = threadIdx.x % GROUP;
+  const int grp = threadIdx.x / kGroup;
+  const int g = threadIdx.x % kGroup;
   float4* gc = L.gc + grp * (a.md.n_spheres + a.md.n_links);
-  for (int rd = blockIdx.y; rd < rounds; rd += gridDim.y) {
+  const int n_groups = blockDim.x / kGroup;
+  const int rounds = (T + n_groups - 1) / n_groups;
+  for (int rd = 0; rd < rounds; ++rd) {
     const int t = rd * n_groups + grp;
     const bool active = t < T;
     WaypointNodes<MAXN, true> K;
@@ -1664,13 +1943,13 @@ __global__ __launch_bounds__(GROUP == kWave ? kScoWaveThreads : kMaxTrajThreads)
 #pragma unroll
       for (int c = 0; c < MAXN; ++c) q[c] = (c < A) ? a.x[(w0 + t) * A + c] : 0.f;
       waypoint_fk<MAXN, true>(a.md, L, q, K);
-      waypoint_centres<MAXN, true, GROUP>(a.md, L, K, gc);
+      waypoint_centres<MAXN, true>(a.md, L, K, gc);
     }
     __syncthreads();
     if (active) {
       for (int gi = 0; gi < G; ++gi) {
         float dk, gn[MAXN], gq[MAXN];
-        group_smooth_min<MAXN, GROUP>(a.md, L, K, gc, a.gstart, gi, a.tau, dk, gn);
+        group_smooth_min<MAXN>(a.md, L, K, gc, a.gstart, gi, a.tau, dk, gn);
         if (!(dk < INFINITY)) {
 #pragma unroll
           for (int c = 0; c < MAXN; ++c) gq[c] = 0.f;
@@ -1681,10 +1960,64 @@ __global__ __launch_bounds__(GROUP == kWave ? kScoWaveThreads : kMaxTrajThreads)
         if (g == 0) a.out_d[row] = dk;
 #pragma unroll
         for (int c = 0; c < MAXN; ++c)
-          if (c < A && c % GROUP == g) a.out_J[row * A + c] = gq[c];
+          if (c < A && c % kGroup == g) a.out_J[row * A + c] = gq[c];
       }
     }
     __syncthreads();
+  }
+}
+
+// The same with a wave per waypoint and workgroups along y sharing a trajectory's
+// waypoints: with few waypoints eight lanes each leave the chip idle (96 paths of
+// 24 to 64 waypoints: 528 waves on 96 of 256 CUs; 544 -> 241 us a launch among 512
+// spheres).  What bounds it is the latency of a link's steps (minima over the lanes,
+// the terms through the LDS, the sums in order), so three waves a SIMD are asked for:
+// 168 registers instead of 176, 133 -> 100 us among 32 spheres.
+template <int MAXN>
+__global__ __launch_bounds__(kScoWaveThreads, 3) void traj_sco_linearize_wave_kernel(ScoLinArgs a) {
+  extern __shared__ float4 smem4[];
+  const int b = blockIdx.x;
+  if (b >= a.n_traj) return;  // uniform per block
+  const long long w0 = a.start[b], w1 = a.start[b + 1];
+  if (w0 < 0 || w1 < w0 || w1 > a.n_waypoints || w1 - w0 > a.max_len) return;  // uniform per block
+  const int T = static_cast<int>(w1 - w0);
+  constexpr int n_waves = kScoWaveThreads / kWave;
+  if (static_cast<int>(blockIdx.y) * n_waves >= T) return;  // uniform per block
+  const TrajLds L = stage_traj_model(a.md, 1, reinterpret_cast<char*>(smem4));  // no trajectory vectors
+  const int A = a.md.n_act;
+  const int G = 1 + a.n_wg;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int slot = a.md.n_spheres + a.md.n_links;
+  float4* gc = L.gc + wave * slot;
+  float* words = reinterpret_cast<float*>(L.gc + n_waves * slot) + wave * ScoWave<MAXN>::kWords;
+  for (int t = blockIdx.y * n_waves + wave; t < T; t += gridDim.y * n_waves) {
+    WaypointNodes<MAXN, true> K;
+    float q[MAXN];
+#pragma unroll
+    for (int c = 0; c < MAXN; ++c) q[c] = (c < A) ? a.x[(w0 + t) * A + c] : 0.f;
+    waypoint_fk<MAXN, true>(a.md, L, q, K);
+    waypoint_centres<MAXN, true, kWave>(a.md, L, K, gc);
+    ScoWave<MAXN> sw(a.md, L, K, gc, words);
+    wave_sync();
+    for (int gi = 0; gi < G; ++gi) {
+      float dk, gn[MAXN], gq[MAXN];
+      if (gi == 0)
+        sw.self_group(a.tau, dk, gn);
+      else
+        sw.world_group(a.gstart[gi - 1], a.gstart[gi], a.tau, dk, gn);
+      if (!(dk < INFINITY)) {
+#pragma unroll
+        for (int c = 0; c < MAXN; ++c) gq[c] = 0.f;
+      } else {
+        node_to_actuated<MAXN>(L, a.md.n_nodes, gn, gq);
+      }
+      const long long row = (w0 + t) * G + gi;
+      if (lane == 0) a.out_d[row] = dk;
+#pragma unroll
+      for (int c = 0; c < MAXN; ++c)
+        if (c < A && c == lane) a.out_J[row * A + c] = gq[c];
+    }
+    wave_sync();
   }
 }
 
@@ -2188,7 +2521,6 @@ extern "C" int pk_traj_sco_linearize_f32(void* stream, const pk_traj_model* mode
   a.start = reinterpret_cast<const long long*>(traj_start);
   a.n_traj = n_traj;
   a.max_len = max_len;
-  a.lds_len = max_len;
   a.n_waypoints = n_waypoints;
   a.gstart = world_group_start;
   a.n_wg = n_world_groups;
@@ -2196,24 +2528,25 @@ extern "C" int pk_traj_sco_linearize_f32(void* stream, const pk_traj_model* mode
   a.out_d = out_d;
   a.out_J = out_J;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (pk::sco_wave_per_waypoint(n_waypoints, d.n_world)) {
-    constexpr int kWaves = pk::kScoWaveThreads / pk::kWave;
-    a.lds_len = 1;  // no trajectory vectors in the LDS
-    const pk::TrajLdsLayout lay = traj_lds(d, 1, pk::kScoWaveThreads, false);
-    const size_t wave_lds = lay.gc + sizeof(float4) * kWaves * static_cast<size_t>(d.n_spheres + d.n_links);
+  constexpr int kWaves = pk::kScoWaveThreads / pk::kWave;
+  const size_t wave_lds =
+      traj_lds(d, 1, pk::kScoWaveThreads, false).gc +
+      kWaves * (sizeof(float4) * static_cast<size_t>(d.n_spheres + d.n_links) +
+                sizeof(float) * (maxn == 8 ? pk::ScoWave<8>::kWords : pk::ScoWave<16>::kWords));
+  if (pk::sco_wave_per_waypoint(n_waypoints, d.n_world) && wave_lds <= 160 * 1024) {  // a CU's LDS
     const long long len = std::min<long long>(n_waypoints, max_len);  // of a trajectory, at most
     const dim3 grid(n_traj, static_cast<unsigned>(std::max(1LL, (len + kWaves - 1) / kWaves)));
+    const dim3 block(pk::kScoWaveThreads);
     if (maxn == 8)
-      hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<8, pk::kWave>), grid, dim3(pk::kScoWaveThreads), wave_lds, s, a);
+      hipLaunchKernelGGL(pk::traj_sco_linearize_wave_kernel<8>, grid, block, wave_lds, s, a);
     else
-      hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<16, pk::kWave>), grid, dim3(pk::kScoWaveThreads), wave_lds, s,
-                         a);
-    return pk::check_launch("traj_sco_linearize_kernel");
+      hipLaunchKernelGGL(pk::traj_sco_linearize_wave_kernel<16>, grid, block, wave_lds, s, a);
+    return pk::check_launch("traj_sco_linearize_wave_kernel");
   }
   if (maxn == 8)
-    hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<8, pk::kGroup>), dim3(n_traj), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL(pk::traj_sco_linearize_kernel<8>, dim3(n_traj), dim3(threads), lds, s, a);
   else
-    hipLaunchKernelGGL((pk::traj_sco_linearize_kernel<16, pk::kGroup>), dim3(n_traj), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL(pk::traj_sco_linearize_kernel<16>, dim3(n_traj), dim3(threads), lds, s, a);
   return pk::check_launch("traj_sco_linearize_kernel");
 }
 
