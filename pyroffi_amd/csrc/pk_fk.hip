@@ -528,31 +528,28 @@ static int launch_fk(void* stream, const float* cfg, int64_t batch, int32_t n_ac
 // then the subtree sums and projections of every fourth joint: 28 us.
 constexpr int kVjpWaves = 4;
 
-// One moving joint: its record with the constant joints above folded into ptf.
-struct VjpNode {
-  JointRec r;                  // parent_slot = parent node, joint = slot
-  unsigned long long subtree;  // nodes at or below it
-};
-
-// LDS image; nodes = moving joints the tables may have (J at most).
+// LDS image; nodes = moving joints the tables may have (J at most).  It must not
+// outgrow one lane walking all joints (84 J + 4 * 65 (n_act + 13 J) bytes), which is
+// what a tree whose every joint moves leaves of the LDS: slots and nodes take a byte
+// each, constant chains are kept for constant joints only, and the joint records and
+// the joint -> slot map, which nothing reads once poses and wrenches are written,
+// share their places.
 struct VjpLds {
-  int recs, nodes, rel, anchor, slot_of, lnode, cfg, pose, wrench, total;
+  int nodes, anchor, lnode, cfg, pose, recs, wrench, slot_of, total;
 };
-// The joint records are only needed before the first pose is written and share
-// the poses' place.
 __host__ __device__ inline VjpLds vjp_lds(int J, int L, int n_act, int nodes) {
   VjpLds o;
-  o.nodes = 0;
-  o.rel = o.nodes + static_cast<int>(sizeof(VjpNode)) * nodes;  // constant chain above each slot
-  o.anchor = o.rel + 28 * J;                                // node at or above each slot, -1 none
-  o.slot_of = o.anchor + 4 * J;
-  o.lnode = o.slot_of + 4 * J;                              // node of each link
-  o.cfg = o.lnode + 4 * L;                                  // [a][lane], stride 65
-  o.pose = o.cfg + 4 * n_act * kLaneStride;                 // [node * 7 + c][lane]
+  const int rec = static_cast<int>(sizeof(JointRec));
+  o.nodes = 0;                                        // n moving joints, then J - n constant chains (7 floats), n <= nodes
+  o.anchor = o.nodes + rec * nodes + 28 * (J - nodes);  // node at or above each slot, -1 none
+  o.lnode = o.anchor + J;                             // slot of each link, -1 none
+  o.cfg = (o.lnode + L + 3) / 4 * 4;                  // [a][lane], stride 65
+  o.pose = o.cfg + 4 * n_act * kLaneStride;           // [node * 7 + c][lane]
   o.recs = o.pose;
-  o.wrench = o.pose + 4 * 7 * nodes * kLaneStride;          // [node * 6 + c][lane]
-  const int end = o.wrench + 4 * 6 * nodes * kLaneStride, recs_end = o.recs + static_cast<int>(sizeof(JointRec)) * J;
-  o.total = end > recs_end ? end : recs_end;
+  o.wrench = o.pose + 4 * 7 * nodes * kLaneStride;    // [node * 6 + c][lane]
+  const int recs_end = o.recs + rec * J, end = o.wrench + 4 * 6 * nodes * kLaneStride;
+  o.slot_of = o.wrench > recs_end ? o.wrench : recs_end;
+  o.total = end > o.slot_of + 4 * J ? end : o.slot_of + 4 * J;
   return o;
 }
 
@@ -563,12 +560,13 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
   extern __shared__ char vsmem[];
   const int J = tables.n_joints;
   const VjpLds lay = vjp_lds(J, n_links, n_act, max_nodes);
-  VjpNode* nodes = reinterpret_cast<VjpNode*>(vsmem + lay.nodes);
+  // A moving joint with the constant joints above it folded into ptf (parent_slot =
+  // parent node, joint = slot).
+  JointRec* nodes = reinterpret_cast<JointRec*>(vsmem + lay.nodes);
   JointRec* recs = reinterpret_cast<JointRec*>(vsmem + lay.recs);
-  float* rel = reinterpret_cast<float*>(vsmem + lay.rel);
-  int* anchor = reinterpret_cast<int*>(vsmem + lay.anchor);
   int* slot_of = reinterpret_cast<int*>(vsmem + lay.slot_of);
-  int* lnode = reinterpret_cast<int*>(vsmem + lay.lnode);
+  signed char* anchor = reinterpret_cast<signed char*>(vsmem + lay.anchor);
+  signed char* lnode = reinterpret_cast<signed char*>(vsmem + lay.lnode);
   float* cfg_tile = reinterpret_cast<float*>(vsmem + lay.cfg);
   float* poses = reinterpret_cast<float*>(vsmem + lay.pose);
   float* wrench = reinterpret_cast<float*>(vsmem + lay.wrench);
@@ -582,7 +580,10 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
     const int l = f / n_act, a = f - l * n_act;
     cfg_tile[a * kLaneStride + l] = cfg_blk[f];
   }
-  for (int l = tid; l < n_links; l += kWave * kVjpWaves) lnode[l] = link_parent_joint[l];
+  for (int l = tid; l < n_links; l += kWave * kVjpWaves) {
+    const int pj = link_parent_joint[l];
+    lnode[l] = static_cast<signed char>((pj >= 0 && pj < J) ? pj : -1);
+  }
   stage_joint_records(tables, recs, slot_of);
   // Every wave counts the moving slots for itself (J <= 64: one per lane).
   const bool moving = lane < J && recs[min(lane, J - 1)].kind != 0;
@@ -593,6 +594,8 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
     return;
   }
   auto node_of = [&](int slot) { return __popcll(moves & ((1ull << slot) - 1ull)); };
+  float* rel = reinterpret_cast<float*>(nodes + n_nodes);
+  auto rel_of = [&](int slot) { return rel + 7 * (slot - node_of(slot)); };  // constant slots only
   if (wave == 0 && lane < J) {
     // A parent's slot is below its child's, so the walk up ends.
     Pose T = load_pose(recs[lane].ptf);
@@ -602,26 +605,26 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
       p = recs[p].parent_slot;
     }
     const int par = p >= 0 ? node_of(p) : -1;
-    float* d = rel + 7 * lane;
     if (moving) {
-      VjpNode& n = nodes[node_of(lane)];
-      n.r = recs[lane];
-      n.r.ptf[0] = T.w; n.r.ptf[1] = T.x; n.r.ptf[2] = T.y; n.r.ptf[3] = T.z;
-      n.r.ptf[4] = T.tx; n.r.ptf[5] = T.ty; n.r.ptf[6] = T.tz;
-      n.r.parent_slot = par;
-      n.subtree = 0;
-      T = pose_identity();
+      JointRec& n = nodes[node_of(lane)];
+      n = recs[lane];
+      n.ptf[0] = T.w; n.ptf[1] = T.x; n.ptf[2] = T.y; n.ptf[3] = T.z;
+      n.ptf[4] = T.tx; n.ptf[5] = T.ty; n.ptf[6] = T.tz;
+      n.parent_slot = par;
+    } else {
+      float* d = rel_of(lane);
+      d[0] = T.w; d[1] = T.x; d[2] = T.y; d[3] = T.z; d[4] = T.tx; d[5] = T.ty; d[6] = T.tz;
     }
-    anchor[lane] = moving ? node_of(lane) : par;
-    d[0] = T.w; d[1] = T.x; d[2] = T.y; d[3] = T.z; d[4] = T.tx; d[5] = T.ty; d[6] = T.tz;
+    anchor[lane] = static_cast<signed char>(moving ? node_of(lane) : par);
   }
   __syncthreads();
+  unsigned long long above = 0;  // of node `lane`: itself and its ancestors
+  if (lane < n_nodes)
+    for (int p = lane; p >= 0; p = nodes[p].parent_slot) above |= 1ull << p;
   if (wave == 0) {
-    if (lane < n_nodes)
-      for (int p = lane; p >= 0; p = nodes[p].r.parent_slot) atomicOr(&nodes[p].subtree, 1ull << lane);
     if (lane < n_valid) {
       for (int n = 0; n < n_nodes; ++n) {
-        const JointRec& r = nodes[n].r;
+        const JointRec& r = nodes[n];
         const float q = ((r.src >= 0) ? cfg_tile[r.src * kLaneStride + lane] : 0.f) * r.mul + r.off;
         Pose T = joint_local(r, q);
         if (r.parent_slot >= 0) T = compose(lds_get_pose(poses, r.parent_slot, lane), T);
@@ -629,10 +632,10 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
       }
     }
   } else {
-    // Meanwhile: each link's slot, and from it its node (-1: a link that does not move).
+    // Meanwhile: each link's slot (-1: a link on no joint).
     for (int l = tid - kWave; l < n_links; l += kWave * (kVjpWaves - 1)) {
       const int pj = lnode[l];
-      lnode[l] = (pj >= 0 && pj < J) ? slot_of[pj] : -1;
+      lnode[l] = static_cast<signed char>(pj >= 0 ? slot_of[pj] : -1);
     }
   }
   __syncthreads();
@@ -647,7 +650,8 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
         const int l = l0 + __builtin_ctzll(m);
         const float gw = g[7 * l], gx = g[7 * l + 1], gy = g[7 * l + 2], gz = g[7 * l + 3];
         const float fx = g[7 * l + 4], fy = g[7 * l + 5], fz = g[7 * l + 6];
-        const Pose T = compose(N, load_pose(rel + 7 * lnode[l]));
+        const int slot = uniform_i(lnode[l]);
+        const Pose T = ((moves >> slot) & 1ull) ? N : compose(N, load_pose(rel_of(slot)));
         W[0] += fx; W[1] += fy; W[2] += fz;
         W[3] += (T.ty * fz - T.tz * fy) + 0.5f * (T.w * gx - gw * T.x + (T.y * gz - T.z * gy));
         W[4] += (T.tz * fx - T.tx * fz) + 0.5f * (T.w * gy - gw * T.y + (T.z * gx - T.x * gz));
@@ -661,11 +665,12 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
   // Subtree sums and projections; a node's dq contribution replaces the first
   // component of its pose, which no other node reads here.
   for (int n = wave; n < n_nodes; n += kVjpWaves) {
-    const JointRec& r = nodes[n].r;
+    const JointRec& r = nodes[n];
     float d = 0.f;
+    const unsigned long long subtree = __ballot((above >> n) & 1ull);  // nodes at or below n
     if (r.src >= 0) {
       float W[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (unsigned long long m = nodes[n].subtree; m != 0; m &= m - 1ull) {
+      for (unsigned long long m = subtree; m != 0; m &= m - 1ull) {
         const float* w = wrench + 6 * __builtin_ctzll(m) * kLaneStride + lane;
 #pragma unroll
         for (int c = 0; c < 6; ++c) W[c] += w[c * kLaneStride];
@@ -692,7 +697,7 @@ __global__ __launch_bounds__(kWave * kVjpWaves) void fk_vjp_kernel(
   for (int a = wave; a < n_act; a += kVjpWaves) {
     float d = 0.f;
     for (int n = n_nodes - 1; n >= 0; --n)
-      if (nodes[n].r.src == a) d += poses[7 * n * kLaneStride + lane];
+      if (nodes[n].src == a) d += poses[7 * n * kLaneStride + lane];
     cfg_tile[a * kLaneStride + lane] = d;
   }
   __syncthreads();
@@ -744,13 +749,7 @@ extern "C" int pk_fk_vjp_f32(void* stream, const float* cfg, int64_t batch, int3
                              int32_t n_links, const float* cot_links, float* out_dq) {
   const pk::RobotTables t{twists, parent_tf, parent_idx, act_idx, mimic_mul,
                           mimic_off, mimic_act_idx, topo_inv, n_joints, n_act};
-  // Any joint may move; a table of 46 joints that all do is one too many for the
-  // LDS and reported as NaN, as a broken bound is.
-  int32_t moving = n_joints;
-  if (n_joints == 46 && n_links >= 0 && n_links <= pk::kMaxJoints + 1 &&
-      pk::vjp_lds(n_joints, n_links, n_act, moving).total > 160 * 1024)
-    --moving;
-  return launch_fk_vjp(stream, cfg, batch, n_act, t, link_parent_joint, n_links, moving, cot_links, out_dq);
+  return launch_fk_vjp(stream, cfg, batch, n_act, t, link_parent_joint, n_links, n_joints, cot_links, out_dq);  // any may move
 }
 
 extern "C" int pk_fk_vjp_moving_f32(void* stream, const float* cfg, int64_t batch, int32_t n_act,
