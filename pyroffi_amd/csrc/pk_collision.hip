@@ -186,11 +186,12 @@ __host__ __device__ inline int sweep_words_per_wave(int src, bool min_only, int 
 }
 
 // Bounding ball of one link's spheres in the link frame: xyz = centre (of the
-// spheres' box), w = radius, and `near` = min_k(|c_k - centre| - r_k).  For an
-// obstacle o of radius R with s = |o - centre| - R, the link's distance lies in
-// [s - w, s + near].  Spheres that no minimum takes (a NaN or infinite centre, a
-// radius of -inf) are left out; a radius of +inf gives w = near = +inf about the
-// origin, which rules nothing out.
+// spheres' box), and with `near` = min_k(|c_k - centre| - r_k) and `far` =
+// max_k(|c_k - centre| + r_k), w = far - near.  For an obstacle o of radius R with
+// s = |o - centre| - R, the link's distance lies in [s - far, s + near].  Spheres
+// that no minimum takes (a NaN or infinite centre, a radius of -inf) are left out; a
+// radius that is negative or +inf gives w = near = +inf about the origin, which rules
+// nothing out.
 __device__ __forceinline__ float4 link_ball(const float4* sl, int k0, int k1, float& near) {
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   bool any = false, sane = true;
@@ -201,7 +202,7 @@ __device__ __forceinline__ float4 link_ball(const float4* sl, int k0, int k1, fl
     const float4 s = sl[k];
     if (!counted(s)) continue;
     any = true;
-    sane = sane && s.w < INFINITY;
+    sane = sane && s.w >= 0.f && s.w < INFINITY;
     const float c[3] = {s.x, s.y, s.z};
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -210,21 +211,35 @@ __device__ __forceinline__ float4 link_ball(const float4* sl, int k0, int k1, fl
     }
   }
   const float bx = 0.5f * lo[0] + 0.5f * hi[0], by = 0.5f * lo[1] + 0.5f * hi[1], bz = 0.5f * lo[2] + 0.5f * hi[2];
-  float rb = -INFINITY;
+  float far = -INFINITY;
   near = INFINITY;
   for (int k = k0; k < k1; ++k) {
     const float4 s = sl[k];
     if (!counted(s)) continue;
     const float dx = s.x - bx, dy = s.y - by, dz = s.z - bz;
     const float d = sqrtf(dx * dx + dy * dy + dz * dz);
-    rb = fmaxf(rb, d + s.w);
+    far = fmaxf(far, d + s.w);
     near = fminf(near, d - s.w);
   }
-  sane = sane && fabsf(rb) < 1e6f;
-  // Slack for the rounding of the placed centre and of the distances.
-  near = any && sane ? near + 1e-5f : INFINITY;
-  if (!any) return make_float4(0.f, 0.f, 0.f, -INFINITY);
-  return sane ? make_float4(bx, by, bz, rb + 1e-5f) : make_float4(0.f, 0.f, 0.f, INFINITY);
+  sane = sane && fabsf(far) < 1e6f;
+  if (!any || !sane) {
+    near = INFINITY;
+    return make_float4(0.f, 0.f, 0.f, any ? INFINITY : -INFINITY);
+  }
+  return make_float4(bx, by, bz, far - near);
+}
+
+// The ball of a link at pose p in the world, w = near + what `s` and the bounds may be
+// off by: the rounding of the centre, by the size of its coordinates, and the stretch
+// of a quaternion that is not quite (or not at all) of unit length, which lengthens
+// vectors by at most 1 + 4 ||q|^2 - 1|.  far = w + local.w, off by as much.
+__device__ __forceinline__ float4 placed_ball(const float* p, const float4& local, float near) {
+  float wx, wy, wz;
+  quat_rotate(p[0], p[1], p[2], p[3], local.x, local.y, local.z, wx, wy, wz);
+  const float x = wx + p[4], y = wy + p[5], z = wz + p[6];
+  const float qq = p[0] * p[0] + p[1] * p[1] + p[2] * p[2] + p[3] * p[3];
+  const float off = 1e-5f + 4e-6f * (fabsf(x) + fabsf(y) + fabsf(z)) + 4.f * fabsf(qq - 1.f) * (local.w + near);
+  return make_float4(x, y, z, near + off);
 }
 
 // Exact minimum of the wave's `count` candidates (one per lane), into gmin.
@@ -254,7 +269,7 @@ __device__ __forceinline__ void candidate_min(int lane, int count, const float4*
 // pair that starts above it, and the few that are left (on Panda among 256
 // obstacles a few dozen of 2816) are collected, one per lane, and measured.
 // Lane i keeps the least s of link i, so at most 64 links are taken at a time.
-// Panda, 65536 configurations x 256 obstacles with poses and self pairs: 273 -> 220 us.
+// Panda, 65536 configurations x 256 obstacles with poses and self pairs: 273 -> 225 us.
 template <int T>
 __device__ __forceinline__ void world_min_culled(int lane, int n_balls, const float4* ball, const float4* local_ball,
                                                  const unsigned* brange, const float4* sc, float4* cand,
@@ -277,17 +292,17 @@ __device__ __forceinline__ void world_min_culled(int lane, int n_balls, const fl
   }
   int count = 0;
   unsigned long long hits =
-      __ballot(lane < n_balls && !(first - local_ball[min(lane, n_balls - 1)].w > upper));
+      __ballot(lane < n_balls && !(first - (ball[min(lane, n_balls - 1)].w + local_ball[min(lane, n_balls - 1)].w) > upper));
   while (hits) {
     const int i = __builtin_ctzll(hits);
     hits &= hits - 1;
     const float4 b = ball[i];
-    const float rb = local_ball[i].w;
+    const float far = b.w + local_ball[i].w;
     const unsigned range = brange[i];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const float s = clear(b, t);
-      const bool in = s == s && !(s - rb > upper);
+      const bool in = s == s && !(s - far > upper);
       const unsigned long long m = __ballot(in);
       if (m == 0) continue;
       const int add = __popcll(m);
@@ -442,6 +457,11 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
   const int chunk = kWave * T;
   const int n_chunks = (M + chunk - 1) / chunk;
   float ox[T], oy[T], oz[T], orad[T];
+  // Minimum only: where a configuration is placed farther than this from the world's
+  // origin, its coordinates are taken from its first ball's link, (0, 0, 0) else: sums
+  // of offset and position then lose no more than they do near the origin.
+  constexpr float kFar = 4.f;
+  float base[3] = {0.f, 0.f, 0.f};
   auto load_obstacles = [&](int c) {
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -449,6 +469,7 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
       if (m < M) {
         ox[t] = a.world[4 * m]; oy[t] = a.world[4 * m + 1];
         oz[t] = a.world[4 * m + 2]; orad[t] = a.world[4 * m + 3];
+        if constexpr (CULL) { ox[t] -= base[0]; oy[t] -= base[1]; oz[t] -= base[2]; }
       } else {  // never the minimum: infinitely far
         ox[t] = 0.f; oy[t] = 0.f; oz[t] = 0.f; orad[t] = -INFINITY;
       }
@@ -471,6 +492,25 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
       const float* pb = a.link_poses + b * L * 7;
       for (int f = lane; f < L * 7; f += kWave) ptile[f] = pb[f];
       wave_sync();
+      if constexpr (CULL) {
+        const float* p = ptile + 7 * slink[n_balls > 0 ? brange[0] & 0xffffu : 0];
+        float at[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) at[j] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(p[4 + j])));
+        const float size = fmaxf(fmaxf(fabsf(at[0]), fabsf(at[1])), fabsf(at[2]));
+        const bool far = n_balls > 0 && size > kFar && fabsf(at[0]) + fabsf(at[1]) + fabsf(at[2]) < INFINITY;
+        if (far || base[0] != 0.f || base[1] != 0.f || base[2] != 0.f) {
+#pragma unroll
+          for (int j = 0; j < 3; ++j) base[j] = far ? at[j] : 0.f;
+          if (n_chunks > 0) load_obstacles(0);
+          wave_sync();
+          for (int n = lane; n < L; n += kWave) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) ptile[7 * n + 4 + j] -= base[j];
+          }
+          wave_sync();
+        }
+      }
       for (int k = lane; k < K; k += kWave) {
         const float* p = ptile + 7 * slink[k];
         const float4 s = sl[k];
@@ -480,13 +520,8 @@ __global__ __launch_bounds__(kWave * kSweepWaves, T == 8 ? 3 : 6) void sweep_ker
         if (!CULL) se[k] = make_float4(-2.f * wx, -2.f * wy, -2.f * wz, wx * wx + wy * wy + wz * wz);
       }
       if constexpr (CULL) {
-        for (int i = lane; i < n_balls; i += kWave) {
-          const float* p = ptile + 7 * slink[brange[i] & 0xffffu];
-          const float4 s = lball[i];
-          float wx, wy, wz;
-          quat_rotate(p[0], p[1], p[2], p[3], s.x, s.y, s.z, wx, wy, wz);
-          ball[i] = make_float4(wx + p[4], wy + p[5], wz + p[6], bnear[i]);
-        }
+        for (int i = lane; i < n_balls; i += kWave)
+          ball[i] = placed_ball(ptile + 7 * slink[brange[i] & 0xffffu], lball[i], bnear[i]);
       }
     } else {
       const long long BK = a.batch * K;

@@ -93,3 +93,25 @@ def test_no_obstacles_and_no_spheres():
     poses, start, spheres, world = _case(4, 5, 3, 8, 5)
     assert (_sweep(poses, start, spheres, world[:0], rows=False) == np.float32(1e9)).all()
     assert (_sweep(poses, np.zeros(6, np.int32), spheres[:0], world, rows=False) == np.float32(1e9)).all()
+
+
+@pytest.mark.parametrize("far", [100.0, 3000.0])
+def test_scene_far_from_the_origin(far):
+    """Robot and obstacles together at `far` metres, a power-of-two grid of 2^-12 m keeping the
+    offsets exact: the distances are those of a scene at the origin, to the same tolerance."""
+    poses, start, spheres, world = _case(200, 13, 9, 200, 17)
+    poses[..., 4:] = np.round(poses[..., 4:] * 4096) / 4096 + np.round(far * 4096) / 4096
+    world[:, :3] = np.round(world[:, :3] * 4096) / 4096 + np.round(far * 4096) / 4096
+    assert (np.abs(poses[..., 4:]) < 2**12).all()  # 24 bits: exact
+    got = _sweep(poses, start, spheres, world, rows=False)
+    np.testing.assert_allclose(got, _reference(poses, start, spheres, world), atol=TOL, rtol=0)
+
+
+@pytest.mark.parametrize("scale", [0.25, 0.999, 1.001, 1.5])
+def test_quaternions_that_are_not_of_unit_length(scale):
+    """The placement is linear in the sphere's offset, whatever the quaternion: the minimum is that
+    of the rows' own formula.  Offsets up to 3 m: TOL."""
+    poses, start, spheres, world = _case(300, 9, 12, 100, 23)
+    poses[::2, :, :4] *= np.float32(scale)
+    got, ref = _sweep(poses, start, spheres, world, rows=False), _reference(poses, start, spheres, world)
+    np.testing.assert_allclose(got, ref, atol=TOL, rtol=0)
