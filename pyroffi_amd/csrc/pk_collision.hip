@@ -174,7 +174,14 @@ __device__ __forceinline__ void link_sweep(int n, int g0, int g1, const float4* 
 // The candidates of the configuration minimum: (link, obstacle) pairs that a
 // link's bounding ball cannot rule out.  A wave holds at most one per lane.
 constexpr int kCandidates = kWave;
-constexpr int kCullMinSpheres = 12;  // see launch_sweep
+
+// Whether the configuration minimum is worth its bounds, whose fixed part a robot of
+// few spheres does not win back.  32768 configurations, every pair / culled, us, links x
+// spheres among 64, 256 and 512 obstacles: 3 x 4, 33 / 31, 49 / 46, 89 / 67; 12 x 1, 46 /
+// 42, 68 / 63, 119 / 94; 11 x 5, 115 / 60, 179 / 108, 333 / 188; below 12 it depends on
+// how they lie: 11 x 1, 42 / 40, 62 / 60, 109 / 88, but 5 x 2, 32 / 33, 48 / 56, 83 / 83;
+// 3 x 3, 28 / 29, 42 / 44, 71 / 60; 4 x 2, 28 / 31, 40 / 46, 69 / 70.
+inline bool cull_pays(int n_spheres, int n_world) { return n_spheres >= (n_world > 256 ? 9 : 12); }
 
 // LDS of one wave: the world spheres and a blank, then the expanded entries (rows)
 // or the placed balls and the candidates (minimum only); pose tile, pair minima.
@@ -733,13 +740,9 @@ static int launch_sweep(void* stream, const SweepArgs& a) {
            sizeof(int) * ((L + 1) + (SRC == 0 ? K : 0) + (K + 1) + (L + 1)) +
            sizeof(float) * (SRC == 0 ? L : 0) + per_wave * kSweepWaves;
   };
-  // The bounds cost a fixed part of each configuration, which a robot of very few
-  // spheres does not win back.  32768 configurations, every pair / culled, us: 2 links
-  // x 2 spheres 19 / 23 (64 obstacles), 42 / 53 (512); 2 x 4, 27 / 29 (128), 65 / 58;
-  // 11 x 1, 43 / 38, 110 / 90; 2 x 8, 39 / 30, 111 / 54; 11 x 5, 114 / 58, 343 / 199.
-  // A very long entry list can also need more LDS with the candidates' buffers than
+  // A very long entry list can need more LDS with the candidates' buffers than
   // without: such a launch sweeps every pair.
-  const bool cull = SRC == 0 && a.out_world == nullptr && a.out_min != nullptr && K >= kCullMinSpheres &&
+  const bool cull = SRC == 0 && a.out_world == nullptr && a.out_min != nullptr && cull_pays(K, a.n_world) &&
                     lds_bytes(true) <= 150 * 1024;
   const size_t lds = lds_bytes(cull);
   PK_REQUIRE(a.n_entries == 0 || K < 1024, "self entries address at most 1023 spheres (got %d)", K);

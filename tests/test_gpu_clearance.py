@@ -47,7 +47,7 @@ def _sweep(poses, start, spheres, world, rows):
 
 
 @pytest.mark.parametrize("B,L,per_link,M", [(1, 1, 1, 1), (6, 2, 12, 1), (5, 3, 6, 64), (300, 13, 9, 65), (37, 13, 9, 129),
-                                            (21, 65, 3, 256), (9, 65, 3, 1100), (2, 4, 250, 513)])
+                                            (21, 65, 3, 256), (50, 2, 9, 256), (50, 2, 9, 257), (9, 65, 3, 1100), (2, 4, 250, 513)])
 def test_minimum_of_random_scenes(B, L, per_link, M):
     case = _case(B, L, per_link, M, B + L + M)
     got, ref = _sweep(*case, rows=False), _reference(*case)
