@@ -649,7 +649,7 @@ __device__ __forceinline__ float group_waypoint_coll(const TrajModelDev& md, con
   // path of 128 waypoints, cost and gradient 371 us.)
   GridCell next, after;
   int ahead[kItems];
-  next = grid_cell_of(md.grid, md.n_world, gc[min(g, Ks - 1)], g < Ks);
+  next = grid_cell_of(md.grid, md.n_world, gc[max(min(g, Ks - 1), 0)], g < Ks);
   grid_items(next, 0, ahead);
   after = grid_cell_of(md.grid, md.n_world, gc[max(min(g + kGroup, Ks - 1), 0)], g + kGroup < Ks);
   for (int s = g; s < Ks; s += kGroup) {
