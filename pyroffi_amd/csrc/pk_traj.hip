@@ -620,12 +620,17 @@ __device__ __forceinline__ void wave_world_coll(const TrajModelDev& md, const Tr
   }
 }
 
+// How a kernel finds the obstacles near its spheres: in the grid, one lookup after the
+// other (kLookup) or reading ahead (kLookupAhead), or with the wave's waypoints
+// sharing a search (kHulls, wave_world_coll).
+enum WorldSearch { kLookup, kLookupAhead, kHulls };
+
 // Collision cost of one waypoint, evaluated by the kGroup lanes of a group
 // (lane g = threadIdx.x % kGroup) from the centres in gc, and with GRAD the
 // group's dcost/dq_node (per node, before the mimic map).  Every lane of the
-// group returns the group totals.  HULL: the world term by wave_world_coll, for
-// which every lane of the wave calls this, `active` or not.
-template <int MAXN, bool GRAD, bool HULL>
+// group returns the group totals.  With kHulls every lane of the wave calls this,
+// `active` or not.
+template <int MAXN, bool GRAD, WorldSearch SEARCH>
 __device__ __forceinline__ float group_waypoint_coll(const TrajModelDev& md, const TrajLds& L, const WaypointNodes<MAXN, GRAD>& K,
                                      const float4* gc, bool active, float (&gn)[MAXN]) {
   const int g = threadIdx.x % kGroup;
@@ -637,84 +642,104 @@ __device__ __forceinline__ float group_waypoint_coll(const TrajModelDev& md, con
 #pragma unroll
   for (int a = 0; a < MAXN; ++a) gn[a] = 0.f;
 
-  if constexpr (HULL) {
+  // World: spheres s = g, g + kGroup, ... of the waypoint.  Obstacle o of a sphere s
+  // that is within the margin of it: the (link, world sphere) term is owned by the
+  // link's lowest-index sphere within the margin; the owner takes the minimum over the
+  // link.
+  struct LinkOf {
+    int k0, k1, mask;  // its spheres, its ancestors
+  };
+  auto link_of = [&](int s) {
+    const int l = L.sph_link[s], node = L.link_node[l];
+    return LinkOf{L.link_sph[l], L.link_sph[l + 1], node >= 0 ? L.anc[node] : 0};
+  };
+  auto near_obstacle = [&](int s, const LinkOf& link, const float4& c, const float4& o, float dx, float dy, float dz,
+                           float dist, float d) {
+    const int k0 = link.k0, k1 = link.k1;
+    for (int s2 = k0; s2 < s; ++s2) {
+      const float4 c2 = gc[s2];
+      const float ex = o.x - c2.x + e, ey = o.y - c2.y + e, ez = o.z - c2.z + e;
+      if (sqrtf(ex * ex + ey * ey + ez * ez) - c2.w - o.w < margin) return;
+    }
+    float bd = d, bdist = dist, bx = dx, by = dy, bz = dz, bcx = c.x, bcy = c.y, bcz = c.z;
+    for (int s2 = s + 1; s2 < k1; ++s2) {
+      const float4 c2 = gc[s2];
+      const float ex = o.x - c2.x + e, ey = o.y - c2.y + e, ez = o.z - c2.z + e;
+      const float dd = sqrtf(ex * ex + ey * ey + ez * ez);
+      if (dd - c2.w - o.w < bd) {
+        bd = dd - c2.w - o.w; bdist = dd; bx = ex; by = ey; bz = ez; bcx = c2.x; bcy = c2.y; bcz = c2.z;
+      }
+    }
+    float df;
+    cost += traj_act(bd, margin, mode, df);
+    if (GRAD && df != 0.f) {
+      const float k = -df / bdist;
+      pull_point<MAXN, GRAD>(K, link.mask, bcx, bcy, bcz, k * bx, k * by, k * bz, gn);
+    }
+  };
+  if constexpr (SEARCH == kHulls) {
     wave_world_coll<MAXN, GRAD>(md, L, K, gc, active, cost, gn);
     if (!active) return 0.f;
-  } else {
-  // World: spheres s = g, g + kGroup, ... of the waypoint.  A sphere's lookup
-  // is a chain of global loads (the cell's entry, then its obstacle indices),
-  // which one wave cannot hide: the entry is read two spheres ahead and the
-  // first kItems indices one sphere ahead, and further ones kItems at a time.
-  // (Read one by one, the chain was most of a pass: Panda, 1024 obstacles, one
-  // path of 128 waypoints, cost and gradient 371 us.)
-  GridCell next, after;
-  int ahead[kItems];
-  next = grid_cell_of(md.grid, md.n_world, gc[max(min(g, Ks - 1), 0)], g < Ks);
-  grid_items(next, 0, ahead);
-  after = grid_cell_of(md.grid, md.n_world, gc[max(min(g + kGroup, Ks - 1), 0)], g + kGroup < Ks);
-  for (int s = g; s < Ks; s += kGroup) {
-    const float4 c = gc[s];
-    const GridCell cell = next;
-    int m8[kItems];
-#pragma unroll
-    for (int u = 0; u < kItems; ++u) m8[u] = ahead[u];
-    next = after;
-    grid_items(next, 0, ahead);
-    after = grid_cell_of(md.grid, md.n_world, gc[min(s + 2 * kGroup, Ks - 1)], s + 2 * kGroup < Ks);
-    const int total = cell.count;
-    if (total == 0) continue;
-    const int l = L.sph_link[s];
-    const int k0 = L.link_sph[l], k1 = L.link_sph[l + 1];
-    const int node = L.link_node[l];
-    const int mask = node >= 0 ? L.anc[node] : 0;
-    for (int i0 = 0; i0 < total; i0 += kItems) {
-    if (i0 > 0) grid_items(cell, i0, m8);
-    unsigned near = 0;  // obstacles of this batch within the margin
-#pragma unroll
-    for (int u = 0; u < kItems; ++u) {
-      const int m = m8[u];
-      if (i0 + u >= total || m < 0 || m >= md.n_world) continue;
-      const float4 o = L.world[m];
-      const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
-      if (sqrtf(dx * dx + dy * dy + dz * dz) - c.w - o.w < margin) near |= 1u << u;
-    }
-    for (; near != 0; near &= near - 1) {
-      const int u0 = __builtin_ctz(near);
-      int m = m8[0];
-#pragma unroll
-      for (int u = 1; u < kItems; ++u)
-        if (u == u0) m = m8[u];
-      const float4 o = L.world[m];
-      const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
-      const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
-      const float d = dist - c.w - o.w;
-      // The (link, world sphere) term is owned by the link's lowest-index
-      // sphere within the margin; the owner takes the minimum over the link.
-      bool owner = true;
-      for (int s2 = k0; s2 < s; ++s2) {
-        const float4 c2 = gc[s2];
-        const float ex = o.x - c2.x + e, ey = o.y - c2.y + e, ez = o.z - c2.z + e;
-        if (sqrtf(ex * ex + ey * ey + ez * ez) - c2.w - o.w < margin) { owner = false; break; }
+  } else if constexpr (SEARCH == kLookup) {
+    for (int s = g; s < Ks; s += kGroup) {
+      const float4 c = gc[s];
+      const GridCell cell = grid_cell_of(md.grid, md.n_world, c, true);
+      for (int i = 0; i < cell.count; ++i) {
+        const int m = cell.items != nullptr ? cell.items[i] : i;
+        if (m < 0 || m >= md.n_world) continue;
+        const float4 o = L.world[m];
+        const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
+        const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+        const float d = dist - c.w - o.w;
+        if (d < margin) near_obstacle(s, link_of(s), c, o, dx, dy, dz, dist, d);
       }
-      if (!owner) continue;
-      float bd = d, bdist = dist, bx = dx, by = dy, bz = dz, bcx = c.x, bcy = c.y, bcz = c.z;
-      for (int s2 = s + 1; s2 < k1; ++s2) {
-        const float4 c2 = gc[s2];
-        const float ex = o.x - c2.x + e, ey = o.y - c2.y + e, ez = o.z - c2.z + e;
-        const float dd = sqrtf(ex * ex + ey * ey + ez * ez);
-        if (dd - c2.w - o.w < bd) {
-          bd = dd - c2.w - o.w; bdist = dd; bx = ex; by = ey; bz = ez; bcx = c2.x; bcy = c2.y; bcz = c2.z;
+    }
+  } else {
+    // A sphere's lookup is a chain of global loads (the cell's entry, then its
+    // obstacle indices), which one wave cannot hide: the entry is read two spheres
+    // ahead and the first kItems indices one sphere ahead, and further ones kItems at a
+    // time.  (Read one by one, the chain was most of a pass: Panda, 1024 obstacles, one
+    // path of 128 waypoints, cost and gradient 371 us.)
+    GridCell next, after;
+    int ahead[kItems];
+    next = grid_cell_of(md.grid, md.n_world, gc[max(min(g, Ks - 1), 0)], g < Ks);
+    grid_items(next, 0, ahead);
+    after = grid_cell_of(md.grid, md.n_world, gc[max(min(g + kGroup, Ks - 1), 0)], g + kGroup < Ks);
+    for (int s = g; s < Ks; s += kGroup) {
+      const float4 c = gc[s];
+      const GridCell cell = next;
+      int m8[kItems];
+#pragma unroll
+      for (int u = 0; u < kItems; ++u) m8[u] = ahead[u];
+      next = after;
+      grid_items(next, 0, ahead);
+      after = grid_cell_of(md.grid, md.n_world, gc[min(s + 2 * kGroup, Ks - 1)], s + 2 * kGroup < Ks);
+      if (cell.count == 0) continue;
+      const LinkOf link = link_of(s);
+      for (int i0 = 0; i0 < cell.count; i0 += kItems) {
+        if (i0 > 0) grid_items(cell, i0, m8);
+        unsigned near = 0;  // obstacles of this batch within the margin
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+          const int m = m8[u];
+          if (i0 + u >= cell.count || m < 0 || m >= md.n_world) continue;
+          const float4 o = L.world[m];
+          const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
+          if (sqrtf(dx * dx + dy * dy + dz * dz) - c.w - o.w < margin) near |= 1u << u;
+        }
+        for (; near != 0; near &= near - 1) {
+          const int u0 = __builtin_ctz(near);
+          int m = m8[0];
+#pragma unroll
+          for (int u = 1; u < kItems; ++u)
+            if (u == u0) m = m8[u];
+          const float4 o = L.world[m];
+          const float dx = o.x - c.x + e, dy = o.y - c.y + e, dz = o.z - c.z + e;
+          const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+          near_obstacle(s, link, c, o, dx, dy, dz, dist, dist - c.w - o.w);
         }
       }
-      float df;
-      cost += traj_act(bd, margin, mode, df);
-      if (GRAD && df != 0.f) {
-        const float k = -df / bdist;
-        pull_point<MAXN, GRAD>(K, mask, bcx, bcy, bcz, k * bx, k * by, k * bz, gn);
-      }
     }
-    }
-  }
   }
 
   // Self: active pairs split over the group's lanes, bounding-sphere culled.
@@ -782,7 +807,7 @@ __device__ __forceinline__ void node_to_actuated(const TrajLds& L, int N, const 
 // configuration of task i, done(i, cost, gq) consumes the group totals (every
 // lane of the group calls it).  All threads run the same number of rounds, so
 // the workgroup barriers inside are uniform.
-template <int MAXN, bool GRAD, bool HULL, typename TaskFn, typename DoneFn>
+template <int MAXN, bool GRAD, WorldSearch SEARCH, typename TaskFn, typename DoneFn>
 __device__ __forceinline__ void for_each_waypoint(const TrajModelDev& md, const TrajLds& L, int n_tasks,
                                                   TaskFn task, DoneFn done) {
   const int grp = threadIdx.x / kGroup;
@@ -801,9 +826,9 @@ __device__ __forceinline__ void for_each_waypoint(const TrajModelDev& md, const 
       waypoint_centres<MAXN, GRAD>(md, L, K, gc);
     }
     __syncthreads();
-    if (active || HULL) {
+    if (active || SEARCH == kHulls) {
       float gn[MAXN], gq[MAXN];
-      const float c = group_waypoint_coll<MAXN, GRAD, HULL>(md, L, K, gc, active, gn);
+      const float c = group_waypoint_coll<MAXN, GRAD, SEARCH>(md, L, K, gc, active, gn);
       if (active) {
         if (GRAD) node_to_actuated<MAXN>(L, N, gn, gq);
         done(i, c, gq);
@@ -817,7 +842,7 @@ __device__ __forceinline__ void for_each_waypoint(const TrajModelDev& md, const 
 // threads receiving the totals; with GRAD, L.vg = gradient of
 // w_smooth smooth + w_limits limits + w_coll coll (endpoint rows zeroed when
 // mask_ends).  Leaves the accelerations of x in L.vt; uses L.vd as scratch.
-template <int MAXN, bool GRAD, bool HULL = false>
+template <int MAXN, bool GRAD, WorldSearch SEARCH>
 __device__ __forceinline__ void traj_value_grad(const TrajModelDev& md, const TrajLds& L, const float* X, int T,
                                                 const TrajWeights& w, float w_coll, bool mask_ends,
                                                 float (&comps)[3]) {
@@ -826,7 +851,7 @@ __device__ __forceinline__ void traj_value_grad(const TrajModelDev& md, const Tr
   const int tid = threadIdx.x;
   float coll = 0.f, lim = 0.f, sm = 0.f;
   const bool leader = (tid % kGroup) == 0;
-  for_each_waypoint<MAXN, GRAD, HULL>(
+  for_each_waypoint<MAXN, GRAD, SEARCH>(
       md, L, T,
       [&](int t, float (&q)[MAXN]) {
 #pragma unroll
@@ -900,10 +925,10 @@ __device__ __forceinline__ void traj_value_grad(const TrajModelDev& md, const Tr
   comps[2] = v3[2];
 }
 
-template <int MAXN, bool GRAD>
+template <int MAXN, bool GRAD, WorldSearch SEARCH>
 __device__ __forceinline__ void traj_value_grad(const TrajModelDev& md, const TrajLds& L, int T, const TrajWeights& w,
                                                 float w_coll, bool mask_ends, float (&comps)[3]) {
-  traj_value_grad<MAXN, GRAD>(md, L, L.vx, T, w, w_coll, mask_ends, comps);
+  traj_value_grad<MAXN, GRAD, SEARCH>(md, L, L.vx, T, w, w_coll, mask_ends, comps);
 }
 
 // Line search of _lbfgs_direct_solve on x + alpha_k d, alpha in {1, .5, .25,
@@ -911,7 +936,7 @@ __device__ __forceinline__ void traj_value_grad(const TrajModelDev& md, const Tr
 // (first index on ties).  The points are evaluated in that order and the
 // search stops at the first acceptable one, which picks the same step as
 // evaluating all five.  Returns the step index and its cost components.
-template <int MAXN>
+template <int MAXN, WorldSearch SEARCH>
 __device__ __forceinline__ int traj_line_search(const TrajModelDev& md, const TrajLds& L, int T, const TrajWeights& w,
                                 float w_coll, float thresh, float& p_sm, float& p_lim, float& p_col) {
   const int A = md.n_act;
@@ -957,7 +982,7 @@ __device__ __forceinline__ int traj_line_search(const TrajModelDev& md, const Tr
   for (int k = 0; k < kNumAlphas; ++k) {
     const float al = traj_alpha(k);
     float ck = 0.f;
-    for_each_waypoint<MAXN, false, false>(
+    for_each_waypoint<MAXN, false, SEARCH>(
         md, L, T,
         [&](int t, float (&q)[MAXN]) {
 #pragma unroll
@@ -1008,20 +1033,37 @@ struct CostArgs {
 // Waypoints from which the cost kernel takes the world term by wave_world_coll.
 constexpr int kHullWaypoints = 24;
 
-// A wave tests every obstacle against every link, where the grid looks up every
-// sphere and few obstacles leave its cells nearly empty.  150 paths of 48 waypoints,
-// cost and gradient, grid / hulls, us: Panda (59 spheres on 13 links) 88 / 88 among
-// 32 obstacles, 137 / 96 among 128, 357 / 192 among 1024; UR5 (40 spheres, 17 links
-// with any) 145 / 158 among 128, 275 / 308 among 1024.
+// Where the shared search wins: a wave tests every obstacle against every link, where
+// the grid looks up every sphere, so it takes many spheres a link (of all links; the
+// host knows no other number, and eight in ten of them carry spheres) and obstacles
+// enough to fill the grid's cells.  150 paths of 48 waypoints (Baxter 32), cost and
+// gradient, grid / shared, us, among 128 and 512 obstacles, below the line: UR5 (40
+// spheres on 23 links) 129 / 150, 162 / 231, with 68 172 / 176, 233 / 253; Panda with 44
+// on 13 85 / 86, 126 / 125; Baxter (75 on 44) 381 / 446, 547 / 596, with 132 528 / 516,
+// 825 / 677; above it: Panda with 55 96 / 91, 151 / 130, Panda (59) 118 / 91, 199 / 132;
+// Fetch with 75 on 17 133 / 123, 282 / 187; Fetch (111) 165 / 134, 416 / 213; Baxter with
+// 264 802 / 631, 1357 / 823; UR5 with 136 276 / 223, 432 / 306.
 inline bool use_hulls(const TrajModelDev& md) {
   return md.n_world >= 128 && md.n_spheres >= 4 * md.n_links;
 }
 
-// HULLS: launched with use_hulls (a kernel of its own, so that the other keeps its registers).
-template <int MAXN, bool HULLS>
+// Where reading ahead wins: a lookup that finds an empty cell has nothing to read, and
+// few obstacles leave most cells empty.  One by one / ahead, us, 150 paths of 48
+// waypoints among 32, 64, 192, 256 and 512 obstacles: Panda's cost and gradient 77 / 85,
+// 134 / 126, 159 / 140, 230 / 192, 244 / 192 (Baxter 328 / 335, 359 / 359, 408 / 400, 471
+// / 425, 605 / 548); six L-BFGS iterations 584 / 646, 801 / 806, 912 / 810, 1281 / 1061,
+// 1120 / 942 (UR5 at 192 776 / 759, four paths 738 / 783; Baxter at 192 and 256 2019 /
+// 1996, 2231 / 2024); five CHOMP iterations 1661 / 1910, 2347 / 2514, 2992 / 2795 (UR5
+// 2435 / 2491), 3790 / 3529, 3795 / 3388.  CHOMP for more than eight nodes, which spills
+// 30 registers with it, gains nothing: 5588 / 6157, 6026 / 6430, 6912 / 7308, 7807 / 7751,
+// 9245 / 9228.
+inline bool cost_looks_ahead(const TrajModelDev& md) { return md.n_world >= 64; }
+inline bool solvers_look_ahead(const TrajModelDev& md) { return md.n_world >= 256; }
+
+template <int MAXN, WorldSearch SEARCH>
 __global__ __launch_bounds__(kMaxTrajThreads) void traj_cost_kernel(CostArgs a) {
   extern __shared__ float4 smem4[];
-  const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4), HULLS);
+  const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4), SEARCH == kHulls);
   const int b = a.subset ? a.subset[blockIdx.x] : static_cast<int>(blockIdx.x);
   if (b < 0 || b >= a.n_traj) return;  // uniform per block
   const long long w0 = a.start[b], w1 = a.start[b + 1];
@@ -1034,15 +1076,16 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_cost_kernel(CostArgs a) 
   // Neighbouring waypoints of a short path are too far apart to share a search
   // (1024 obstacles, 150 paths, cost and gradient, grid against hulls: 8
   // waypoints 161 / 261 us, 32: 307 / 230, 128: 293 / 181).
-  if (HULLS && T >= kHullWaypoints) {
+  constexpr WorldSearch kShort = SEARCH == kHulls ? kLookupAhead : SEARCH;
+  if (SEARCH == kHulls && T >= kHullWaypoints) {
     if (a.out_grad != nullptr)
-      traj_value_grad<MAXN, true, true>(a.md, L, L.vx, T, a.w, a.w_coll, false, comps);
+      traj_value_grad<MAXN, true, SEARCH>(a.md, L, T, a.w, a.w_coll, false, comps);
     else
-      traj_value_grad<MAXN, false, true>(a.md, L, L.vx, T, a.w, a.w_coll, false, comps);
+      traj_value_grad<MAXN, false, SEARCH>(a.md, L, T, a.w, a.w_coll, false, comps);
   } else if (a.out_grad != nullptr) {
-    traj_value_grad<MAXN, true>(a.md, L, T, a.w, a.w_coll, false, comps);
+    traj_value_grad<MAXN, true, kShort>(a.md, L, T, a.w, a.w_coll, false, comps);
   } else {
-    traj_value_grad<MAXN, false>(a.md, L, T, a.w, a.w_coll, false, comps);
+    traj_value_grad<MAXN, false, kShort>(a.md, L, T, a.w, a.w_coll, false, comps);
   }
   if (a.out_grad != nullptr) {
     for (int i = threadIdx.x; i < T * A; i += blockDim.x) a.out_grad[w0 * A + i] = L.vg[i];
@@ -1074,7 +1117,7 @@ struct LbfgsArgs {
   float* out_cost;  // (B)
 };
 
-template <int MAXN>
+template <int MAXN, WorldSearch SEARCH>
 __global__ __launch_bounds__(kMaxTrajThreads) void traj_lbfgs_kernel(LbfgsArgs a) {
   extern __shared__ float4 smem4[];
   const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4));
@@ -1122,7 +1165,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_lbfgs_kernel(LbfgsArgs a
   for (int k = a.it0; k < a.it1; ++k) {
     if (k > 0 && k % a.escalation == 0) w_coll = fminf(w_coll * a.penalty_scale, a.w_coll_max);
     float comps[3];
-    traj_value_grad<MAXN, true>(a.md, L, T, a.w, w_coll, true, comps);
+    traj_value_grad<MAXN, true, SEARCH>(a.md, L, T, a.w, w_coll, true, comps);
     const float cost = a.w.w_smooth * comps[0] + a.w.w_limits * comps[1] + w_coll * comps[2];
     if (k == 0) {
       for (int i = tid; i < n; i += blockDim.x) {
@@ -1205,7 +1248,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_lbfgs_kernel(LbfgsArgs a
     }
     __syncthreads();
     float p_sm = 0.f, p_lim = 0.f, p_col = 0.f;
-    const int pick = traj_line_search<MAXN>(a.md, L, T, a.w, w_coll, cost * (1.f - 1e-4f), p_sm, p_lim, p_col);
+    const int pick = traj_line_search<MAXN, SEARCH>(a.md, L, T, a.w, w_coll, cost * (1.f - 1e-4f), p_sm, p_lim, p_col);
     const float al = traj_alpha(pick);
     for (int i = tid; i < n; i += blockDim.x) {
       xp[i] = L.vx[i];
@@ -1285,7 +1328,7 @@ __device__ __forceinline__ float get_at(const float (&v)[MAXN], int a) {
   return r;
 }
 
-template <int MAXN>
+template <int MAXN, WorldSearch SEARCH>
 __global__ __launch_bounds__(kMaxTrajThreads) void traj_chomp_kernel(ChompArgs a) {
   extern __shared__ float4 smem4[];
   const TrajLds L = stage_traj_model(a.md, a.max_len, reinterpret_cast<char*>(smem4));
@@ -1310,7 +1353,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_chomp_kernel(ChompArgs a
       continue;
     }
     float comps[3];
-    traj_value_grad<MAXN, true>(a.md, L, L.vx, T, a.w, w_coll, false, comps);
+    traj_value_grad<MAXN, true, SEARCH>(a.md, L, L.vx, T, a.w, w_coll, false, comps);
     const float cost = a.w.w_smooth * comps[0] + a.w.w_limits * comps[1] + w_coll * comps[2];
     float g2 = 0.f;
     for (int i = tid; i < n; i += blockDim.x) g2 += L.vg[i] * L.vg[i];
@@ -1386,7 +1429,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_chomp_kernel(ChompArgs a
         L.vg[i] = L.vx[i] + fminf(fmaxf(al * L.vd[i], -a.max_delta), a.max_delta);
       __syncthreads();
       float tc[3];
-      traj_value_grad<MAXN, false>(a.md, L, L.vg, T, a.w, w_coll, false, tc);
+      traj_value_grad<MAXN, false, SEARCH>(a.md, L, L.vg, T, a.w, w_coll, false, tc);
       const float c = a.w.w_smooth * tc[0] + a.w.w_limits * tc[1] + w_coll * tc[2];
       if (c < best || (kk < pick && c == best)) {
         best = c;
@@ -1410,7 +1453,7 @@ __global__ __launch_bounds__(kMaxTrajThreads) void traj_chomp_kernel(ChompArgs a
     __syncthreads();
   }
   float comps[3];
-  traj_value_grad<MAXN, false>(a.md, L, L.vx, T, a.w, a.w_coll_max, false, comps);
+  traj_value_grad<MAXN, false, SEARCH>(a.md, L, L.vx, T, a.w, a.w_coll_max, false, comps);
   for (int i = tid; i < n; i += blockDim.x) a.out_traj[off + i] = L.vx[i];
   if (tid == 0) a.out_cost[b] = a.w.w_smooth * comps[0] + a.w.w_limits * comps[1] + a.w_coll_max * comps[2];
 }
@@ -2374,13 +2417,17 @@ extern "C" int pk_traj_cost_grad_f32(void* stream, const pk_traj_model* model, c
   a.out_grad = out_grad;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (maxn == 8 && hulls)
-    hipLaunchKernelGGL((pk::traj_cost_kernel<8, true>), dim3(blocks), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_cost_kernel<8, pk::kHulls>), dim3(blocks), dim3(threads), lds, s, a);
+  else if (maxn == 8 && pk::cost_looks_ahead(d))
+    hipLaunchKernelGGL((pk::traj_cost_kernel<8, pk::kLookupAhead>), dim3(blocks), dim3(threads), lds, s, a);
   else if (maxn == 8)
-    hipLaunchKernelGGL((pk::traj_cost_kernel<8, false>), dim3(blocks), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_cost_kernel<8, pk::kLookup>), dim3(blocks), dim3(threads), lds, s, a);
   else if (hulls)
-    hipLaunchKernelGGL((pk::traj_cost_kernel<16, true>), dim3(blocks), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_cost_kernel<16, pk::kHulls>), dim3(blocks), dim3(threads), lds, s, a);
+  else if (pk::cost_looks_ahead(d))
+    hipLaunchKernelGGL((pk::traj_cost_kernel<16, pk::kLookupAhead>), dim3(blocks), dim3(threads), lds, s, a);
   else
-    hipLaunchKernelGGL((pk::traj_cost_kernel<16, false>), dim3(blocks), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_cost_kernel<16, pk::kLookup>), dim3(blocks), dim3(threads), lds, s, a);
   return pk::check_launch("traj_cost_kernel");
 }
 
@@ -2437,10 +2484,14 @@ extern "C" int pk_traj_lbfgs_f32(void* stream, const pk_traj_model* model, const
   a.out_best = out_best;
   a.out_cost = out_best_cost;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (maxn == 8)
-    hipLaunchKernelGGL(pk::traj_lbfgs_kernel<8>, dim3(blocks), dim3(threads), lds, s, a);
+  if (maxn == 8 && pk::solvers_look_ahead(d))
+    hipLaunchKernelGGL((pk::traj_lbfgs_kernel<8, pk::kLookupAhead>), dim3(blocks), dim3(threads), lds, s, a);
+  else if (maxn == 8)
+    hipLaunchKernelGGL((pk::traj_lbfgs_kernel<8, pk::kLookup>), dim3(blocks), dim3(threads), lds, s, a);
+  else if (pk::solvers_look_ahead(d))
+    hipLaunchKernelGGL((pk::traj_lbfgs_kernel<16, pk::kLookupAhead>), dim3(blocks), dim3(threads), lds, s, a);
   else
-    hipLaunchKernelGGL(pk::traj_lbfgs_kernel<16>, dim3(blocks), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_lbfgs_kernel<16, pk::kLookup>), dim3(blocks), dim3(threads), lds, s, a);
   return pk::check_launch("traj_lbfgs_kernel");
 }
 
@@ -2489,10 +2540,12 @@ extern "C" int pk_traj_chomp_f32(void* stream, const pk_traj_model* model, const
   a.out_cost = out_cost;
   a.out_trace = out_trace;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (maxn == 8)
-    hipLaunchKernelGGL(pk::traj_chomp_kernel<8>, dim3(n_traj), dim3(threads), lds, s, a);
+  if (maxn == 8 && pk::solvers_look_ahead(d))
+    hipLaunchKernelGGL((pk::traj_chomp_kernel<8, pk::kLookupAhead>), dim3(n_traj), dim3(threads), lds, s, a);
+  else if (maxn == 8)
+    hipLaunchKernelGGL((pk::traj_chomp_kernel<8, pk::kLookup>), dim3(n_traj), dim3(threads), lds, s, a);
   else
-    hipLaunchKernelGGL(pk::traj_chomp_kernel<16>, dim3(n_traj), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL((pk::traj_chomp_kernel<16, pk::kLookup>), dim3(n_traj), dim3(threads), lds, s, a);
   return pk::check_launch("traj_chomp_kernel");
 }
 

@@ -1,4 +1,5 @@
-"""The trajectory cost's ways to find obstacles: a robot without spheres."""
+"""The trajectory cost's and solvers' ways to find obstacles: a robot without spheres, and grid
+lookups one by one (few obstacles) against lookups that read ahead."""
 
 from types import SimpleNamespace
 
@@ -8,7 +9,10 @@ import torch
 from conftest import load_robot, random_cfgs
 
 from pyroffi_amd.collision import RobotCollisionSpherized
-from pyroffi_amd.optimization_engines._lbfgs_trajopt_optimization import TrajModel, flatten_trajs, traj_cost
+from pyroffi_amd.optimization_engines import ChompTrajOptConfig
+from pyroffi_amd.optimization_engines._chomp_optimization import chomp_run
+from pyroffi_amd.optimization_engines._lbfgs_trajopt_optimization import (BatchedLbfgsTrajOpt, LbfgsTrajOptConfig,
+                                                                          TrajModel, flatten_trajs, traj_cost)
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +39,36 @@ def test_robot_without_spheres(name, M):
         out.append(traj_cost(model, *flatten_trajs(paths, model.device), w)[0])
     assert not out[0][:, 2].any()
     assert torch.equal(out[0][:, :2], out[1][:, :2])
+
+
+@pytest.mark.parametrize("name", ["panda", "fetch", "baxter"])
+@pytest.mark.parametrize("solver,M,more", [("cost", 1, 70), ("cost", 63, 1), ("lbfgs", 200, 56), ("chomp", 200, 56)])
+def test_lookups_read_ahead_or_not(name, solver, M, more):
+    """The same world with and without obstacles out of reach, which take it past the number
+    from which lookups read ahead: the same terms in the same order, so the same bits."""
+    robot, path = load_robot(name)
+    coll = RobotCollisionSpherized.from_urdf(path)
+    few = _world(M, M)
+    far = _world(more, M + 1)
+    far[:, 2] += 6.0
+    paths = []
+    for T in (5, 17, 23):  # shorter than the shared search takes
+        a, b = random_cfgs(robot, 2, seed=T)
+        s = np.linspace(0, 1, T)[:, None]
+        paths.append(((1 - s) * a + s * b).astype(np.float32))
+    out = []
+    for world in (few, np.concatenate([few, far])):
+        if solver == "lbfgs":
+            cfg = LbfgsTrajOptConfig(n_iters=4)
+            out.append(BatchedLbfgsTrajOpt(TrajModel(robot, coll, world, cfg.collision_margin), paths, cfg).solve()[:2])
+            continue
+        if solver == "chomp":
+            cfg = ChompTrajOptConfig(n_iters=4)
+            model = TrajModel(robot, coll, world, cfg.collision_margin, mode=0)
+            out.append(chomp_run(model, *flatten_trajs(paths, model.device), cfg)[:2])
+            continue
+        model = TrajModel(robot, coll, world, 0.05)
+        out.append(traj_cost(model, *flatten_trajs(paths, model.device), (1.0, 1.0, 0.5, 0.1, 1.0, 2.0)))
+    for x, y in zip(*out):
+        assert torch.equal(x, y)
+    assert (out[0][0][:, 2] > 0).any() if solver == "cost" else True
