@@ -2,12 +2,14 @@
 // whose result is a full distance tensor ([B, K, M] per sphere, [B, N, M] per
 // link over mixed obstacle kinds), and the JAX path's distance conventions.
 //
-// These outputs are large and each element is a few flops, so the kernels are
-// bound by the output write: a flat grid-stride loop gives consecutive lanes
-// consecutive output elements (coalesced 256-byte rows per wave), and the
-// inputs of an element (one robot sphere, one obstacle) come through the
-// caches.  The fused sweep in pk_collision.hip remains the fast path for
-// sphere-only worlds and reduced outputs.
+// The flat kernels (per-sphere outputs, rows from placed spheres, and rows whose
+// tables do not fit the LDS) are bound by the output write: a grid-stride loop gives
+// consecutive lanes consecutive output elements (coalesced 256-byte rows per wave),
+// and the inputs of an element (one robot sphere, one obstacle) come through the
+// caches.  Rows from link poses (link_rows_kernel, self_rows_kernel) take a handful
+// of sphere tests an element and are bound by those: they place a configuration's
+// spheres into the LDS once.  The fused sweep in pk_collision.hip remains the fast
+// path for sphere-only worlds and reduced outputs.
 #include "pk_geom.h"
 #include "pk_model.h"
 
@@ -297,19 +299,29 @@ __device__ __forceinline__ void wave_rows(const RowArgs& a, const float4* pos, c
   }
 }
 
-// Rows of one obstacle kind.  A wave per link pays where it has two obstacles
-// a lane (200 spheres, 111 robot spheres, both collision residuals of 4099
-// configurations: 208 -> 163 us); with 48 to 96 of a kind and two spheres a link
-// it is slower than lane by lane (210 against 197 us), which also takes the
-// half-spaces, of which a scene has a handful.
+// Rows of one obstacle kind.  A wave per link pays where it has two obstacles a lane:
+// it takes whole passes of 128, so that its time steps where lane by lane it grows.
+// 4096 configurations, lane by lane / a wave per link, us, 64, 65, 96, 128, 129, 256
+// obstacles: spheres, Fetch 46 / 48, 59 / 49, 68 / 50, 72 / 49, 84 / 63, 122 / 63, UR5 26
+// / 30, 30 / 31, 36 / 31, 42 / 31, 46 / 39, 69 / 39; capsules, Fetch 51 / 56, 66 / 58, 76
+// / 58, 81 / 58, 96 / 90, 140 / 90, UR5 29 / 34, 34 / 35, 41 / 35, 47 / 35, 51 / 55, 79 /
+// 56; boxes, which hold fifteen registers an obstacle and share no square root, Fetch 51
+// / 78, 67 / 79, 76 / 80, 80 / 80, 95 / 136, 139 / 136, Baxter 43 / 57, 49 / 59, 60 / 59,
+// 73 / 58, 81 / 103, 137 / 105 (112 obstacles 71 / 59): only passes at least seven eighths
+// full pay.  Half-spaces, of which a scene has a handful, stay lane by lane.
 constexpr int kWaveRowsMin = 65;
+
+__device__ __forceinline__ bool box_waves_pay(int n) {
+  const int places = (n + 2 * kWave - 1) / (2 * kWave) * (2 * kWave);
+  return 8 * n >= 7 * places;
+}
 
 template <int KIND, bool JAX>
 __device__ __forceinline__ void rows_of_kind(const RowArgs& a, const float4* pos, const int* cnt, const int* order,
                                              int part, long long row0, int M, int col) {
   const int n = KIND == 0 ? a.w.count[0] : (KIND == 1 ? a.w.count[1] : (KIND == 2 ? a.w.count[2] : a.w.count[3]));
   if constexpr (KIND < 3) {
-    if (n >= kWaveRowsMin) {
+    if (n >= kWaveRowsMin && (KIND != 2 || box_waves_pay(n))) {
       if (KIND != 0 || n <= 2 * kWave) wave_rows<KIND, JAX, 2>(a, pos, cnt, order, part, row0, M, col);
       else wave_rows<KIND, JAX, KIND == 0 ? 4 : 2>(a, pos, cnt, order, part, row0, M, col);
       return;

@@ -112,3 +112,29 @@ def test_residuals_equal_activated_distances(name):
         d = coll.compute_self_collision_distance(robot, q)
         got = self_collision_cost(q, robot, coll, None, margin, weight)
         torch.testing.assert_close(got, (colldist_from_sdf(d, margin) * weight).flatten(), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("kind,M", [(k, m) for k in ("capsules", "boxes") for m in (64, 65, 111, 112, 128, 129, 256, 300)])
+def test_many_capsules_or_boxes(oracle_mod, kind, M):
+    """Lane by lane and a wave per link (capsules from 65 of them, boxes where a pass of 128 is
+    seven eighths full), point capsules and links without spheres among them."""
+    rng = np.random.default_rng(M)
+    B, L, S = 7, 6, 5
+    poses, table = _poses(rng, B, L), _table(rng, L, S, -1e9)
+    c = rng.uniform(-1, 1, (M, 3))
+    if kind == "capsules":
+        end = c + rng.normal(0, 0.3, (M, 3)) * (np.arange(M) % 7 != 0)[:, None]
+        obs = np.concatenate([c, end, rng.uniform(0.02, 0.1, (M, 1))], 1).astype(np.float32)
+    else:
+        axes, _ = np.linalg.qr(rng.normal(size=(M, 3, 3)))
+        obs = np.concatenate([c, axes.transpose(0, 2, 1).reshape(M, 9), rng.uniform(0.02, 0.3, (M, 3))], 1)
+        obs = obs.astype(np.float32)
+    world = {k: np.zeros((0, n), np.float32) for k, n in (("spheres", 4), ("capsules", 7), ("boxes", 15),
+                                                          ("halfspaces", 6))}
+    world[kind] = obs
+    got, _ = ops.sphere_world_links(torch.as_tensor(poses, device="cuda"), torch.as_tensor(table, device="cuda"), world)
+    r = np.broadcast_to(table[None, :, :, 3], (B, L, S)).astype(np.float64)
+    d = oracle_mod.obstacle_dist(_centres(poses, table).reshape(-1, 3), np.maximum(r, 0).reshape(-1),
+                                 **{kind: obs.astype(np.float64)}).reshape(B, L, S, M)
+    ref = np.minimum(np.where(r[..., None] < 0, np.inf, d).min(2), 1e9)
+    _check(got.cpu().numpy(), ref)
