@@ -485,7 +485,7 @@ __global__ __launch_bounds__(kRowThreads) void self_rows_kernel(SelfRowArgs a) {
 // False when the tables do not fit the LDS (jax_self_kernel then takes them).
 static bool launch_self_rows(hipStream_t s, SelfRowArgs a) {
   const long long LS = static_cast<long long>(a.n_links) * a.s_per_link;
-  if (LS > kRowSlots || a.n_links >= 32768 || a.n_pairs > 8192) return false;
+  if (LS > kRowSlots || a.n_links > kRowSlots || a.n_pairs > 8192) return false;
   // Enough configurations for two rounds of lanes, while their spheres take
   // at most 32 KiB.
   a.tile = std::max(1, std::min(2 * kRowThreads / a.n_pairs, LS > 0 ? static_cast<int>(2048 / LS) : 8));
@@ -500,9 +500,10 @@ static bool launch_self_rows(hipStream_t s, SelfRowArgs a) {
 // sorting; fewer configurations than that share each among workgroups.
 template <bool JAX>
 static bool launch_link_rows(hipStream_t s, RowArgs a) {
-  const int LS = a.n_links * a.s_per_link;
+  const long long LS = static_cast<long long>(a.n_links) * a.s_per_link;
   const long long per = a.n_links * static_cast<long long>(a.w.total());
-  if (static_cast<long long>(a.n_links) * a.s_per_link > kRowSlots || per > 0x3fffffffLL) return false;
+  // (Links without a slot have their two words each in the LDS all the same.)
+  if (LS > kRowSlots || a.n_links > kRowSlots || per > 0x3fffffffLL) return false;
   constexpr long long kGroups = 256LL * 4;
   long long parts = 1;
   if (a.batch < kGroups)

@@ -81,6 +81,21 @@ def test_rows_of_random_tables(B, L, S, M):
     _check(om.cpu().numpy(), d.reshape(B, -1).min(1))
 
 
+def test_more_links_than_the_tables_hold():
+    """Links without a slot, more than their words fit the LDS: no sphere anywhere."""
+    L = 30000
+    poses = torch.zeros((2, L, 7), device="cuda")
+    poses[..., 0] = 1
+    table = torch.zeros((L, 0, 4), device="cuda")
+    world = torch.ones((3, 4), device="cuda")
+    pi, pj = (torch.arange(k, k + 5, dtype=torch.int32, device="cuda") for k in (0, L - 5))
+    ow, osf = ops.sphere_distances_jax(poses, table, world, pi, pj)
+    assert torch.isinf(ow).all() and torch.isinf(osf).all()
+    none = {"capsules": np.zeros((0, 7)), "boxes": np.zeros((0, 15)), "halfspaces": np.zeros((0, 6))}
+    ow, _ = ops.sphere_world_links(poses, table, {"spheres": world, **none}, world_min=False)
+    assert (ow == 1e9).all()
+
+
 def test_nan_spheres_are_skipped():
     """A NaN centre or radius takes no part in a minimum, whatever its place in the table."""
     rng = np.random.default_rng(5)
