@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kWave * kHingeWaves, 4) void pose_hinge_kernel(Hing
     for (int k = lstart[n]; k < lstart[n + 1]; ++k) {
       const float4 q = sl[k];
       const float dx = q.x - b.x, dy = q.y - b.y, dz = q.z - b.z;
-      b.w = fminf(fmaxf(b.w, sqrtf(dx * dx + dy * dy + dz * dz) + q.w), 1e29f);
+      b.w = fminf(fmaxf(b.w, sqrtf(dx * dx + dy * dy + dz * dz) + fmaxf(q.w, 0.f)), 1e29f);
     }
     if (lstart[n] == lstart[n + 1]) b = make_float4(0.f, 0.f, 0.f, -1e30f);
     lb[n] = b;
@@ -208,7 +208,14 @@ __global__ __launch_bounds__(kWave * kHingeWaves, 4) void pose_hinge_kernel(Hing
       const float4 s = k < K ? sl[k] : lb[k - K];
       float wx, wy, wz;
       quat_rotate(p[0], p[1], p[2], p[3], s.x, s.y, s.z, wx, wy, wz);
-      sc[k] = make_float4(wx + p[4], wy + p[5], wz + p[6], s.w);  // bc follows sc
+      float r = s.w;
+      if (k >= K) {
+        // A quaternion that is not of unit length stretches the link's offsets by at
+        // most 1 + 4 ||q|^2 - 1| (finite also for a NaN pose).
+        const float qq = p[0] * p[0] + p[1] * p[1] + p[2] * p[2] + p[3] * p[3];
+        r = fminf(fmaf(4.f * fabsf(qq - 1.f), fmaxf(r, 0.f), r), 1e29f);
+      }
+      sc[k] = make_float4(wx + p[4], wy + p[5], wz + p[6], r);  // bc follows sc
     }
     wave_sync();
 

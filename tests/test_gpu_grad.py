@@ -146,3 +146,30 @@ def test_fk_adjoint_root_link_and_zero_cotangent():
     g[:, 0] = 1.0  # the root link is the constant identity: no gradient
     (dq,) = torch.autograd.grad(poses, q, g)
     assert float(dq.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("scale", [0.25, 1.0, 1.001, 2.0])
+def test_quaternions_that_are_not_of_unit_length(scale):
+    """The hinge sum over link poses as they come: the sphere placement is linear in the sphere's
+    offset, whatever the quaternion, and so must the links' bounding spheres be.  FP32 sums of a
+    few hundred terms: 1e-4 of the cost."""
+    from pyroffi_amd.kernels import ops
+
+    rng = np.random.default_rng(31)
+    B, L, per, M, margin = 200, 7, 9, 150, 0.05
+    quat = rng.normal(size=(B, L, 4))
+    quat *= scale / np.linalg.norm(quat, axis=-1, keepdims=True)
+    poses = np.concatenate([quat, rng.uniform(-1, 1, (B, L, 3))], -1).astype(np.float32)
+    spheres = np.concatenate([rng.normal(0, 0.15, (L * per, 3)), rng.uniform(0.02, 0.1, (L * per, 1))],
+                             1).astype(np.float32)
+    world = np.concatenate([rng.uniform(-1.5, 1.5, (M, 3)), rng.uniform(0.02, 0.2, (M, 1))], 1).astype(np.float32)
+    none = np.zeros(0, np.int32)
+    cost, _ = ops.pose_hinge_cost(poses, spheres, np.arange(L + 1) * per, world, margin, -1, None, np.zeros((0, 6)),
+                                  none, none, none, np.zeros(0, np.float32), none, np.full(L, -1), 1, want_grad=False)
+    p = np.repeat(poses.astype(np.float64), per, axis=1)
+    c = np.broadcast_to(spheres[None, :, :3].astype(np.float64), p.shape[:2] + (3,))
+    u = 2 * np.cross(p[..., 1:4], c)
+    c = c + p[..., :1] * u + np.cross(p[..., 1:4], u) + p[..., 4:]
+    d = np.linalg.norm(c[:, :, None] - world[:, :3], axis=-1) - spheres[None, :, None, 3] - world[:, 3]
+    ref = (np.maximum(margin - d, 0) ** 2).sum((1, 2))
+    np.testing.assert_allclose(cost.cpu().numpy(), ref, rtol=1e-4, atol=1e-6)
