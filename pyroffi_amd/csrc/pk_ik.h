@@ -1338,13 +1338,26 @@ inline long long wave_seed_limit() {
 }
 
 // Seeds of one wave when they share the collision penalty, whose cost grows
-// with them while the LM step's does not: as many as keep at most two waves
-// per SIMD, up to the 8 groups of 8 lanes.
+// with them while the LM step's does not: as many as keep every wave resident
+// (two a SIMD of the 8-wide kernel; one of the 16-wide, whose 487 registers leave
+// room for no second: 1952 seeds of Baxter, 32 spheres, 10 iterations, one seed a wave
+// in two rounds 1046 us, two seeds 565), up to the 8 groups of 8 lanes.
+template <int MAXA>
 inline int coop_seeds_per_wave(long long n_all) {
+  constexpr int waves = MAXA == 8 ? 2 : 1;  // a SIMD holds
   int n = 1;
-  while (n < 8 && n_all > 2 * wave_seed_limit() * n) n *= 2;
+  while (n < 8 && n_all > waves * wave_seed_limit() * n) n *= 2;
   return n;
 }
+
+// Whether sharing pays: the wave goes through its seeds one after the other, where
+// lanes of their own test `pairs` (robot spheres x obstacles) side by side.  Ten
+// iterations, a lane for itself / shared, us: Panda (59 spheres), 12000 seeds (8 a
+// wave), 1, 8 and 16 obstacles 306 / 521, 521 / 556, 780 / 574, 6400 seeds (4), 1 and 4
+// 291 / 340, 372 / 345, 3840 seeds (2), 1 279 / 253; UR5 (40), 12000, 8 and 16 397 / 496,
+// 564 / 498; Fetch (111), 12000, 4 and 8 533 / 612, 728 / 697; Baxter (75), 6400 (8), 8
+// and 16 828 / 1039, 1108 / 1040, 3840 (4), 2 and 8 597 / 683, 831 / 708.
+inline bool coop_pays(long long pairs, int per_wave) { return pairs >= 10LL * per_wave * per_wave; }
 
 template <int MAXA, int NEE>
 __device__ __forceinline__ void store_iterate(WaveLds<MAXA, NEE>& wl, const Pose* P, const Pose* Tee, const float* r) {
@@ -1744,9 +1757,11 @@ inline int launch_ik(void* stream, const IkArgs& a, bool batched, int grid_waves
   if (n_all * 8 <= kSmallBatchLanes) {
     constexpr int G = 8;
     const size_t lds_c = pen_lds_offset<MAXA, NEE>(a) + pen_lds_bytes<MAXA>(Kin);
-    if (coll && lds_c <= 150 * 1024) {
+    const int per_wave = coop_seeds_per_wave<MAXA>(n_all);
+    const long long pairs = static_cast<long long>(Kin) * (M + a.n_caps + a.n_boxes + a.n_hs);
+    if (coll && lds_c <= 150 * 1024 && coop_pays(pairs, per_wave)) {
       IkArgs b = a;
-      b.seeds_per_wave = coop_seeds_per_wave(n_all);
+      b.seeds_per_wave = per_wave;
       dim3 grid((a.n_seeds + b.seeds_per_wave - 1) / b.seeds_per_wave, a.n_problems);
       hipLaunchKernelGGL((ls_ik_kernel<MAXA, NEE, G, true>), grid, dim3(kWave), lds_c, s, b);
     } else {
