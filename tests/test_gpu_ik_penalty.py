@@ -61,3 +61,22 @@ def _check(oracle_mod, name, n_seeds, world):
                                     lambda_init=1e-2, **okw)
         close = np.isclose(errs.cpu().numpy(), oerrs, rtol=1e-4, atol=1e-5)
         assert close.all() if iters == 0 else close.mean() >= 0.99, (iters, close.mean())
+
+
+@pytest.mark.parametrize("name,m", [("panda", 4), ("fetch", 2), ("baxter", 3)])
+def test_shared_or_not_gives_the_same_bits(name, m):
+    """Seeds among few others share the penalty over the wave, among many and few obstacles each
+    lane tests for itself: the same sums."""
+    robot, path = load_robot(name)
+    links = (robot.links.names.index(HAND[name]),)
+    rng = np.random.default_rng(m)
+    lo, hi = robot.joints.lower_limits, robot.joints.upper_limits
+    tgt = np.asarray(robot.forward_kinematics(random_cfgs(robot, 1, seed=2).astype(np.float32)))[:, list(links)]
+    seeds = rng.uniform(lo, hi, (1, 12000, len(lo))).astype(np.float32)
+    world = np.concatenate([rng.uniform(-0.6, 0.6, (m, 3)), np.full((m, 1), 0.3)], 1).astype(np.float32)
+    rs, rj, ws, ok = prepare_ls_collision_buffers(robot, RobotCollisionSpherized.from_urdf(path), world)
+    assert ok
+    run = lambda s: ls_ik_run(robot, s, tgt, links, max_iter=5, collision=(rs, rj, ws, 1e4, 0.02))  # noqa: E731
+    cfgs, errs = run(seeds)
+    few_cfgs, few_errs = run(seeds[:, 3000:4100])
+    assert (few_cfgs == cfgs[:, 3000:4100]).all() and (few_errs == errs[:, 3000:4100]).all()
