@@ -482,10 +482,32 @@ __global__ __launch_bounds__(kRowThreads) void self_rows_kernel(SelfRowArgs a) {
   }
 }
 
-// False when the tables do not fit the LDS (jax_self_kernel then takes them).
+// Where the kernels that place a configuration's spheres once pay against the flat
+// ones, which place a link's slots for every element but have neither tables to sort
+// nor barriers.  Flat / placed, us (JAX conventions; links x slots): 64 configurations
+// among 128 obstacles Panda (13 x 18) 6 / 10, Fetch (17 x 28) 10 / 17; 1000 among 32, 64
+// Panda 12 / 12, 19 / 14, UR5 (23 x 9) 11 / 10, 18 / 14, Fetch 20 / 21, 34 / 28, Baxter (44
+// x 4) 10 / 13, 18 / 18; 16000 among 8, 16, 32 Panda 32 / 56, 60 / 60, 115 / 75, Fetch 60 /
+// 82, 117 / 100, 224 / 120, Baxter 30 / 46, 57 / 64, 119 / 102.
+inline bool placed_rows_pay(long long batch, int L, int S, int M) {
+  const long long tests = static_cast<long long>(M) * S;  // of a link, padding included
+  return M >= 24 && tests >= 192 && batch * L >= ((1LL << 23) + tests - 1) / tests;
+}
+
+// The same for the self pairs: 1000, 2000 and 4000 configurations Panda (66 pairs) 7 /
+// 11, 9 / 11, 12 / 12, UR5 (231) 7 / 7, 10 / 9, 16 / 14, Fetch (120) 10 / 14, 15 / 14, 27 /
+// 20, Baxter (903) 10 / 9, 18 / 14, 30 / 23.
+inline bool placed_self_pays(long long batch, int S, int P) {
+  const long long tests = static_cast<long long>(P) * S;
+  return tests > 0 && batch >= ((1LL << 22) + tests - 1) / tests;
+}
+
+// False when that does not pay or the tables do not fit the LDS (jax_self_kernel then
+// takes them).
 static bool launch_self_rows(hipStream_t s, SelfRowArgs a) {
   const long long LS = static_cast<long long>(a.n_links) * a.s_per_link;
   if (LS > kRowSlots || a.n_links > kRowSlots || a.n_pairs > 8192) return false;
+  if (!placed_self_pays(a.batch, a.s_per_link, a.n_pairs)) return false;
   // Enough configurations for two rounds of lanes, while their spheres take
   // at most 32 KiB.
   a.tile = std::max(1, std::min(2 * kRowThreads / a.n_pairs, LS > 0 ? static_cast<int>(2048 / LS) : 8));
@@ -495,7 +517,8 @@ static bool launch_self_rows(hipStream_t s, SelfRowArgs a) {
   return true;
 }
 
-// Launch of link_rows_kernel, or false when its tables do not fit the LDS.
+// Launch of link_rows_kernel, or false when it does not pay or its tables do not fit
+// the LDS.
 // Four workgroups a CU loop over the configurations, which spreads the table's
 // sorting; fewer configurations than that share each among workgroups.
 template <bool JAX>
@@ -504,6 +527,7 @@ static bool launch_link_rows(hipStream_t s, RowArgs a) {
   const long long per = a.n_links * static_cast<long long>(a.w.total());
   // (Links without a slot have their two words each in the LDS all the same.)
   if (LS > kRowSlots || a.n_links > kRowSlots || per > 0x3fffffffLL) return false;
+  if (!placed_rows_pay(a.batch, a.n_links, a.s_per_link, a.w.total())) return false;
   constexpr long long kGroups = 256LL * 4;
   long long parts = 1;
   if (a.batch < kGroups)

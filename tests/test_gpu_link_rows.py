@@ -1,7 +1,9 @@
 """Per-link distance rows against float64 numpy, where the kernels' table sorting and lane
 strides can go wrong: interior and repeated padding, unsorted and repeated radii, links with
 no sphere, NaN entries, one obstacle to several hundred, one configuration (its rows shared
-among workgroups) to more than the launch has workgroups, and tables too large for the LDS."""
+among workgroups) to more than the launch has workgroups, and tables too large for the LDS.
+Few configurations or obstacles take flat kernels; the others are reached by the same poses
+many times over, every copy equal to the first."""
 
 import numpy as np
 import pytest
@@ -38,6 +40,24 @@ def _centres(poses, table):
     return c + w * u + np.cross(np.broadcast_to(v, u.shape), u) + poses[:, :, None, 4:]
 
 
+def _copies(B, L, S, M, P=0):
+    """Copies of B poses from which the rows (and self pairs, if any) are placed once."""
+    n = -(-(1 << 23) // (B * L * S * M))
+    return max(n, -(-(1 << 22) // (B * S * P)) if P else 0)
+
+
+def _many(run, poses, n):
+    """The rows of n copies of the poses; equal, so the first is returned."""
+    out = []
+    for x in run(torch.as_tensor(np.tile(poses, (n, 1, 1)), device="cuda")):
+        if x is not None:
+            x = x.reshape(n, len(poses), *x.shape[1:])
+            assert torch.equal(x, x[:1].expand_as(x))
+            x = x[0]
+        out.append(x)
+    return out
+
+
 def _check(got, ref):
     big = ref >= 1e8
     np.testing.assert_array_equal(got >= 1e8, big)
@@ -64,6 +84,14 @@ def test_rows_of_random_tables(B, L, S, M):
     ow, osf = ops.sphere_distances_jax(*(torch.as_tensor(x, device="cuda") for x in (poses, table, world, pi, pj)))
     _check(ow.cpu().numpy(), d)
     _check(osf.cpu().numpy(), own)
+    n = _copies(B, L, S, M, 40)
+    dev = [torch.as_tensor(x, device="cuda") for x in (table, world, pi, pj)]
+    mow, mosf = _many(lambda p: ops.sphere_distances_jax(p, *dev), poses, n)
+    _check(mow.cpu().numpy(), d)
+    _check(mosf.cpu().numpy(), own)
+    mcost, mself = _many(lambda p: ops.sphere_distances_jax(p, *dev, cost=(0.2, 3.0)), poses, n)
+    torch.testing.assert_close(mcost, colldist_from_sdf(mow, 0.2) * 3.0, rtol=1e-5, atol=1e-6)
+    torch.testing.assert_close(mself, colldist_from_sdf(mosf, 0.2) * 3.0, rtol=1e-5, atol=1e-6)
     cost, _ = ops.sphere_distances_jax(*(torch.as_tensor(x, device="cuda") for x in (poses, table, world, pi, pj)),
                                        self_pairs=False, cost=(0.2, 3.0))
     torch.testing.assert_close(cost, colldist_from_sdf(ow, 0.2) * 3.0, rtol=1e-5, atol=1e-6)
@@ -79,6 +107,9 @@ def test_rows_of_random_tables(B, L, S, M):
     ow, om = ops.sphere_world_links(torch.as_tensor(poses, device="cuda"), torch.as_tensor(table, device="cuda"), w)
     _check(ow.cpu().numpy(), d)
     _check(om.cpu().numpy(), d.reshape(B, -1).min(1))
+    mow, _ = _many(lambda p: ops.sphere_world_links(p, torch.as_tensor(table, device="cuda"), w, world_min=False),
+                   poses, n)
+    _check(mow.cpu().numpy(), d)
 
 
 def test_more_links_than_the_tables_hold():
@@ -108,16 +139,18 @@ def test_nan_spheres_are_skipped():
             bad, good = table.copy(), table.copy()
             bad[0, place, col] = np.nan
             good[0, place] = [0, 0, 0, -1e9]
-            a, _ = ops.sphere_world_links(cuda(poses), cuda(bad), {"spheres": world, **none})
-            b, _ = ops.sphere_world_links(cuda(poses), cuda(good), {"spheres": world, **none})
-            torch.testing.assert_close(a, b, rtol=0, atol=0)
+            for n in (1, _copies(6, 3, 8, 70)):
+                rows = lambda t: _many(lambda p: ops.sphere_world_links(p, cuda(t), {"spheres": world, **none}),  # noqa: E731
+                                       poses, n)[0]
+                torch.testing.assert_close(rows(bad), rows(good), rtol=0, atol=0)
 
 
+@pytest.mark.parametrize("copies", [1, 100])
 @pytest.mark.parametrize("name", ("panda", "baxter"))
-def test_residuals_equal_activated_distances(name):
+def test_residuals_equal_activated_distances(name, copies):
     robot, path = load_robot(name)
     coll = RobotCollisionSpherized.from_urdf(path)
-    q = torch.as_tensor(random_cfgs(robot, 37, seed=4).astype(np.float32), device="cuda")
+    q = torch.as_tensor(random_cfgs(robot, 37, seed=4).astype(np.float32), device="cuda").repeat(copies, 1)
     rng = np.random.default_rng(6)
     world = np.concatenate([rng.uniform(-1, 1, (50, 3)), rng.uniform(0.02, 0.2, (50, 1))], 1).astype(np.float32)
     for margin, weight in ((0.05, 2.0), (0.2, torch.tensor(3.0, device="cuda")), (np.float32(0.1), 1)):
@@ -147,7 +180,8 @@ def test_many_capsules_or_boxes(oracle_mod, kind, M):
     world = {k: np.zeros((0, n), np.float32) for k, n in (("spheres", 4), ("capsules", 7), ("boxes", 15),
                                                           ("halfspaces", 6))}
     world[kind] = obs
-    got, _ = ops.sphere_world_links(torch.as_tensor(poses, device="cuda"), torch.as_tensor(table, device="cuda"), world)
+    tab = torch.as_tensor(table, device="cuda")
+    got, _ = _many(lambda p: ops.sphere_world_links(p, tab, world, world_min=False), poses, _copies(B, L, S, M))
     r = np.broadcast_to(table[None, :, :, 3], (B, L, S)).astype(np.float64)
     d = oracle_mod.obstacle_dist(_centres(poses, table).reshape(-1, 3), np.maximum(r, 0).reshape(-1),
                                  **{kind: obs.astype(np.float64)}).reshape(B, L, S, M)
