@@ -44,8 +44,10 @@ PEAK_FP32_TFLOPS = 157.3
 PEAK_FP32_UNPACKED_TFLOPS = 78.6
 PEAK_HBM_GBS = 8000.0
 # Algorithmic work per configuration (flop convention: sphere-sphere distance
-# including the min = 12; SE(3) sphere placement ~ 33 per sphere).
+# including the min = 12; SE(3) sphere placement ~ 33 per sphere).  The world
+# minimum needs one bound per (link with spheres, obstacle), not every sphere pair.
 K_SPHERES = 59
+K_SPHERE_LINKS = 11
 SELF_SPHERE_PAIRS = 1230
 # LM-IK: algorithmic flops per LM iteration per seed for Panda without
 # collision (FK + Jacobian 1.6 k, normal equations 0.7 k, Cholesky 0.3 k, five
@@ -54,7 +56,7 @@ SELF_SPHERE_PAIRS = 1230
 IK_FLOP_PER_SEED_ITER = 9600
 IK_FLOP_PLACEMENT = 33
 IK_FLOP_PAIR = 13
-FLOP_SWEEP = K_SPHERES * M_WORLD * 12 + SELF_SPHERE_PAIRS * 12 + K_SPHERES * 33
+FLOP_SWEEP = K_SPHERE_LINKS * M_WORLD * 12 + SELF_SPHERE_PAIRS * 12 + K_SPHERES * 33
 BYTES_FK = 7 * 4 + 13 * 7 * 4  # cfg in + link poses out
 BYTES_SWEEP = 13 * 7 * 4 + 4 + 66 * 4  # link poses in + min + self pairs out
 
@@ -806,7 +808,9 @@ def grad_bench(reps: int, cpu_sample: int):
     e1.record(stream)
     e1.synchronize()
     kms = e0.elapsed_time(e1) / reps
-    flop = K_SPHERES * m * 13 * 3  # forward 13 flop per pair, backward ~2x forward
+    # One bound per (link with spheres, obstacle) and the placement; the pairs within
+    # the margin, about one in a thousand, and the tree's adjoint are not counted.
+    flop = K_SPHERE_LINKS * m * 12 + K_SPHERES * 33
     # CPU: FP64 oracle cost + central-difference gradient (15 cost evaluations per config).
     t_or = oracle.Tables.of(robot)
     sp = oracle.padded_spheres(coll)
